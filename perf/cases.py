@@ -1,0 +1,543 @@
+"""The workloads that performance work on this package is measured by: what a user has it do, through its
+public entry points, over the sizes, options and directions that are used in earnest.
+
+A case is a dict of plain values with a "kind":
+
+  image     one call of Imager.run_device: K frames in device memory to K images
+  windows   one call of SubaperturePlan.run: windows of uneven pulse counts of one dwell
+  compress  one call of isar_pulse_compress: raw IFDS echoes to compressed profiles
+  judge     one image formation from given phases (a BACK run) and its entropies, as the
+            warm start judges a candidate
+  train     one training step of the warm-start network up to its gradients
+
+`exact` gives the same outputs in 64 bits from plain torch.
+"""
+import ctypes
+import math
+
+import numpy as np
+import torch
+
+import isar_imaging_cuda_amd as isar
+from isar_imaging_cuda_amd import learned, subaperture, synth
+
+W = 512
+LIGHT = 3e8
+DEV = "cuda:0"
+
+# Scenes (synth presets): 1 a slowly turning target without range walk compensation, 2 a fast ship-sized
+# target, 3 the scene of 1 after coarse tracking, 4 range-aligned frames with uniform phase errors.
+
+# Chunk rows, autofocus form, chirp-z length and threads per pulse count of the dwell workload, as bench.py sets them.
+WINDOW_TUNING = {128: (2, 3, 256, 256), 192: (4, 1, 512, 256), 256: (4, 1, 512, 256), 384: (4, 1, 1024, 256),
+                 512: (4, 3, 1024, 256)}
+
+
+def _image(name, scene, pulses, cells, frames, **more):
+    case = {"kind": "image", "scene": scene, "pulses": pulses, "cells": cells, "frames": frames,
+            "distinct": min(frames, 64), "type": 2, "hpc": True, "mtrc": True, "quirk": True, "iterations": 120,
+            "form": 0, "chunk": 8, "graph": False}
+    case.update(more)
+    return {**case, "name": name} if name else case
+
+
+def listed():
+    return [
+        # the smallest frame size of the package's own configurations, one frame with every knob left alone:
+        # launches and latency
+        _image("one_128x1024", 1, 128, 1024, 1),
+        # the drop-in's unit of work, with the session's settings: resident autofocus, two-row chunks, a graph
+        _image("one_256x4096", 2, 256, 4096, 1, form=4, chunk=2, graph=True),
+        # a short batch, as a receiver hands over what it has collected; the whole slow-time window
+        _image("batch13_192x2048", 3, 192, 2048, 13, quirk=False),
+        # the largest batch the default autofocus spreads over several workgroups per frame
+        _image("batch32_256x4096", 2, 256, 4096, 32),
+        # range profiles that were pulse-compressed on ingest (IFDS), imaged without MTRC
+        _image("ifds96_256x4096", 1, 256, 4096, 96, type=1, hpc=False, mtrc=False),
+        # long windows at the wider sampling
+        _image("batch40_512x8192", 3, 512, 8192, 40),
+        # throughput imaging: the headline workload (64 distinct frames repeated)
+        _image("batch1024_256x4096", 2, 256, 4096, 1024, chunk=16),
+        # the largest frames the package takes, a few at a time
+        _image("batch8_1024x16384", 3, 1024, 16384, 8, form=4),
+        # a whole recording: 64 sliding windows of one dwell in one graph launch
+        {"name": "windows64_8192x4096", "kind": "windows", "dwell": 8192, "cells": 4096, "count": 64},
+        # ingest of raw chirp echoes
+        {"name": "compress256x6000", "kind": "compress", "echoes": 256, "length": 6000},
+        # the warm start's judgement of one candidate phase per frame
+        {"name": "judge256_256x2048", "kind": "judge", "scene": 4, "pulses": 256, "cells": 2048, "frames": 256,
+         "distinct": 64},
+        # training the 256-pulse network
+        {"name": "train_m256_b256", "kind": "train", "pulses": 256, "batch": 256},
+    ]
+
+
+def _log_int(rng, low, high):
+    return int(round(math.exp(rng.uniform(math.log(low), math.log(high)))))
+
+
+def draw(rng):
+    kind = rng.choices(["image", "windows", "compress", "judge", "train"], [6, 1, 1, 1, 1])[0]
+    if kind == "compress":
+        return {"kind": kind, "echoes": _log_int(rng, 16, 2048), "length": _log_int(rng, 2100, 16000)}
+    if kind == "train":
+        return {"kind": kind, "pulses": rng.choice([64, 128, 192, 256, 384, 512, 1024]),
+                "batch": _log_int(rng, 16, 1024)}
+    if kind == "windows":
+        return {"kind": kind, "dwell": _log_int(rng, 1024, 8192), "cells": rng.choice([1024, 2048, 4096]),
+                "count": _log_int(rng, 5, 64)}
+    cells = rng.choice([1024, 2048, 4096, 8192, 16384])
+    if kind == "judge":
+        pulses = rng.choice([128, 192, 256])
+        frames = _log_int(rng, 4, 256)
+        return {"kind": kind, "scene": 4, "pulses": pulses, "cells": min(cells, 4096), "frames": frames,
+                "distinct": min(frames, 64)}
+    pulses = rng.choice([64, 128, 192, 256, 384, 512, 1024])
+    frames = _log_int(rng, 1, min(512, (1 << 27) // (pulses * cells)))
+    scene = 2 if pulses == 256 else rng.choice([1, 3])
+    more = {}
+    option = rng.randrange(8)
+    if option == 0:
+        more = {"type": 1, "hpc": False, "scene": 1}
+    elif option == 1:
+        more = {"mtrc": False}
+    elif option == 2:
+        more = {"quirk": False}
+    elif option == 3:
+        more = {"hpc": False, "scene": 3}
+    if frames <= 32 and rng.random() < 0.5:
+        more["form"] = 4
+    more["chunk"] = rng.choice([2, 4, 8, 8, 16])
+    more.setdefault("scene", scene)
+    case = _image(None, scene, pulses, cells, frames)
+    case.update(more)
+    return case
+
+
+# ------------------------------------------------------------------------------------------
+# inputs
+# ------------------------------------------------------------------------------------------
+def _frames(case, seed):
+    """`distinct` synthetic frames (K, M, N, 2), the velocities (K, M) and the radar header."""
+    cfg = synth.preset(case["scene"], echo_num=case["pulses"], range_num=case["cells"])
+    n = case["distinct"]
+    echo = torch.empty((n, case["pulses"], case["cells"], 2), dtype=torch.float32, device=DEV)
+    vel = torch.empty((n, case["pulses"]), dtype=torch.float64, device=DEV)
+    synth.frames_device(cfg, [(seed + 1) * 100_003 + k for k in range(n)], echo.data_ptr(), vel.data_ptr())
+    if case.get("type") == 1:   # compressed range profiles of the same scene
+        x = torch.roll(torch.view_as_complex(echo), case["cells"] // 2, dims=2)
+        x = torch.roll(torch.fft.fft(x, dim=2), case["cells"] // 2, dims=2)
+        echo = torch.view_as_real(x).contiguous()
+    return echo, vel, synth.radar_header(cfg)
+
+
+def _batch(case, echo, vel):
+    """The distinct frames repeated to the batch size."""
+    K = case["frames"]
+    if K == echo.shape[0]:
+        return echo, vel
+    idx = torch.arange(K, device=DEV) % echo.shape[0]
+    return echo[idx].contiguous(), vel[idx].contiguous()
+
+
+def _radar(case, header):
+    return isar.RadarParams(case["pulses"], case["cells"], header["band_width"], header["fc"], header["Tp"],
+                            header["Fs"])
+
+
+def _phases(case, seed):
+    """Per-pulse phases as a warm start proposes them: a smooth drift and noise."""
+    g = torch.Generator().manual_seed(seed + 17)
+    M, K = case["pulses"], case["frames"]
+    t = torch.linspace(-1, 1, M, dtype=torch.float64)
+    c = torch.randn((K, 3), generator=g, dtype=torch.float64)
+    ph = c[:, :1] * t ** 2 + c[:, 1:2] * t ** 3 + c[:, 2:] * t ** 4
+    ph = ph + 0.3 * torch.randn((K, M), generator=g, dtype=torch.float64)
+    return torch.stack([torch.cos(ph), torch.sin(ph)], dim=-1).to(torch.float32).to(DEV)
+
+
+def _windows(case, seed):
+    cfg = synth.preset(3, echo_num=case["dwell"], range_num=case["cells"])
+    echo = torch.empty((1, case["dwell"], case["cells"], 2), dtype=torch.float32, device=DEV)
+    vel = torch.empty((1, case["dwell"]), dtype=torch.float64, device=DEV)
+    synth.frames_device(cfg, [(seed + 1) * 100_003], echo.data_ptr(), vel.data_ptr())
+    first, pulses = subaperture.sliding_windows(case["dwell"], case["count"], seed=7)
+    return echo[0], vel[0], synth.radar_header(cfg), first, pulses
+
+
+def _echoes(case, seed):
+    cfg = synth.preset(6, echo_num=case["echoes"], range_num=case["length"], tp=40e-6, seed=(seed + 1) * 100_003)
+    iq, vel = synth.ifds(cfg)
+    raw = np.ascontiguousarray(np.stack([iq.real, iq.imag], axis=-1).astype(np.int16))
+    return torch.from_numpy(raw).to(DEV), torch.from_numpy(vel).to(DEV), synth.radar_header(cfg)
+
+
+def _net(case, seed):
+    widths = learned.widths_for(case["pulses"])
+    g = torch.Generator().manual_seed(seed + 23)
+    params = learned.he_init(widths, seed=seed % (1 << 31))
+
+    def phasors(cols):
+        ph = torch.randn((case["batch"], cols // 2), generator=g, dtype=torch.float64)
+        x = torch.stack([torch.cos(ph), torch.sin(ph)], dim=-1).reshape(case["batch"], cols)
+        return x.to(torch.float32).to(DEV)
+
+    return widths, params, phasors(widths[0]), phasors(widths[-1])
+
+
+def _options(case, **more):
+    o = dict(data_type=case["type"], if_hpc=case["hpc"], if_mtrc=case["mtrc"], quirk_q1=case["quirk"],
+             iterations=case["iterations"])
+    return isar.Options(**{**o, **more})
+
+
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind == "train":
+        widths, params, x, target = _net(case, seed)
+        net = learned.Mlp(widths, case["batch"])
+        net.set_params(params)
+        out = torch.empty((case["batch"], widths[-1]), dtype=torch.float32, device=DEV)
+        return {"case": case, "net": net, "x": x, "target": target, "out": out, "grad": torch.empty_like(out),
+                "loss": torch.empty(case["batch"], dtype=torch.float64, device=DEV)}
+    if kind == "compress":
+        iq, vel, h = _echoes(case, seed)
+        p = isar.RadarParams(case["echoes"], 4096, h["band_width"], h["fc"], h["Tp"], h["Fs"]).c()
+        fn = isar.lib().isar_pulse_compress
+        fn.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int] + [ctypes.c_void_p] * 5
+        return {"case": case, "params": p, "fn": fn, "iq": iq, "vel": vel,
+                "out": torch.empty((case["echoes"], 4096, 2), dtype=torch.float32, device=DEV),
+                "offsets": torch.empty(case["echoes"], dtype=torch.int32, device=DEV)}
+    stream = torch.cuda.current_stream().cuda_stream
+    if kind == "windows":
+        echo, vel, h, first, pulses = _windows(case, seed)
+        plan = subaperture.SubaperturePlan(
+            isar.RadarParams(256, case["cells"], h["band_width"], h["fc"], h["Tp"], h["Fs"]), case["dwell"], first, pulses)
+        keys = ("ra_chunk", "autofocus_mode", "czt_length", "czt_threads")
+        plan.set_tuning({m: dict(zip(keys, t)) for m, t in WINDOW_TUNING.items()})
+        img = torch.empty(plan.image_floats, dtype=torch.float32, device=DEV)
+        return {"case": case, "plan": plan, "echo": echo, "vel": vel, "img": img, "options": isar.Options(),
+                "stream": stream}
+    echo, vel, h = _frames(case, seed)
+    echo, vel = _batch(case, echo, vel)
+    im = isar.Imager(_radar(case, h), max_frames=case["frames"])
+    img = torch.empty((case["frames"], case["pulses"], W), dtype=torch.float32, device=DEV)
+    state = {"case": case, "im": im, "echo": echo, "vel": vel, "img": img, "stream": stream}
+    if kind == "judge":
+        im.run_device(echo.data_ptr(), vel.data_ptr(), 0, case["frames"], isar.Options(iterations=1, stage_mode=1),
+                      stream=stream)
+        state["phi"] = _phases(case, seed)
+        state["entropy"] = torch.empty(case["frames"], dtype=torch.float64, device=DEV)
+        state["options"] = isar.Options(iterations=0, stage_mode=2, warm_start=True)
+        return state
+    im.set_autofocus_mode(case["form"])
+    im.set_ra_chunk(min(case["chunk"], case["pulses"] // 2))
+    im.set_graph_mode(case["graph"])
+    state["options"] = _options(case)
+    return state
+
+
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "train":
+        net, b = state["net"], case["batch"]
+        net.forward(b, state["x"].data_ptr(), state["out"].data_ptr())
+        learned.mse(b, net.widths[-1], state["out"].data_ptr(), state["target"].data_ptr(), state["grad"].data_ptr(),
+                    state["loss"].data_ptr())
+        net.backward(b, state["grad"].data_ptr())
+        # the gradients come out through the host, which is the one way the interface gives them
+        return {"pred": state["out"], "loss": state["loss"], "grads": net.get_grads()}
+    if kind == "compress":
+        rc = state["fn"](ctypes.byref(state["params"]), case["echoes"], case["length"], state["iq"].data_ptr(),
+                         state["vel"].data_ptr(), state["out"].data_ptr(), state["offsets"].data_ptr(),
+                         torch.cuda.current_stream().cuda_stream)
+        if rc:
+            raise isar.ImagingError("isar_pulse_compress: %d" % rc)
+        return {"profiles": state["out"], "offsets": state["offsets"]}
+    if kind == "windows":
+        state["plan"].run(state["echo"].data_ptr(), state["vel"].data_ptr(), state["img"].data_ptr(), state["options"],
+                          graph=True, stream=state["stream"])
+        return {"images": state["img"]}
+    if kind == "judge":
+        K = case["frames"]
+        state["im"].run_device(0, 0, state["img"].data_ptr(), K, state["options"], phi0_ptr=state["phi"].data_ptr(),
+                               stream=state["stream"])
+        learned.image_entropy(K, case["pulses"] * W, state["img"].data_ptr(), state["entropy"].data_ptr(),
+                              state["stream"])
+        return {"images": state["img"], "entropy": state["entropy"]}
+    state["im"].run_device(state["echo"].data_ptr(), state["vel"].data_ptr(), state["img"].data_ptr(), case["frames"],
+                           state["options"], stream=state["stream"])
+    return {"images": state["img"]}
+
+
+# ------------------------------------------------------------------------------------------
+# what a pass cannot do without
+# ------------------------------------------------------------------------------------------
+def _fft_flops(n, count):
+    return 5.0 * n * math.log2(n) * count
+
+
+def _frame_work(M, N, iterations=120, bins=64, mtrc=True):
+    """Bytes: the echo and velocities in, the image out. Flops: one transform per row and per pair profile
+    and correlation of the alignment, of the rows that move at each merge level, of the selected bins twice
+    per iteration, and of the image formation."""
+    levels = math.ceil(math.log2(M))
+    rows = M + levels * (M / 2) + 2 * (M - 1)
+    flops = _fft_flops(N, rows) + iterations * _fft_flops(M, 2 * bins) + _fft_flops(M, 2 * W)
+    if mtrc:
+        flops += _fft_flops(2 * M, 2 * W) + _fft_flops(W, 2 * M)
+    return 8.0 * M * N + 8.0 * M + 4.0 * M * W, flops
+
+
+def work(case):
+    kind = case["kind"]
+    if kind == "train":
+        widths = learned.widths_for(case["pulses"])
+        n = sum(a * b for a, b in zip(widths[:-1], widths[1:]))
+        params = n + sum(widths[1:])
+        return {"bytes": 4.0 * case["batch"] * (widths[0] + 2 * widths[-1]) + 4.0 * 2 * params,
+                "flops": 6.0 * case["batch"] * n - 2.0 * case["batch"] * widths[0] * widths[1]}
+    if kind == "compress":
+        nfft = 1 << case["length"].bit_length()
+        return {"bytes": case["echoes"] * (4.0 * case["length"] + 8.0 * 4096 + 12),
+                "flops": _fft_flops(nfft, 3 * case["echoes"])}
+    if kind == "windows":
+        _, pulses = subaperture.sliding_windows(case["dwell"], case["count"], seed=7)
+        per = [_frame_work(int(m), case["cells"]) for m in pulses]
+        return {"bytes": 8.0 * case["dwell"] * (case["cells"] + 1) + 4.0 * W * float(pulses.sum()),
+                "flops": sum(f for _, f in per)}
+    M, K = case["pulses"], case["frames"]
+    if kind == "judge":   # the kept cut and phases in, the image and entropies out
+        return {"bytes": K * (8.0 * M * W + 8.0 * M + 4.0 * M * W + 8),
+                "flops": K * (_fft_flops(2 * M, 2 * W) + _fft_flops(W, 2 * M) + 6.0 * M * W)}
+    b, f = _frame_work(M, case["cells"], case["iterations"], mtrc=case["mtrc"])
+    return {"bytes": K * b, "flops": K * f}
+
+
+# ------------------------------------------------------------------------------------------
+# the same outputs in 64 bits
+# ------------------------------------------------------------------------------------------
+def _hamming64(n):
+    k = torch.arange(n, dtype=torch.float64, device=DEV)
+    return 0.54 - 0.46 * torch.cos(2 * math.pi * k / (n - 1))
+
+
+def _cis(phase):
+    return torch.polar(torch.ones_like(phase), phase)
+
+
+def _align64(S):
+    """Hierarchical correlation alignment of (K, M, N) rows; returns the aligned range profiles."""
+    K, M, N = S.shape
+    k = torch.arange(N, dtype=torch.float64, device=DEV)
+    S = S * (_hamming64(N) * (1 - 2 * (k % 2)))
+    s = 1
+    while s < M:
+        groups = -(-M // s)
+        e = torch.fft.ifft(S, dim=2)
+        e = e.real ** 2 + e.imag ** 2
+        if groups * s != M:
+            e = torch.cat([e, torch.zeros((K, groups * s - M, N), dtype=e.dtype, device=DEV)], dim=1)
+        g = e.reshape(K, groups, s, N).sum(2).sqrt()
+        del e
+        pairs = groups // 2
+        a, b = g[:, 0:2 * pairs:2], g[:, 1:2 * pairs:2]
+        c = torch.fft.ifft(torch.fft.fft(a, dim=2) * torch.fft.fft(b, dim=2).conj(), dim=2).real * N
+        c = torch.roll(c, -(N // 2), dims=2)
+        i = c.abs().argmax(dim=2, keepdim=True)
+        f1, f2, f3 = (c.gather(2, (i + d) % N) for d in (-1, 0, 1))
+        fa, fb = (f1 + f3 - 2 * f2) / 2, (f3 - f1) / 2
+        delta = torch.where((i > 0) & (i < N - 1) & (fa != 0), -fb / (2 * torch.where(fa != 0, fa, 1.0)), 0.0)
+        lag = (i + delta - N / 2)[..., 0]
+        for p in range(pairs):
+            r0, r1 = (2 * p + 1) * s, min(M, (2 * p + 2) * s)
+            S[:, r0:r1] *= _cis(-2 * math.pi * (lag[:, p:p + 1] * k / N))[:, None, :]
+        s *= 2
+    return torch.fft.ifft(S, dim=2)
+
+
+def _centre_cut64(P):
+    """Centring shift and range window of one frame's profiles (M, N): the (M, 512) cut."""
+    M, N = P.shape
+    a = P.abs()
+    arp = (a / a.max()).sum(0).div(M).cpu().numpy()
+    srt = np.sort(arp)
+    inter, half = 30, 4
+    d = np.abs(srt[inter:] - srt[:-inter] - inter * np.abs(srt).max() / N)
+    thr = srt[int(np.argmin(d)) + inter // 2]
+    idx = np.nonzero(arp > thr)[0]
+    run = np.concatenate([[0.0], np.cumsum(arp)])
+    lo, hi = np.maximum(idx - half, 0), np.minimum(idx + half, N - 1)
+    total = run[hi + 1] - run[lo]
+    div = np.where(idx - half < 0, half + idx + 1.0, np.where(idx + half > N - 1, N - idx - half - 1.0, 2 * half + 1.0))
+    kept = idx[total / div >= thr]
+    shift = 0
+    if kept.size:
+        shift = -(int(kept.sum()) // int(kept.size) - N // 2)
+    P = torch.roll(P, shift, dims=1)
+    key = P[0].real.abs() + P[0].imag.abs()
+    off = min(max(int(key.argmax()) - W // 2, 0), N - W)
+    return P[:, off:off + W]
+
+
+def _tracking64(X):
+    """Doppler-centroid phase of (M, cols), 0 for the first pulse."""
+    ang = torch.cumsum(torch.angle((X[:-1].conj() * X[1:]).sum(1)), 0)
+    return torch.cat([torch.zeros(1, dtype=X.dtype, device=DEV), _cis(-ang)])
+
+
+def _select64(X):
+    M = X.shape[0]
+    top = X.abs().amax(0)
+    thr = float(np.float32(1.48) * (np.float32(int(top.trunc().sum())) / np.float32(W)))
+    tgt = int((top > thr).sum())
+    img = torch.fft.fft(_tracking64(X)[:, None] * X, dim=0)
+    p = img.real ** 2 + img.imag ** 2
+    E = p.sum(0)
+    q = p / E
+    H = -(torch.where(q > 0, q * torch.log(q), 0.0)).sum(0)
+    order = torch.argsort(E, descending=True, stable=True)[:tgt]
+    order = order[torch.argsort(H[order], stable=True)]
+    U = 2 << max(0, (tgt // 2).bit_length() - 1) if tgt // 2 else 2
+    bins = torch.zeros(U, dtype=torch.int64, device=DEV)
+    bins[:min(U, tgt)] = order[:U]
+    return torch.sort(bins)[0]
+
+
+def _autofocus64(X, iterations):
+    """(K, M, W) cuts to their phases (K, M)."""
+    K, M, _ = X.shape
+    bins = [_select64(x) for x in X]
+    U = max(b.numel() for b in bins)
+    S = torch.zeros((K, M, U), dtype=X.dtype, device=DEV)
+    phi = torch.empty((K, M), dtype=X.dtype, device=DEV)
+    for f in range(K):
+        sel = X[f][:, bins[f]]
+        phi[f] = _tracking64(sel)
+        S[f, :, :bins[f].numel()] = sel
+    conj = S.conj()
+    for _ in range(iterations):
+        G = torch.fft.fft(phi[:, :, None] * S, dim=1)
+        acc = (conj * torch.fft.ifft(G * G.abs(), dim=1)).sum(2)
+        phi = acc / acc.abs()
+    return phi
+
+
+def _form64(X, phi, header, ifds, mtrc, quirk):
+    """Image formation of (K, M, W) cuts with their phases."""
+    K, M, _ = X.shape
+    X = X * phi[:, :, None]
+    if mtrc:
+        B, fc = float(header["band_width"]), float(header["fc"])
+        X = torch.roll(X, W // 2, dims=2)
+        X = torch.fft.fft(X, dim=2) if ifds else torch.fft.ifft(X, dim=2)
+        n = torch.arange(W, dtype=torch.float64, device=DEV)
+        alpha = 1.0 - B / (2 * fc) + B / (fc * (W - 1.0)) * n
+        F = 2 * M if M & (M - 1) == 0 else 1 << (2 * M - 1).bit_length()
+        m = torch.arange(M, dtype=torch.float64, device=DEV)
+        quad = _cis(math.pi * (m ** 2)[:, None] * alpha / M)
+        filt = torch.zeros((F, W), dtype=torch.complex128, device=DEV)
+        filt[:M] = quad
+        filt[F - M + 1:] = quad[1:].flip(0)
+        pre = quad.conj() * _cis(math.pi * m[:, None] * alpha)
+        Y = torch.fft.fft(X * pre, n=F, dim=1) * torch.fft.fft(filt, dim=0)
+        X = torch.fft.ifft(Y, dim=1)[:, :M] * quad.conj()
+        del Y
+        X = torch.roll(torch.fft.ifft(torch.roll(X, M // 2, dims=1), dim=1), M // 2, dims=1)
+        X = torch.roll(torch.roll(torch.fft.fft(X, dim=2), W // 2, dims=2), M // 2, dims=1)
+        if ifds:
+            X = X.flip(2)
+    h = _hamming64(M)
+    if quirk:
+        X = X.clone()
+        X[:, 0] = X[:, 0] * h[torch.arange(W, device=DEV) // M]
+    else:
+        X = X * h[:, None]
+    X = torch.roll(torch.fft.fft(X, dim=1), M // 2, dims=1)
+    if ifds:
+        X = X.flip(1)
+    return X.abs()
+
+
+def _cuts64(echo, vel, header, ifds, hpc):
+    """Aligned, centred and cut frames of float32 echoes (K, M, N, 2)."""
+    S = torch.view_as_complex(echo.to(torch.float64).contiguous())
+    N = S.shape[2]
+    if ifds:
+        S = torch.roll(torch.fft.ifft(torch.roll(S, N // 2, dims=2), dim=2), N // 2, dims=2)
+    elif hpc:
+        t = torch.arange(N, dtype=torch.float64, device=DEV) / float(header["Fs"])
+        coef = -4 * math.pi * (float(header["band_width"]) / header["Tp"]) / LIGHT
+        S = S * _cis(coef * vel[:, :, None] * t ** 2)
+    P = _align64(S)
+    del S
+    return torch.stack([_centre_cut64(p) for p in P])
+
+
+def _images64(echo, vel, header, iterations=120, ifds=False, hpc=True, mtrc=True, quirk=True):
+    K, M, N = echo.shape[:3]
+    step = max(1, (1 << 26) // (M * N))
+    out = []
+    for i in range(0, K, step):
+        X = _cuts64(echo[i:i + step], vel[i:i + step], header, ifds, hpc)
+        out.append(_form64(X, _autofocus64(X, iterations), header, ifds, mtrc, quirk))
+    return torch.cat(out)
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "train":
+        widths, params, x, target = _net(case, seed)
+        flat = torch.from_numpy(params).to(DEV).double().requires_grad_()
+        a, at = x.double(), 0
+        for i, (n, o) in enumerate(zip(widths[:-1], widths[1:])):
+            w, b = flat[at:at + n * o].reshape(n, o), flat[at + n * o:at + n * o + o]
+            at += n * o + o
+            a = a @ w + b
+            if i + 2 < len(widths):
+                a = torch.relu(a)
+        d = a - target.double()
+        loss = d.square().mean()
+        loss.backward()
+        return {"pred": a.detach(), "loss": d.detach().square().sum(1) / d.numel(), "grads": flat.grad}
+    if kind == "compress":
+        iq, vel, h = _echoes(case, seed)
+        nfft = 1 << case["length"].bit_length()
+        x = torch.complex(iq[..., 0].double(), iq[..., 1].double())
+        S = int(h["Fs"] * h["Tp"])
+        v2 = (2 * vel / LIGHT)[:, None]
+        k = torch.arange(S, dtype=torch.float64, device=DEV)
+        t = (1 - v2) * (-h["Tp"] / 2 + k * h["Tp"] / (S - 1))
+        ref = _cis((-2 * math.pi * h["fc"] * v2 / (1 - v2) + math.pi * h["band_width"] / h["Tp"] * t) * t) * _hamming64(S)
+        y = torch.fft.ifft(torch.fft.fft(ref, n=nfft, dim=1).conj() * torch.fft.fft(x, n=nfft, dim=1), dim=1)
+        off = ((y.real.abs() + y.imag.abs()).argmax(1) - 2048).clamp(0, nfft - 4096)
+        y = y.gather(1, off[:, None] + torch.arange(4096, device=DEV))
+        return {"profiles": torch.view_as_real(y), "offsets": off.to(torch.int32)}
+    if kind == "windows":
+        echo, vel, h, first, pulses = _windows(case, seed)
+        out = [None] * len(pulses)
+        for m in sorted(set(int(p) for p in pulses)):
+            at = [i for i, p in enumerate(pulses) if p == m]
+            e = torch.stack([echo[first[i]:first[i] + m] for i in at])
+            v = torch.stack([vel[first[i]:first[i] + m] for i in at])
+            for i, img in zip(at, _images64(e, v, h)):
+                out[i] = img.reshape(-1)
+        return {"images": torch.cat(out)}
+    echo, vel, h = _frames(case, seed)
+    if kind == "judge":
+        phi = torch.view_as_complex(_phases(case, seed).double())
+        X = torch.cat([_cuts64(echo[i:i + 16], vel[i:i + 16], h, False, True) for i in range(0, echo.shape[0], 16)])
+        n, img = X.shape[0], []
+        for i in range(0, case["frames"], n):
+            q = phi[i:i + n]
+            img.append(_form64(X[:q.shape[0]], q, h, False, True, True))
+        img = torch.cat(img)
+        p = img.square().reshape(case["frames"], -1)
+        p = p / p.sum(1, keepdim=True)
+        return {"images": img, "entropy": -torch.where(p > 0, p * torch.log(p), 0.0).sum(1)}
+    img = _images64(echo, vel, h, case["iterations"], case["type"] == 1, case["hpc"] and case["type"] == 2, case["mtrc"],
+                    case["quirk"])
+    if case["frames"] != img.shape[0]:
+        img = img[torch.arange(case["frames"], device=DEV) % img.shape[0]]
+    return {"images": img}
