@@ -6,8 +6,8 @@ A case is a dict of plain values with a "kind":
   image     one call of Imager.run_device: K frames in device memory to K images
   windows   one call of SubaperturePlan.run: windows of uneven pulse counts of one dwell
   compress  one call of isar_pulse_compress: raw IFDS echoes to compressed profiles
-  judge     one image formation from given phases (a BACK run) and its entropies, as the
-            warm start judges a candidate
+  judge     one image formation from candidate phases (a BACK run), its entropies and the choice
+            between candidate and incumbent, as the warm start judges a start
   train     one training step of the warm-start network up to its gradients
 
 `exact` gives the same outputs in 64 bits from plain torch.
@@ -145,9 +145,9 @@ def _radar(case, header):
                             header["Fs"])
 
 
-def _phases(case, seed):
+def _phases(case, seed, which):
     """Per-pulse phases as a warm start proposes them: a smooth drift and noise."""
-    g = torch.Generator().manual_seed(seed + 17)
+    g = torch.Generator().manual_seed(2 * seed + 17 + which)
     M, K = case["pulses"], case["frames"]
     t = torch.linspace(-1, 1, M, dtype=torch.float64)
     c = torch.randn((K, 3), generator=g, dtype=torch.float64)
@@ -226,15 +226,25 @@ def prepare(case, seed):
     if kind == "judge":
         im.run_device(echo.data_ptr(), vel.data_ptr(), 0, case["frames"], isar.Options(iterations=1, stage_mode=1),
                       stream=stream)
-        state["phi"] = _phases(case, seed)
-        state["entropy"] = torch.empty(case["frames"], dtype=torch.float64, device=DEV)
         state["options"] = isar.Options(iterations=0, stage_mode=2, warm_start=True)
+        state["phi"], state["phi_best"] = _phases(case, seed, 0), _phases(case, seed, 1)
+        state["start"] = torch.empty_like(state["phi"])
+        state["entropy"], state["entropy_best"] = (torch.empty(case["frames"], dtype=torch.float64, device=DEV)
+                                                   for _ in range(2))
+        _judge(state, "phi_best", "entropy_best")
         return state
     im.set_autofocus_mode(case["form"])
     im.set_ra_chunk(min(case["chunk"], case["pulses"] // 2))
     im.set_graph_mode(case["graph"])
     state["options"] = _options(case)
     return state
+
+
+def _judge(state, phi, entropy):
+    case, K = state["case"], state["case"]["frames"]
+    state["im"].run_device(0, 0, state["img"].data_ptr(), K, state["options"], phi0_ptr=state[phi].data_ptr(),
+                           stream=state["stream"])
+    learned.image_entropy(K, case["pulses"] * W, state["img"].data_ptr(), state[entropy].data_ptr(), state["stream"])
 
 
 def run(state):
@@ -260,12 +270,11 @@ def run(state):
                           graph=True, stream=state["stream"])
         return {"images": state["img"]}
     if kind == "judge":
-        K = case["frames"]
-        state["im"].run_device(0, 0, state["img"].data_ptr(), K, state["options"], phi0_ptr=state["phi"].data_ptr(),
-                               stream=state["stream"])
-        learned.image_entropy(K, case["pulses"] * W, state["img"].data_ptr(), state["entropy"].data_ptr(),
-                              state["stream"])
-        return {"images": state["img"], "entropy": state["entropy"]}
+        _judge(state, "phi", "entropy")
+        learned.select_phase(case["frames"], case["pulses"], state["phi_best"].data_ptr(),
+                             state["entropy_best"].data_ptr(), state["phi"].data_ptr(), state["entropy"].data_ptr(),
+                             state["start"].data_ptr(), state["stream"])
+        return {"images": state["img"], "start": state["start"]}
     state["im"].run_device(state["echo"].data_ptr(), state["vel"].data_ptr(), state["img"].data_ptr(), case["frames"],
                            state["options"], stream=state["stream"])
     return {"images": state["img"]}
@@ -308,8 +317,8 @@ def work(case):
         return {"bytes": 8.0 * case["dwell"] * (case["cells"] + 1) + 4.0 * W * float(pulses.sum()),
                 "flops": sum(f for _, f in per)}
     M, K = case["pulses"], case["frames"]
-    if kind == "judge":   # the kept cut and phases in, the image and entropies out
-        return {"bytes": K * (8.0 * M * W + 8.0 * M + 4.0 * M * W + 8),
+    if kind == "judge":   # the kept cut and both phases in, the image and the chosen phase out
+        return {"bytes": K * (8.0 * M * W + 3 * 8.0 * M + 4.0 * M * W),
                 "flops": K * (_fft_flops(2 * M, 2 * W) + _fft_flops(W, 2 * M) + 6.0 * M * W)}
     b, f = _frame_work(M, case["cells"], case["iterations"], mtrc=case["mtrc"])
     return {"bytes": K * b, "flops": K * f}
@@ -526,16 +535,19 @@ def exact(case, seed):
         return {"images": torch.cat(out)}
     echo, vel, h = _frames(case, seed)
     if kind == "judge":
-        phi = torch.view_as_complex(_phases(case, seed).double())
+        phases = [_phases(case, seed, i) for i in range(2)]
         X = torch.cat([_cuts64(echo[i:i + 16], vel[i:i + 16], h, False, True) for i in range(0, echo.shape[0], 16)])
-        n, img = X.shape[0], []
-        for i in range(0, case["frames"], n):
-            q = phi[i:i + n]
-            img.append(_form64(X[:q.shape[0]], q, h, False, True, True))
-        img = torch.cat(img)
-        p = img.square().reshape(case["frames"], -1)
-        p = p / p.sum(1, keepdim=True)
-        return {"images": img, "entropy": -torch.where(p > 0, p * torch.log(p), 0.0).sum(1)}
+        n, images, entropies = X.shape[0], [], []
+        for phi in phases:
+            q = torch.view_as_complex(phi.double())
+            img = torch.cat([_form64(X[:q[i:i + n].shape[0]], q[i:i + n], h, False, True, True)
+                             for i in range(0, case["frames"], n)])
+            p = img.square().reshape(case["frames"], -1)
+            p = p / p.sum(1, keepdim=True)
+            images.append(img)
+            entropies.append(-torch.where(p > 0, p * torch.log(p), 0.0).sum(1))
+        take = entropies[0] < entropies[1]
+        return {"images": images[0], "start": torch.where(take[:, None, None], phases[0], phases[1]).double()}
     img = _images64(echo, vel, h, case["iterations"], case["type"] == 1, case["hpc"] and case["type"] == 2, case["mtrc"],
                     case["quirk"])
     if case["frames"] != img.shape[0]:
