@@ -7,16 +7,15 @@ namespace isar {
 template <int N, int E, int DIR>
 __global__ __launch_bounds__(N / E) void k_debug_fft(const float2* in, float2* out) {
     HIP_DYNAMIC_SHARED(float2, lds);
-    constexpr int R0 = FftPlan<N, E>::R[0];
-    constexpr int RL = FftPlan<N, E>::R[FftPlan<N, E>::NP - 1];
+    constexpr bool REV = DIR > 0;   // inverse transforms in the reversed order, as the column kernels run them
     const size_t base = static_cast<size_t>(blockIdx.x) * N;
     const int tid = threadIdx.x;
     float2 x[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) x[e] = in[base + fft_in_pos<N, E, R0>(tid, e)];
-    fft<N, E, DIR>(x, lds, tid);
+    for (int e = 0; e < E; ++e) x[e] = in[base + fft_in_pos<N, E, REV>(tid, e)];
+    fft<N, E, DIR, false, REV>(x, lds, tid);
 #pragma unroll
-    for (int e = 0; e < E; ++e) out[base + fft_out_pos<N, E, RL>(tid, e)] = x[e];
+    for (int e = 0; e < E; ++e) out[base + fft_out_pos<N, E, REV>(tid, e)] = x[e];
 }
 
 // 256 / (N / E) transforms per workgroup, each on N / E threads of one wave with its own LDS
@@ -27,19 +26,18 @@ template <int N, int E, int DIR>
 __global__ __launch_bounds__(256) void k_debug_fft_grouped(const float2* in, float2* out, int batch) {
     HIP_DYNAMIC_SHARED(float2, lds);
     constexpr int TPF = N / E, G = 256 / TPF;
-    constexpr int R0 = FftPlan<N, E>::R[0];
-    constexpr int RL = FftPlan<N, E>::R[FftPlan<N, E>::NP - 1];
+    constexpr bool REV = DIR > 0;   // inverse transforms in the reversed order, as the column kernels run them
     const int g = threadIdx.x / TPF, lane = threadIdx.x % TPF;
     const int t = blockIdx.x * G + g;
     const bool valid = t < batch;
     const size_t base = static_cast<size_t>(valid ? t : 0) * N;
     float2 x[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) x[e] = valid ? in[base + fft_in_pos<N, E, R0>(lane, e)] : make_float2(0.0f, 0.0f);
-    fft<N, E, DIR, true>(x, lds + g * lds_padded_size(N), lane);
+    for (int e = 0; e < E; ++e) x[e] = valid ? in[base + fft_in_pos<N, E, REV>(lane, e)] : make_float2(0.0f, 0.0f);
+    fft<N, E, DIR, true, REV>(x, lds + g * lds_padded_size(N), lane);
     if (valid) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) out[base + fft_out_pos<N, E, RL>(lane, e)] = x[e];
+        for (int e = 0; e < E; ++e) out[base + fft_out_pos<N, E, REV>(lane, e)] = x[e];
     }
 }
 

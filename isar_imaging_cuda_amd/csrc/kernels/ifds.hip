@@ -10,11 +10,7 @@ namespace isar {
 namespace {
 constexpr int kPcE = 16;
 template <int NF>
-__device__ __forceinline__ int pc_in(int tid, int e) { return fft_in_pos<NF, kPcE, FftPlan<NF, kPcE>::R[0]>(tid, e); }
-template <int NF>
-__device__ __forceinline__ int pc_out(int tid, int e) {
-    return fft_out_pos<NF, kPcE, FftPlan<NF, kPcE>::R[FftPlan<NF, kPcE>::NP - 1]>(tid, e);
-}
+__device__ __forceinline__ int pc_in(int tid, int e) { return fft_in_pos<NF, kPcE>(tid, e); }
 }  // namespace
 
 // iq: echoes x len int16 I/Q pairs; out: echoes x cut complex. Phases of the reference chirp in FP64.
@@ -54,15 +50,14 @@ __global__ __launch_bounds__(NF / kPcE) void k_pulse_compress(PcJob P) {
     fft<NF, kPcE, -1>(x, lds, tid);
 #pragma unroll
     for (int e = 0; e < kPcE; ++e) x[e] = cconjmul(r[e], x[e]);   // elementwiseMultiplyConjA
-    relayout_out_to_in<NF, kPcE>(x, lds, tid);
-    fft<NF, kPcE, +1>(x, lds, tid);
+    fft<NF, kPcE, +1, false, true>(x, lds, tid);   // back to the layout of the echo
     const float inv = 1.0f / NF;
     float best = -1.0f;
     int bi = 0;
 #pragma unroll
     for (int e = 0; e < kPcE; ++e) {
         x[e] = cscale(x[e], inv);
-        const int k = pc_out<NF>(tid, e);
+        const int k = pc_in<NF>(tid, e);
         const float a = fabsf(x[e].x) + fabsf(x[e].y);   // cublasIcamax: |Re| + |Im|, first index
         if (a > best || (a == best && k < bi)) { best = a; bi = k; }
     }
@@ -72,7 +67,7 @@ __global__ __launch_bounds__(NF / kPcE) void k_pulse_compress(PcJob P) {
     float2* dst = P.out + static_cast<size_t>(echo) * P.cut;
 #pragma unroll
     for (int e = 0; e < kPcE; ++e) {
-        const int k = pc_out<NF>(tid, e) - off;
+        const int k = pc_in<NF>(tid, e) - off;
         if (k >= 0 && k < P.cut) dst[k] = x[e];
     }
     if (tid == 0 && P.offsets) P.offsets[echo] = off;

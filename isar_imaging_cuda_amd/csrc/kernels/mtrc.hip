@@ -31,18 +31,14 @@ struct CztCfg {
     static constexpr int NT = NT_;
     static constexpr int CT = NT / TPF;
     static_assert(F % E == 0 && NT % TPF == 0, "chirp-z tile");
-    static constexpr int R0 = FftPlan<F, E>::R[0];
-    static constexpr int RL = FftPlan<F, E>::R[FftPlan<F, E>::NP - 1];
-    __device__ static int in(int lane, int e) { return fft_in_pos<F, E, R0>(lane, e); }
-    __device__ static int out(int lane, int e) { return fft_out_pos<F, E, RL>(lane, e); }
+    __device__ static int in(int lane, int e) { return fft_in_pos<F, E>(lane, e); }
+    __device__ static int out(int lane, int e) { return fft_out_pos<F, E>(lane, e); }
 };
 
 template <int W>
-__device__ __forceinline__ int row_in(int lane, int e) { return fft_in_pos<W, kRowE, FftPlan<W, kRowE>::R[0]>(lane, e); }
+__device__ __forceinline__ int row_in(int lane, int e) { return fft_in_pos<W, kRowE>(lane, e); }
 template <int W>
-__device__ __forceinline__ int row_out(int lane, int e) {
-    return fft_out_pos<W, kRowE, FftPlan<W, kRowE>::R[FftPlan<W, kRowE>::NP - 1]>(lane, e);
-}
+__device__ __forceinline__ int row_out(int lane, int e) { return fft_out_pos<W, kRowE>(lane, e); }
 }  // namespace
 
 // Bluestein filter spectra: table[n][:] = FFT_F(v), v[t] = exp(+j pi alpha_n t^2 / M) for
@@ -113,49 +109,63 @@ __global__ __launch_bounds__(kRowsPerBlock * W / kRowE) void k_mtrc_rows(Job J) 
 // Chirp-z transform along slow time for a tile of range bins (mtrc.cu:42-52, 125-192):
 // X[k] = exp(-j pi a k^2/M) / F * IFFT_F( FFT_F(y) * table_n )[k],
 // y[m] = x[m] exp(j pi a m (M - m) / M) for m < M. Also writes sum_k X[k] per bin.
-template <int F, int NTW>
-__global__ __launch_bounds__(NTW) void k_mtrc_czt(Job J) {
+// HALF: F = 2 M (a power of two), so slots 8 ... 15 of every thread lie past M: they are zero going in and
+// not formed coming out, with their table entries and transposes.
+template <int F, int NTW, bool HALF>
+__global__ __launch_bounds__(NTW, 4) void k_mtrc_czt(Job J) {
     using C = CztCfg<F, NTW>;
     constexpr int CT = C::CT, TPF = C::TPF, E = C::E, NT = C::NT;
+    constexpr int EM = HALF ? E / 2 : E;   // slots that can lie before M
     HIP_DYNAMIC_SHARED(float2, sm);
     const int tile = xcd_tile(blockIdx.x, gridDim.x), f = blockIdx.y, tid = threadIdx.x;
-    const int M = J.M, W = J.W;
+    const int M = HALF ? F / 2 : J.M, W = J.W;
     const int g = tid / TPF, lane = tid % TPF;
     const int n0 = tile * CT, n = n0 + g;
-    const float2* S = J.stm + static_cast<size_t>(f) * M * W;
-    for (int idx = tid; idx < M * CT; idx += NT) {
-        const int m = idx / CT, c = idx % CT;
-        sm[m * (CT + 1) + c] = S[static_cast<size_t>(m) * W + n0 + c];
-    }
-    __syncthreads();
     const float2* pre = J.czt_pre + static_cast<size_t>(n) * M;
     const float2* post = J.czt_post + static_cast<size_t>(n) * M;
+    auto pos = [&](int e) { return HALF ? C::in(lane, e) : min(C::in(lane, e), M - 1); };
+    auto before_m = [&](int e) { return HALF || C::in(lane, e) < M; };
+    // the table rows are read ahead of their use, in full (past M the last entry, which is not used):
+    // one at a time under a test of the position they cost more than the transforms
+    float2 pre_v[EM];
+#pragma unroll
+    for (int e = 0; e < EM; ++e) pre_v[e] = pre[pos(e)];
+    load_column_tile<NT, CT>(J.stm + static_cast<size_t>(f) * M * W, W, n0, M, sm, tid);
+    __syncthreads();
     float2 x[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int pos = C::in(lane, e);
-        x[e] = pos < M ? cmul(sm[pos * (CT + 1) + g], pre[pos]) : make_float2(0.0f, 0.0f);
+    for (int e = 0; e < EM; ++e) {
+        const float2 y = cmul(sm[pos(e) * (CT + 1) + g], pre_v[e]);
+        x[e] = before_m(e) ? y : make_float2(0.0f, 0.0f);
     }
     __syncthreads();
     // a transform within one wave orders its passes by the wave alone (the transpose back below
     // waits for every wave with a barrier of its own)
     constexpr bool kWave = TPF <= 64;
     float2* buf = sm + g * lds_padded_size(F);
-    const FftTwiddles<F, E> tw = fft_twiddles<F, E>(lane);
-    fft<F, E, -1, kWave>(x, buf, lane, tw);
+    if constexpr (HALF && FftPlan<F, E>::R[0] == 16) fft_zero_half<F, -1, kWave>(x, buf, lane);
+    else fft<F, E, -1, kWave>(x, buf, lane);
     const float2* tab = J.czt_table + static_cast<size_t>(n) * F;
+    {
+        float2 t[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) x[e] = cmul(x[e], tab[C::out(lane, e)]);
-    relayout_out_to_in<F, E, kWave>(x, buf, lane);
-    fft<F, E, +1, kWave>(x, buf, lane, tw);
+        for (int e = 0; e < E; ++e) t[e] = tab[C::out(lane, e)];
+        issue_point();
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] = cmul(x[e], t[e]);
+    }
+    fft<F, E, +1, kWave, true>(x, buf, lane);   // back to the layout of the input
     float2 csum = make_float2(0.0f, 0.0f);
-    float2 y[E];
+    float2 y[EM];
+    {
+        float2 p[EM];
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int k = C::out(lane, e);
-        y[e] = make_float2(0.0f, 0.0f);
-        if (k < M) {
-            y[e] = cmul(x[e], post[k]);
+        for (int e = 0; e < EM; ++e) p[e] = post[pos(e)];
+        issue_point();
+#pragma unroll
+        for (int e = 0; e < EM; ++e) {
+            const float2 v = cmul(x[e], p[e]);
+            y[e] = before_m(e) ? v : make_float2(0.0f, 0.0f);
             csum = cadd(csum, y[e]);
         }
     }
@@ -178,10 +188,8 @@ __global__ __launch_bounds__(NTW) void k_mtrc_czt(Job J) {
     }
     // transpose back through LDS for row-contiguous stores
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int k = C::out(lane, e);
-        if (k < M) sm[k * (CT + 1) + g] = y[e];
-    }
+    for (int e = 0; e < EM; ++e)
+        if (before_m(e)) sm[C::in(lane, e) * (CT + 1) + g] = y[e];
     __syncthreads();
     float2* D = J.czt + static_cast<size_t>(f) * M * W;
     for (int idx = tid; idx < M * CT; idx += NT) {
@@ -201,25 +209,20 @@ __global__ __launch_bounds__(256) void k_col_window(Job J) {
     const int g = tid / TPF, lane = tid % TPF;
     const int n0 = tile * CT;
     float2* D = J.czt + static_cast<size_t>(f) * M * W;
-    for (int idx = tid; idx < M * CT; idx += NT) {
-        const int m = idx / CT, c = idx % CT;
-        sm[m * (CT + 1) + c] = D[static_cast<size_t>(m) * W + n0 + c];
-    }
+    load_column_tile<NT, CT>(D, W, n0, M, sm, tid);
     __syncthreads();
     float2 x[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) x[e] = sm[((C::in(lane, e) + M / 2) % M) * (CT + 1) + g];
     __syncthreads();
     float2* buf = sm + g * lds_padded_size(M);
-    const FftTwiddles<M, E> tw = fft_twiddles<M, E>(lane);
-    fft<M, E, +1>(x, buf, lane, tw);
+    fft<M, E, +1>(x, buf, lane);
     const float invM = 1.0f / M;
 #pragma unroll
     for (int e = 0; e < E; ++e) x[e] = cscale(x[e], invM * hamming(C::out(lane, e), M));
-    relayout_out_to_in<M, E>(x, buf, lane);
-    fft<M, E, -1>(x, buf, lane, tw);
+    fft<M, E, -1, false, true>(x, buf, lane);
 #pragma unroll
-    for (int e = 0; e < E; ++e) sm[((C::out(lane, e) + M / 2) % M) * (CT + 1) + g] = x[e];
+    for (int e = 0; e < E; ++e) sm[((C::in(lane, e) + M / 2) % M) * (CT + 1) + g] = x[e];
     __syncthreads();
     for (int idx = tid; idx < M * CT; idx += NT) {
         const int m = idx / CT, c = idx % CT;
@@ -297,12 +300,10 @@ __global__ __launch_bounds__(256) void k_post_nomtrc(Job J) {
     const int W = J.W;
     const int g = tid / TPF, lane = tid % TPF;
     const int n0 = tile * CT, n = n0 + g;
-    const float2* X = J.x + static_cast<size_t>(f) * M * W;
-    const float2* ph = J.phi + static_cast<size_t>(f) * M;
-    for (int idx = tid; idx < M * CT; idx += NT) {
-        const int m = idx / CT, c = idx % CT;
-        sm[m * (CT + 1) + c] = cmul(X[static_cast<size_t>(m) * W + n0 + c], ph[m]);
-    }
+    float2 phi[E];   // read ahead of the tile
+#pragma unroll
+    for (int e = 0; e < E; ++e) phi[e] = elem_u32(J.phi + static_cast<size_t>(f) * M, static_cast<unsigned>(C::in(lane, e)));
+    load_column_tile<NT, CT>(J.x + static_cast<size_t>(f) * M * W, W, n0, M, sm, tid);
     __syncthreads();
     float2 x[E];
     const bool quirk = J.quirk_q1 != 0;
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(256) void k_post_nomtrc(Job J) {
         float w = 1.0f;
         if (quirk) { if (pos == 0) w = hamming(n / M, M); }
         else w = hamming(pos, M);
-        x[e] = cscale(sm[pos * (CT + 1) + g], w);
+        x[e] = cscale(cmul(sm[pos * (CT + 1) + g], phi[e]), w);
     }
     __syncthreads();
     float2* buf = sm + g * lds_padded_size(M);
@@ -383,8 +384,12 @@ hipError_t configure_mtrc_kernels() {
     };
 #define ISAR_SET_F(FF)                                                                          \
     set(reinterpret_cast<const void*>(&k_czt_table<FF>), lds_padded_size(FF) * sizeof(float2)); \
-    set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, 256>), czt_lds<FF, 256>(FF / 2));         \
-    set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, 512>), czt_lds<FF, 512>(FF / 2));
+    set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, 256, false>), czt_lds<FF, 256>(FF / 2));  \
+    set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, 512, false>), czt_lds<FF, 512>(FF / 2));  \
+    if constexpr (FF % 3 != 0) {                                                                 \
+        set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, 256, true>), czt_lds<FF, 256>(FF / 2)); \
+        set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, 512, true>), czt_lds<FF, 512>(FF / 2)); \
+    }
     ISAR_SET_F(128) ISAR_SET_F(256) ISAR_SET_F(384) ISAR_SET_F(512) ISAR_SET_F(768) ISAR_SET_F(1024) ISAR_SET_F(2048)
 #undef ISAR_SET_F
 #define ISAR_SET_M(MM)                                                         \
@@ -413,13 +418,25 @@ void launch_mtrc_rows(const Job& J, hipStream_t s) {
     ISAR_LAUNCH(k_mtrc_rows<kRangeCut>, dim3((J.M + kRowsPerBlock - 1) / kRowsPerBlock, J.K),
                 dim3(kRowsPerBlock * kRangeCut / kRowE), rows_lds(), s, J);
 }
+namespace {
+template <int F, int NTW>
+void mtrc_czt(const Job& J, hipStream_t s) {
+    const dim3 grid(J.W / CztCfg<F, NTW>::CT, J.K);
+    const size_t lds = czt_lds<F, NTW>(J.M);
+    if constexpr (F % 3 != 0) {
+        if (2 * J.M == F) {
+            ISAR_LAUNCH((k_mtrc_czt<F, NTW, true>), grid, dim3(NTW), lds, s, J);
+            return;
+        }
+    }
+    ISAR_LAUNCH((k_mtrc_czt<F, NTW, false>), grid, dim3(NTW), lds, s, J);
+}
+}  // namespace
 void launch_mtrc_czt(const Job& J, hipStream_t s) {
     if (J.czt_threads == 512) {
-        ISAR_F_SWITCH(J.F, ISAR_LAUNCH((k_mtrc_czt<FF, 512>), dim3(J.W / CztCfg<FF, 512>::CT, J.K), dim3(512),
-                                       (czt_lds<FF, 512>(J.M)), s, J));
+        ISAR_F_SWITCH(J.F, (mtrc_czt<FF, 512>(J, s)));
     } else {
-        ISAR_F_SWITCH(J.F, ISAR_LAUNCH((k_mtrc_czt<FF, 256>), dim3(J.W / CztCfg<FF, 256>::CT, J.K), dim3(256),
-                                       (czt_lds<FF, 256>(J.M)), s, J));
+        ISAR_F_SWITCH(J.F, (mtrc_czt<FF, 256>(J, s)));
     }
 }
 void launch_col_window(const Job& J, hipStream_t s) {

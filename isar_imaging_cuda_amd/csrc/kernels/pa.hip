@@ -94,26 +94,25 @@ __global__ __launch_bounds__(256) void k_pa_colfft(Job J) {
     using C = ColCfg<M>;
     constexpr int NT = C::NT, CT = C::CT, TPF = C::TPF, E = C::E;
     HIP_DYNAMIC_SHARED(float2, sm);
-    float2* phi = sm;                                    // M
-    float2* work = phi + M;                              // tile / transform buffers
+    float2* work = sm;                                   // tile / transform buffers
     const int tile = xcd_tile(blockIdx.x, gridDim.x), f = blockIdx.y, tid = threadIdx.x;
     const int W = J.W;
     const int g = tid / TPF, lane = tid % TPF;
     const int n0 = tile * CT, n = n0 + g;
 
-    for (int m = tid; m < M; m += NT) phi[m] = J.dopphi[static_cast<size_t>(f) * M + m];
-
-    const float2* X = J.x + static_cast<size_t>(f) * M * W;
-    for (int idx = tid; idx < M * CT; idx += NT) {
-        const int m = idx / CT, c = idx % CT;
-        work[m * (CT + 1) + c] = X[static_cast<size_t>(m) * W + n0 + c];
+    float2 phi[E];   // read ahead of the tile
+    {
+        const float2* d = J.dopphi + static_cast<size_t>(f) * M;
+#pragma unroll
+        for (int e = 0; e < E; ++e) phi[e] = elem_u32(d, static_cast<unsigned>(C::in(lane, e)));
     }
+    load_column_tile<NT, CT>(J.x + static_cast<size_t>(f) * M * W, W, n0, M, work, tid);
     __syncthreads();
     float2 x[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int pos = C::in(lane, e);
-        x[e] = cmul(phi[pos], work[pos * (CT + 1) + g]);
+        x[e] = cmul(phi[e], work[pos * (CT + 1) + g]);
     }
     __syncthreads();
     float2* buf = work + g * lds_padded_size(M);
@@ -327,8 +326,9 @@ __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
     float2* buf = bufs + g * lds_padded_size(M);
     const float invM = 1.0f / static_cast<float>(M);
     const bool resident = U <= CF;   // one chunk: the columns stay in registers
-    // the twiddle powers stay in registers for all iterations' transforms
-    const FftTwiddlePowers<M, E> tw = fft_twiddle_powers<M, E>(fft_twiddles<M, E>(lane));
+    // the twiddle constants stay in registers for all iterations' transforms
+    const auto fwd = fft_twiddles<M, E>(lane);
+    const auto inv = fft_twiddles<M, E, true>(lane);
     float2 s[E];
     for (int it = 0; it < J.iterations; ++it) {
         float2 acc[RPT];
@@ -345,17 +345,12 @@ __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
             float2 x[E];
 #pragma unroll
             for (int e = 0; e < E; ++e) x[e] = cmul(phi[C::in(lane, e)], s[e]);
-            fft<M, E, -1, true>(x, buf, lane, tw);
+            fft<M, E, -1, true>(x, buf, lane, fwd);
 #pragma unroll
             for (int e = 0; e < E; ++e) x[e] = cscale(x[e], cabs_hw(x[e]));
-            relayout_out_to_in<M, E, true>(x, buf, lane);
-            fft<M, E, +1, true>(x, buf, lane, tw);
+            fft<M, E, +1, true, true>(x, buf, lane, inv);   // back to the layout of s
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int pos = C::out(lane, e);
-                const float2 sv = C::same_layout ? s[e] : (valid ? col[pos] : make_float2(0.0f, 0.0f));
-                buf[pos] = af_term<M>(sv, x[e], invM);
-            }
+            for (int e = 0; e < E; ++e) buf[C::in(lane, e)] = af_term<M>(s[e], x[e], invM);
             __syncthreads();
             const int ncol = min(CF, U - c0);
             if constexpr (Q > 1) {
@@ -507,15 +502,22 @@ __device__ __forceinline__ float2* af_part_of(const Job& J, int f, int it) {
     return J.af_part + (static_cast<size_t>(it & 1) * J.K + f) * per_frame;
 }
 
+// Twiddle constants of a column's forward and reversed inverse transform.
+template <int M>
+struct AfTwiddles {
+    decltype(fft_twiddles<M, AfCfg<M>::E>(0)) fwd;
+    decltype(fft_twiddles<M, AfCfg<M>::E, true>(0)) inv;
+    __device__ explicit AfTwiddles(int lane) : fwd(fft_twiddles<M, AfCfg<M>::E>(lane)), inv(fft_twiddles<M, AfCfg<M>::E, true>(lane)) {}
+};
+
 // One iteration's work on one sub-chunk of a frame's selected bins: the SUB columns (column
 // c0 + tid / TPF in s, first-pass layout, zero where invalid) are multiplied by the phase phi
 // (M values), transformed, scaled by |G|, transformed back, multiplied by conj(S) (af_term) and
 // left in bufs; then the per-pulse sums over the sub-chunk's ncol columns, each added column by
 // column, are handed to put(m, sum). Every thread of the workgroup calls it.
 template <int M, typename Put>
-__device__ __forceinline__ void af_subchunk(const float2 (&s)[AfCfg<M>::E], const float2* phi, const float2* col,
-                                            bool valid, int ncol, float2* bufs, int tid,
-                                            const FftTwiddles<M, AfCfg<M>::E>& tw, Put put) {
+__device__ __forceinline__ void af_subchunk(const float2 (&s)[AfCfg<M>::E], const float2* phi,
+                                            int ncol, float2* bufs, int tid, const AfTwiddles<M>& tw, Put put) {
     using A = AfCfg<M>;
     using C = ColCfg<M>;
     constexpr int E = A::E, TPF = A::TPF, NTS = A::SUB * TPF;
@@ -525,17 +527,12 @@ __device__ __forceinline__ void af_subchunk(const float2 (&s)[AfCfg<M>::E], cons
     float2 x[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) x[e] = cmul(phi[C::in(lane, e)], s[e]);
-    fft<M, E, -1, true>(x, buf, lane, tw);
+    fft<M, E, -1, true>(x, buf, lane, tw.fwd);
 #pragma unroll
     for (int e = 0; e < E; ++e) x[e] = cscale(x[e], cabs_hw(x[e]));
-    relayout_out_to_in<M, E, true>(x, buf, lane);
-    fft<M, E, +1, true>(x, buf, lane, tw);
+    fft<M, E, +1, true, true>(x, buf, lane, tw.inv);   // back to the layout of s
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int pos = C::out(lane, e);
-        const float2 sv = C::same_layout ? s[e] : (valid ? col[pos] : make_float2(0.0f, 0.0f));
-        buf[pos] = af_term<M>(sv, x[e], invM);
-    }
+    for (int e = 0; e < E; ++e) buf[C::in(lane, e)] = af_term<M>(s[e], x[e], invM);
     __syncthreads();
     for (int m = tid; m < M; m += NTS) {
         float2 t = make_float2(0.0f, 0.0f);
@@ -567,12 +564,12 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_cols(Job J
     const int u = c0 + tid / TPF, lane = tid % TPF;
     const bool valid = u < U;
     const float2* col = J.su + static_cast<size_t>(f) * W * M + static_cast<size_t>(valid ? u : 0) * M;
-    const FftTwiddles<M, E> tw = fft_twiddles<M, E>(lane);
+    const AfTwiddles<M> tw(lane);
     float2 s[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) s[e] = valid ? col[C::in(lane, e)] : make_float2(0.0f, 0.0f);
     float2* part = af_part_of<M>(J, f, it) + static_cast<size_t>(j) * M;
-    af_subchunk<M>(s, phi, col, valid, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) { part[m] = t; });
+    af_subchunk<M>(s, phi, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) { part[m] = t; });
 }
 
 // The exchange words of frame f in the resident form: per iteration parity, sub-chunk q < W/SUB
@@ -662,7 +659,7 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(J
     const int u = c0 + tid / TPF, lane = tid % TPF;
     const bool valid = u < U;
     const float2* col = J.su + static_cast<size_t>(f) * W * M + static_cast<size_t>(valid ? u : 0) * M;
-    const FftTwiddles<M, E> tw = fft_twiddles<M, E>(lane);
+    const AfTwiddles<M> tw(lane);
     float2 s[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) s[e] = valid ? col[C::in(lane, e)] : make_float2(0.0f, 0.0f);
@@ -676,7 +673,7 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(J
         uint64_t* words = af_words_of<M>(J, f, it);
         if constexpr (kTagged) {
             const unsigned tag = (epoch << 7) | static_cast<unsigned>(it);
-            af_subchunk<M>(s, phi, col, valid, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) {
+            af_subchunk<M>(s, phi, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) {
                 uint64_t* w = words + (static_cast<size_t>(j) * M + m) * 2;
                 xwg_store(w, xwg_word(t.x, tag));
                 xwg_store(w + 1, xwg_word(t.y, tag));
@@ -684,7 +681,7 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(J
             for (int m = tid; m < M; m += NTS)
                 phi[m] = af_phase_tagged<M>(words, nsub, m, tag, J.af_wait_polls, waiting, J.dec[f].status);
         } else {
-            af_subchunk<M>(s, phi, col, valid, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) {
+            af_subchunk<M>(s, phi, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) {
                 uint64_t v;
                 __builtin_memcpy(&v, &t, sizeof v);
                 xwg_store(words + static_cast<size_t>(j) * M + m, v);
@@ -732,7 +729,7 @@ template <int M>
 size_t colfft_lds() {
     using C = ColCfg<M>;
     const size_t work = std::max(static_cast<size_t>(M) * (C::CT + 1), static_cast<size_t>(C::CT) * lds_padded_size(M));
-    return M * sizeof(float2) + work * sizeof(float2);
+    return work * sizeof(float2);
 }
 template <int M>
 size_t autofocus_lds() {

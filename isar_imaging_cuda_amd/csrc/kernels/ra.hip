@@ -17,18 +17,19 @@ namespace {
 
 constexpr int kE = 16;   // elements per thread for the row transforms
 
+// Range cell (or bin) of register slot e of a thread, before and after a row transform.
 template <int N>
-__device__ __forceinline__ int in_pos(int tid, int e) { return fft_in_pos<N, kE, FftPlan<N, kE>::R[0]>(tid, e); }
-template <int N>
-__device__ __forceinline__ int out_pos(int tid, int e) {
-    return fft_out_pos<N, kE, FftPlan<N, kE>::R[FftPlan<N, kE>::NP - 1]>(tid, e);
+__device__ __forceinline__ int row_pos(int tid, int e) {
+    static_assert(FftPlan<N, kE>::R[0] == 16 && FftPlan<N, kE>::R[FftPlan<N, kE>::NP - 1] == 16, "one layout");
+    return tid + e * (N / kE);
 }
 
 // Dynamic LDS of the row kernels: the transform buffer (lds_padded_size(N) float2), 64 floats of
-// reductions, then the 256 twiddles of the stride-16 radix-16 pass (fft_tw16_table_fill).
+// reductions, then the constants of the stride-16 pass.
+constexpr int row_words(int N) { return (lds_padded_size(N) * 2 + 64 + 3) & ~3; }   // 4-byte words before the constants
 template <int N>
-__device__ __forceinline__ float2* tw16_table(float2* lds) {
-    return reinterpret_cast<float2*>(reinterpret_cast<char*>(lds + lds_padded_size(N)) + 64 * sizeof(float));
+__device__ __forceinline__ FftCT* stride16_rows(float2* lds) {
+    return reinterpret_cast<FftCT*>(reinterpret_cast<float*>(lds) + row_words(N));
 }
 
 // Spectrum of row m of frame f with HPC (FP64 phase), window and (-1)^n centring applied, in
@@ -44,81 +45,100 @@ __device__ __forceinline__ float2* tw16_table(float2* lds) {
 // no factor is more than six products from an FP64-reduced value and only the running factor,
 // the group base, d, d^4 and the lane's e^2 factor stay live beside the row. Every FP64 argument
 // is a part of vk n^2 and is reduced at least as exactly as vk n^2 itself.
+//
+// The row's samples and window values are loaded first (RowSamples::load), together, and turned into
+// the spectrum later (spectrum), every element times `scale`, a power of two.
 template <int N, bool ONE_WINDOW = false>
-__device__ __forceinline__ void load_row_raw(float2 (&x)[kE], const Job& J, int f, int m, int tid_) {
+struct RowSamples {
     static_assert(FftPlan<N, kE>::R[0] == 16, "factorised phase assumes a radix-16 first pass");
-    const int tid = opaque(tid_);
-    const long long erow = echo_first_row(J, f) + m;
-    const float2* row = J.data_type == 1 ? J.pre + (static_cast<size_t>(f) * J.M + m) * N
-                                         : J.echo + static_cast<size_t>(erow) * N;
-    const bool hpc = J.if_hpc && J.data_type == 2;
-    const bool hrrp_window = !ONE_WINDOW && J.if_hrrp && J.data_type == 2;
-    auto window = [&](int n) {
-        float w = elem_u32(J.win_range, n);
-        if (hrrp_window) w *= w;
-        return (n & 1) ? -w : w;
-    };
-    if (!hpc) {
-#pragma unroll
-        for (int e = 0; e < kE; ++e) {
-            const int n = in_pos<N>(tid, e);
-            x[e] = cscale(elem_u32(row, n), window(n));
-        }
-        return;
-    }
-    constexpr double S = N / kE;
-    const double vk = J.hpc_k * J.velocity[erow];
-    const double t = static_cast<double>(tid);
-    const double lin = 2.0 * S * vk * t;
-    const float2 d1 = expjpi_reduced(lin);
-    const float2 d4 = expjpi_reduced(4.0 * lin);
-    float2 base = expjpi_reduced(vk * t * t);
-    const double e0 = static_cast<double>(tid & 15);
-    const float2 c = expjpi_reduced((S * S) * vk * (e0 * e0));
-#pragma unroll
-    for (int q = 0; q < kE / 4; ++q) {
-        float2 h = base;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int e = 4 * q + r;
-            const int n = in_pos<N>(tid, e);
-            const float2 ce = make_float2(wave_read_lane(c.x, e), wave_read_lane(c.y, e));
-            x[e] = cscale(cmul(elem_u32(row, n), cmul(h, ce)), window(n));
-            if (r < 3) h = cmul(h, d1);
-        }
-        if (q + 1 < kE / 4) base = cmul(base, d4);
-    }
-}
+    float2 v[kE];
+    float w[kE];
+    double velocity;   // for the compensation phase (0 without)
 
-// Multiply a first-pass-layout row by the lag ramp exp(-j 2 pi n lag / N). With n = tid + e N/16
-// the ramp factors into exp(j pi b tid) * u_e, u_e = exp(j pi b e N/16), b = -2 lag / N. The u_e
-// are the same for every thread: lane e of each wave evaluates u_e and the other lanes read it.
-// Both arguments are reduced in FP64.
+    __device__ __forceinline__ void load(const Job& J, int f, int m, int tid_) {
+        const int tid = opaque(tid_);
+        const long long erow = echo_first_row(J, f) + m;
+        const float2* row = J.data_type == 1 ? J.pre + (static_cast<size_t>(f) * J.M + m) * N
+                                             : J.echo + static_cast<size_t>(erow) * N;
+        velocity = J.if_hpc && J.data_type == 2 ? J.velocity[erow] : 0.0;
+#pragma unroll
+        for (int e = 0; e < kE; ++e) v[e] = elem_u32(row + e * (N / kE), tid);
+#pragma unroll
+        for (int e = 0; e < kE; ++e) w[e] = elem_u32(J.win_range + e * (N / kE), tid);
+        issue_point();
+    }
+
+    __device__ __forceinline__ void spectrum(float2 (&x)[kE], const Job& J, int tid_, float scale) const {
+        const int tid = opaque(tid_);
+        const bool hpc = J.if_hpc && J.data_type == 2;
+        const bool hrrp_window = !ONE_WINDOW && J.if_hrrp && J.data_type == 2;
+        // N/16 is even, so the sign (-1)^n is that of the thread
+        const float sign = (tid & 1) ? -1.0f : 1.0f;
+        auto window = [&](int e) { return sign * (hrrp_window ? w[e] * w[e] : w[e]); };
+        if (!hpc) {
+#pragma unroll
+            for (int e = 0; e < kE; ++e) x[e] = cscale(v[e], scale * window(e));
+            return;
+        }
+        constexpr double S = N / kE;
+        const double vk = uniform(J.hpc_k * velocity);
+        const double t = static_cast<double>(tid);
+        const double lin = 2.0 * S * vk * t;
+        const float2 d1 = expjpi_reduced(lin);
+        const float2 d4 = expjpi_reduced(4.0 * lin);
+        float2 base = cscale(expjpi_reduced(vk * t * t), scale);
+        const double e0 = static_cast<double>(tid & 15);
+        const float2 c = expjpi_reduced((S * S) * vk * (e0 * e0));
+        issue_point();
+#pragma unroll
+        for (int q = 0; q < kE / 4; ++q) {
+            float2 h = base;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e = 4 * q + r;
+                const float2 ce = make_float2(wave_read_lane(c.x, e), wave_read_lane(c.y, e));
+                x[e] = cscale(cmul(v[e], cmul(h, ce)), window(e));
+                if (r < 3) h = cmul(h, d1);
+            }
+            if (q + 1 < kE / 4) base = cmul(base, d4);
+        }
+    }
+};
+
+// Stored spectrum S0 of row m times its lag ramp exp(-j 2 pi n lag / N), lag = before + by, after the first pass of
+// its inverse transform. With n = tid + e N/16 the ramp factors into exp(j pi b tid) * u^e,
+// u = exp(j pi b N / 16) = exp(-j pi lag / 8), b = -2 lag / N. The powers of u are taken by the
+// pass itself, as its twiddle: the eight constants (fft_table::Pow2) are the same for every
+// thread, so lane l < 8 of each wave forms the l-th and the others read it. exp(j pi b tid) is one
+// product per element. Arguments are reduced in FP64.
 template <int N>
-__device__ __forceinline__ void apply_ramp(float2 (&x)[kE], double lag, int tid) {
+__device__ __forceinline__ void load_row_shifted(float2 (&x)[kE], const Job& J, int f, int m, double before, double by,
+                                                 int tid_) {
     static_assert(FftPlan<N, kE>::R[0] == 16, "factorised ramp assumes a radix-16 first pass");
-    if (lag == 0.0) return;
-    const double b = -2.0 * lag / N;
-    const float2 w0 = expjpi_reduced(b * tid);
-    const float2 u = expjpi_reduced(b * static_cast<double>((N / 16) * (tid & 15)));
-#pragma unroll
-    for (int e = 0; e < kE; ++e) {
-        const float2 ue = make_float2(wave_read_lane(u.x, e), wave_read_lane(u.y, e));
-        x[e] = cmul(cmul(x[e], ue), w0);
-    }
-}
-
-// Stored spectrum S0 of row m times its lag ramp.
-template <int N>
-__device__ __forceinline__ void load_row_shifted(float2 (&x)[kE], const Job& J, int f, int m, double lag, int tid_) {
     const int tid = opaque(tid_);
     const float2* row = J.pre + (static_cast<size_t>(f) * J.M + m) * N;
 #pragma unroll
-    for (int e = 0; e < kE; ++e) x[e] = elem_u32(row, static_cast<unsigned>(in_pos<N>(tid, e)));
-    apply_ramp<N>(x, lag, tid);
+    for (int e = 0; e < kE; ++e) x[e] = elem_u32(row + e * (N / kE), tid);
+    issue_point();
+    const double lag = uniform(before + by);
+    const float2 w0 = expjpi_reduced(-2.0 * lag / N * tid);
+    const int l = tid & 7;
+    const double turns = (l == 0 ? 8.0 : l == 1 ? 4.0 : l < 4 ? 2.0 : 1.0) * (-0.125 * lag) +
+                         (l == 3 ? 0.25 : l < 4 ? 0.0 : 0.125 * (l - 4));
+    const float2 cs = expjpi_reduced(turns);
+    const float c = fabsf(cs.x) < 0x1p-30f ? 0x1p-30f : cs.x;
+    const float r = rcp_hw(c);
+    float t = cs.y * r;
+    t = fmaf(fmaf(-t, c, cs.y), r, t);   // cs.y / c to an ulp
+    FftCTs<8> ramp;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ramp.v[i] = FftCT{wave_read_lane(c, i), wave_read_lane(t, i)};
+#pragma unroll
+    for (int e = 0; e < kE; ++e) x[e] = cmul(x[e], w0);
+    dft16_twiddled<+1>(x, ramp);
 }
 
-// Energy profile of group g at merge stride s >= 2, in the first-pass layout. Level 1 (s = 2)
+// Energy profile of group g at merge stride s >= 2. Level 1 (s = 2)
 // energies are complete (written by the fused level-0 pass); from level 2 on, the shifted second
 // subgroup of the previous level is added from its row-chunk partial sums.
 template <int N>
@@ -126,7 +146,7 @@ __device__ __forceinline__ void group_energy(float (&a)[kE], const Job& J, int f
     const int M = J.M;
     const float* base = J.egrp + (static_cast<size_t>(f) * M + static_cast<size_t>(g) * s) * N;
 #pragma unroll
-    for (int e = 0; e < kE; ++e) a[e] = elem_u32(base, in_pos<N>(tid, e));
+    for (int e = 0; e < kE; ++e) a[e] = elem_u32(base, row_pos<N>(tid, e));
     if (s > 2) {
         const int s2 = s / 2;
         const int r0 = (2 * g + 1) * s2;
@@ -136,41 +156,50 @@ __device__ __forceinline__ void group_energy(float (&a)[kE], const Job& J, int f
             for (int h = r0; h < r1; h += R) {
                 const float* pp = J.epart + (static_cast<size_t>(f) * M + h) * N;
 #pragma unroll
-                for (int e = 0; e < kE; ++e) a[e] += elem_u32(pp, in_pos<N>(tid, e));
+                for (int e = 0; e < kE; ++e) a[e] += elem_u32(pp, row_pos<N>(tid, e));
             }
         }
     }
 }
 
-// Correlation of two non-negative profiles given as energies (first-pass layout): the argmax of
+// Correlation of two non-negative profiles given as energies: the argmax of
 // |c| after ifftshift, lowest index on ties (range_alignment.cu:45-61, 108-168). The real
-// correlation comes from one complex FFT of gA + j gB. Every thread gets the argmax.
+// correlation comes from one complex FFT of gA + j gB, whose spectrum lands in the layout that the
+// inverse transform takes, so only the mirrored bins N - k go through LDS. Every thread gets the
+// argmax.
 template <int N>
 __device__ int correlation_argmax(const float (&a)[kE], const float (&b)[kE], float2* lds, float* redv, int* redi,
-                                  int tid, const FftTwiddles<N, kE>& tw, const float2* tab) {
+                                  int tid, const FftTwiddlesLds<N, kE>& tw) {
     constexpr int NT = N / kE;
     float2 x[kE];
 #pragma unroll
     for (int e = 0; e < kE; ++e) x[e] = make_float2(sqrt_hw(a[e]), sqrt_hw(b[e]));
-    fft<N, kE, -1>(x, lds, tid, tw, tab);
+    fft<N, kE, -1>(x, lds, tid, tw);
+    // bin k = tid + e T; its mirror N - k = (T - tid) + (15 - e) T, which is 0 (not N) for k = 0
+    constexpr int T = N / kE;
+    static_assert(FftPlan<N, kE>::R[0] == 16 && T % lds_pad_every(N) == 0, "bins of a thread T apart");
+    {
+        float2* at = lds + lds_pad<N>(tid);
 #pragma unroll
-    for (int e = 0; e < kE; ++e) lds[lds_pad(out_pos<N>(tid, e))] = x[e];
+        for (int e = 0; e < kE; ++e) at[lds_pad<N>(e * T)] = x[e];
+    }
     __syncthreads();
+    const float2* mirror = lds + lds_pad<N>(T - tid);
+    const float2* mirror0 = tid == 0 ? lds : mirror + lds_pad<N>(15 * T);
 #pragma unroll
     for (int e = 0; e < kE; ++e) {
-        const int k = in_pos<N>(tid, e);
-        const float2 zk = lds[lds_pad(k)], zn = lds[lds_pad((N - k) & (N - 1))];
+        const float2 zk = x[e], zn = e == 0 ? *mirror0 : mirror[lds_pad<N>((15 - e) * T)];
         const float2 ga = make_float2(0.5f * (zk.x + zn.x), 0.5f * (zk.y - zn.y));
         const float2 gb = make_float2(0.5f * (zk.y + zn.y), -0.5f * (zk.x - zn.x));
         x[e] = cmulc(ga, gb);
     }
     __syncthreads();
-    fft<N, kE, +1>(x, lds, tid, tw, tab);
+    fft<N, kE, +1>(x, lds, tid, tw);
     float best = -1.0f;
     int bi = 0;
 #pragma unroll
     for (int e = 0; e < kE; ++e) {
-        const int i = (out_pos<N>(tid, e) + N / 2) & (N - 1);
+        const int i = (row_pos<N>(tid, e) + N / 2) & (N - 1);
         const float v = fabsf(x[e].x);
         if (v > best || (v == best && i < bi)) { best = v; bi = i; }
     }
@@ -194,11 +223,9 @@ __device__ __forceinline__ double sqrt_refined(float x) {
 // not read from the FP32 transform: near a broad peak the second
 // difference f1 + f3 - 2 f2 cancels most of its digits, and the transform's rounding alone moved
 // the vertex by up to 2.4e-4 cell at 1024 x 16384, which 120 autofocus iterations amplify into a
-// 1e-3 image difference. The vertex and the lag are FP64. a, b: the two energy profiles, element
-// e of thread tid at range cell pos(tid, e), where pos is the first-pass layout (OUT = false) or
-// the last-pass layout (OUT = true). Must follow correlation_argmax (its barriers end the LDS
-// use). Thread 0 records the lag and argmax; every thread gets the lag.
-template <int N, bool OUT = false>
+// 1e-3 image difference. The vertex and the lag are FP64. a, b: the two energy profiles. Must follow correlation_argmax (its barriers end the LDS use). Thread 0 records
+// the lag and argmax; every thread gets the lag.
+template <int N>
 __device__ double parabola_lag(const float (&a)[kE], const float (&b)[kE], int bi, float2* lds, int tid,
                                double* lag_out, int32_t* imax_out) {
     constexpr int NT = N / kE;
@@ -213,7 +240,7 @@ __device__ double parabola_lag(const float (&a)[kE], const float (&b)[kE], int b
     // across its transforms.
     double* gb = reinterpret_cast<double*>(lds);
     double* red = gb + N;
-    auto pos = [&](int e) { return OUT ? out_pos<N>(tid, e) : in_pos<N>(tid, e); };
+    auto pos = [&](int e) { return row_pos<N>(tid, e); };
 #pragma unroll
     for (int e = 0; e < kE; ++e) gb[pos(e)] = sqrt_refined(opaque(b[e]));
     __syncthreads();
@@ -257,7 +284,7 @@ __device__ double parabola_lag(const float (&a)[kE], const float (&b)[kE], int b
         red[0] = lag;
     }
     __syncthreads();
-    const double lag = red[0];
+    const double lag = uniform(red[0]);
     __syncthreads();
     return lag;
 }
@@ -273,17 +300,17 @@ __global__ __launch_bounds__(N / kE) void k_ifds_pre(Job J) {
     const float2* src = J.echo + static_cast<size_t>(echo_first_row(J, f) + m) * N;
     float2 x[kE];
 #pragma unroll
-    for (int e = 0; e < kE; ++e) x[e] = src[(in_pos<N>(tid, e) + N / 2) & (N - 1)];
+    for (int e = 0; e < kE; ++e) x[e] = src[(row_pos<N>(tid, e) + N / 2) & (N - 1)];
     // getHRRP for IFDS (common.cu:546-558) undoes this stage, ifftshift(FFT(ifftshift(pre))) =
     // the input row, so the profile is the row itself
     if (J.hrrp) {
 #pragma unroll
-        for (int e = 0; e < kE; ++e) J.hrrp[off + ((in_pos<N>(tid, e) + N / 2) & (N - 1))] = x[e];
+        for (int e = 0; e < kE; ++e) J.hrrp[off + ((row_pos<N>(tid, e) + N / 2) & (N - 1))] = x[e];
     }
     fft<N, kE, +1>(x, lds, tid);
     const float inv = 1.0f / N;
 #pragma unroll
-    for (int e = 0; e < kE; ++e) J.pre[off + ((out_pos<N>(tid, e) + N / 2) & (N - 1))] = cscale(x[e], inv);
+    for (int e = 0; e < kE; ++e) J.pre[off + ((row_pos<N>(tid, e) + N / 2) & (N - 1))] = cscale(x[e], inv);
 }
 
 // getHRRP for STRETCH (common.cu:561-571): ifftshift(FFT(hamming_N * row)) of the compensated
@@ -293,18 +320,21 @@ __global__ __launch_bounds__(N / kE) void k_hrrp(Job J) {
     HIP_DYNAMIC_SHARED(float2, lds);
     const int m = blockIdx.x, f = blockIdx.y, tid = threadIdx.x;
     float2 x[kE];
-    load_row_raw<N, true>(x, J, f, m, tid);
+    RowSamples<N, true> row;
+    row.load(J, f, m, tid);
+    row.spectrum(x, J, tid, 1.0f);
     fft<N, kE, -1>(x, lds, tid);
     float2* dst = J.hrrp + (static_cast<size_t>(f) * J.M + m) * N;
 #pragma unroll
-    for (int e = 0; e < kE; ++e) dst[out_pos<N>(tid, e)] = x[e];
+    for (int e = 0; e < kE; ++e) dst[row_pos<N>(tid, e)] = x[e];
 }
 
 // Merge level 0 fused with the spectrum preparation (range_alignment.cu:13-18 and :34-73 at
 // stride 1), one workgroup per row pair (2p, 2p+1): S0 of both rows (stored for the later
 // levels), both energy profiles, their correlation and lag, the shift of row 2p+1 and the
 // merged level-1 energy. Rows 0 and 1 never move again: their aligned profiles and column sums
-// are written here.
+// are written here. The spectra carry the inverse transforms' 1 / N (a power of two), so no
+// profile or energy is scaled later.
 template <int N>
 __global__ __launch_bounds__(N / kE, 4) void k_ra_pair0(Job J) {
     HIP_DYNAMIC_SHARED(float2, lds);
@@ -314,96 +344,62 @@ __global__ __launch_bounds__(N / kE, 4) void k_ra_pair0(Job J) {
     const int p = blockIdx.x, f = blockIdx.y, tid = threadIdx.x;
     const int M = J.M;
     const int ra = 2 * p, rb = 2 * p + 1;
-    const float inv2 = 1.0f / (static_cast<float>(N) * static_cast<float>(N));
-    const float invN = 1.0f / N;
+    constexpr float invN = 1.0f / N;
     const bool final_rows = (p == 0);
     float2* s0a = J.pre + (static_cast<size_t>(f) * M + ra) * N;
     float2* s0b = J.pre + (static_cast<size_t>(f) * M + rb) * N;
     float* dst = J.egrp + (static_cast<size_t>(f) * M + ra) * N;
     float* ap = J.arp_part + static_cast<size_t>(f) * (M / 2) * N;
-    const FftTwiddles<N, kE> tw = fft_twiddles<N, kE>(tid);
-    float2* const tab = tw16_table<N>(lds);
-    fft_tw16_table_fill(tab, tid, NT);
+    RowSamples<N> row;
+    row.load(J, f, ra, tid);
+    const auto tw = fft_twiddles_lds<N, kE>(tid, stride16_rows<N>(lds));
     float2 x[kE];
-    float ea[kE];
+    float ea[kE], eb[kE];
     float mx = 0.0f;
     // Every global location below is re-read only by the thread that wrote it, and the stores
     // into the S0 rows (which st aliases) are ordered by the barriers inside each transform.
-    // row 2p: S0, profile, energy (written now as the first term of the merged energy)
-    load_row_raw<N>(x, J, f, ra, tid);
+    // row 2p: S0, profile, energy (kept in registers as the first term of the merged energy)
+    row.spectrum(x, J, tid, invN);
     {
         const int t = opaque(tid);
 #pragma unroll
-        for (int e = 0; e < kE; ++e) elem_u32(s0a, in_pos<N>(t, e)) = x[e];
+        for (int e = 0; e < kE; ++e) elem_u32(s0a + e * (N / kE), t) = x[e];
     }
-    fft<N, kE, +1>(x, lds, tid, tw, tab);
-    {
-        const int t = opaque(tid);
-#pragma unroll
-        for (int e = 0; e < kE; ++e) {
-            ea[e] = cabs2(x[e]) * inv2;
-            elem_u32(dst, out_pos<N>(t, e)) = ea[e];
-        }
-    }
+    fft<N, kE, +1>(x, lds, tid, tw);
     if (final_rows) {   // row 0 is the reference of the merge tree and never moves
         const int t = opaque(tid);
 #pragma unroll
         for (int e = 0; e < kE; ++e) {
-            const float2 v = cscale(x[e], invN);
-            const int pos = out_pos<N>(t, e);
-            elem_u32(s0a, pos) = v;
-            const float av = cabs_hw(v);
+            const int pos = row_pos<N>(t, e);
+            elem_u32(s0a, pos) = x[e];
+            const float av = cabs_hw(x[e]);
             elem_u32(ap, pos) = av;
             mx = fmaxf(mx, av);
         }
     }
+#pragma unroll
+    for (int e = 0; e < kE; ++e) ea[e] = cabs2(x[e]);
     // row 2p+1: S0 and energy
-    load_row_raw<N>(x, J, f, rb, tid);
+    row.load(J, f, rb, tid);
+    row.spectrum(x, J, tid, invN);
     {
         const int t = opaque(tid);
 #pragma unroll
-        for (int e = 0; e < kE; ++e) elem_u32(s0b, in_pos<N>(t, e)) = x[e];
+        for (int e = 0; e < kE; ++e) elem_u32(s0b + e * (N / kE), t) = x[e];
     }
-    fft<N, kE, +1>(x, lds, tid, tw, tab);
-    // Above 4096 cells the two energy rows do not stay in registers across the correlation's
-    // transforms: row 2p's is in its merged-energy row already, and row 2p+1's goes to that
-    // row's energy slot, which no group at stride >= 2 uses (group heads are even rows). Each
-    // thread reads back only what it wrote.
-    constexpr bool kStash = N > 4096;
-    float* eb_row = J.egrp + (static_cast<size_t>(f) * M + rb) * N;
-    if constexpr (kStash) {
-        const int t = opaque(tid);
+    fft<N, kE, +1>(x, lds, tid, tw);
 #pragma unroll
-        for (int e = 0; e < kE; ++e) elem_u32(eb_row, out_pos<N>(t, e)) = cabs2(x[e]) * inv2;
-    }
-    // the correlation takes the energies in the first-pass layout
-#pragma unroll
-    for (int e = 0; e < kE; ++e) x[e] = make_float2(ea[e], cabs2(x[e]) * inv2);
-    relayout_out_to_in<N, kE>(x, lds, tid);
-    float ta[kE], tb[kE];
-#pragma unroll
-    for (int e = 0; e < kE; ++e) { ta[e] = x[e].x; tb[e] = x[e].y; }
+    for (int e = 0; e < kE; ++e) eb[e] = cabs2(x[e]);
     const size_t idx = static_cast<size_t>(f) * (M - 1) + p;
-    const int bi = correlation_argmax<N>(ta, tb, lds, redv, redi, tid, tw, tab);
-    double lag;
-    if constexpr (kStash) {
-        const int t = opaque(tid);
-#pragma unroll
-        for (int e = 0; e < kE; ++e) {
-            ta[e] = elem_u32(dst, out_pos<N>(t, e));
-            tb[e] = elem_u32(eb_row, out_pos<N>(t, e));
-        }
-        lag = parabola_lag<N, true>(ta, tb, bi, lds, tid, J.lags + idx, J.imax + idx);
-    } else {
-        lag = parabola_lag<N>(ta, tb, bi, lds, tid, J.lags + idx, J.imax + idx);
-    }
+    const int bi = correlation_argmax<N>(ea, eb, lds, redv, redi, tid, tw);
+    const double lag = parabola_lag<N>(ea, eb, bi, lds, tid, J.lags + idx, J.imax + idx);
     // shift row 2p+1 by the lag and merge (range_alignment.cu:66-69)
-    load_row_shifted<N>(x, J, f, rb, lag, tid);
-    fft<N, kE, +1>(x, lds, tid, tw, tab);
+    load_row_shifted<N>(x, J, f, rb, 0.0, lag, tid);
+    fft_after_first<N, kE, +1>(x, lds, tid, tw);
     {
         const int t = opaque(tid);
 #pragma unroll
-        for (int e = 0; e < kE; ++e) elem_u32(dst, out_pos<N>(t, e)) += cabs2(x[e]) * inv2;
+        for (int e = 0; e < kE; ++e) elem_u32(dst + e * (N / kE), t) = ea[e] + cabs2(x[e]);
     }
     if (tid == 0) {
         J.lagsum[static_cast<size_t>(f) * M + ra] = 0.0;
@@ -413,10 +409,9 @@ __global__ __launch_bounds__(N / kE, 4) void k_ra_pair0(Job J) {
         const int t = opaque(tid);
 #pragma unroll
         for (int e = 0; e < kE; ++e) {
-            const float2 v = cscale(x[e], invN);
-            const int pos = out_pos<N>(t, e);
-            elem_u32(s0b, pos) = v;
-            const float av = cabs_hw(v);
+            const int pos = row_pos<N>(t, e);
+            elem_u32(s0b, pos) = x[e];
+            const float av = cabs_hw(x[e]);
             elem_u32(ap, pos) += av;
             mx = fmaxf(mx, av);
         }
@@ -428,7 +423,7 @@ __global__ __launch_bounds__(N / kE, 4) void k_ra_pair0(Job J) {
 // One merge level s >= 2: group energies of pair p and their correlation (range_alignment.cu:
 // 45-61). The first group's energy is kept for the next level.
 template <int N>
-__global__ __launch_bounds__(N / kE) void k_ra_corr(Job J, int s, int pair_base) {
+__global__ __launch_bounds__(N / kE, 4) void k_ra_corr(Job J, int s, int pair_base) {
     HIP_DYNAMIC_SHARED(float2, lds);
     float* redv = reinterpret_cast<float*>(lds + lds_padded_size(N));
     int* redi = reinterpret_cast<int*>(redv + 16);
@@ -437,29 +432,18 @@ __global__ __launch_bounds__(N / kE) void k_ra_corr(Job J, int s, int pair_base)
     const int ngroups = (M + s - 1) / s, npairs = ngroups / 2;
     const bool unpaired = (p == npairs);
     const int gA = unpaired ? ngroups - 1 : 2 * p;
+    const auto tw = fft_twiddles_lds<N, kE>(tid, stride16_rows<N>(lds));
     float a[kE], b[kE];
     group_energy<N>(a, J, f, gA, s, tid);
-    const FftTwiddles<N, kE> tw = fft_twiddles<N, kE>(tid);
-    float2* const tab = tw16_table<N>(lds);
-    fft_tw16_table_fill(tab, tid, N / kE);
     {   // keep the first group's energy for the next level (same head row, same thread)
         float* dst = J.egrp + (static_cast<size_t>(f) * M + static_cast<size_t>(gA) * s) * N;
 #pragma unroll
-        for (int e = 0; e < kE; ++e) elem_u32(dst, in_pos<N>(tid, e)) = a[e];
+        for (int e = 0; e < kE; ++e) elem_u32(dst, row_pos<N>(tid, e)) = a[e];
     }
     if (unpaired) return;
     group_energy<N>(b, J, f, gA + 1, s, tid);
     const size_t idx = static_cast<size_t>(f) * (M - 1) + pair_base + p;
-    const int bi = correlation_argmax<N>(a, b, lds, redv, redi, tid, tw, tab);
-    // read both energies again rather than hold them across the transforms (the first from the
-    // row this thread just wrote)
-    {
-        const float* src = J.egrp + (static_cast<size_t>(f) * M + static_cast<size_t>(gA) * s) * N;
-        const int t = opaque(tid);
-#pragma unroll
-        for (int e = 0; e < kE; ++e) a[e] = elem_u32(src, in_pos<N>(t, e));
-    }
-    group_energy<N>(b, J, f, gA + 1, s, opaque(tid));
+    const int bi = correlation_argmax<N>(a, b, lds, redv, redi, tid, tw);
     (void)parabola_lag<N>(a, b, bi, lds, tid, J.lags + idx, J.imax + idx);
 }
 
@@ -485,18 +469,14 @@ __global__ __launch_bounds__(N / kE, PART == kUpdFinal && N <= 4096 ? 3 : 4) voi
     const int r0 = (2 * p + 1) * s + i * R;
     const int r1 = min(r0 + R, gend);
     if (r0 >= r1) return;
-    const double lag = J.lags[static_cast<size_t>(f) * (M - 1) + pair_base + p];
-    const float inv = 1.0f / (static_cast<float>(N) * static_cast<float>(N));
-    const float invN = 1.0f / N;
+    const double lag = uniform(J.lags[static_cast<size_t>(f) * (M - 1) + pair_base + p]);
     const bool final_rows = PART == kUpdFinal || (PART == kUpdAll && p == 0);
     float acc[kE];
     float mx = 0.0f;
 #pragma unroll
     for (int e = 0; e < kE; ++e) acc[e] = 0.0f;
     float2 x[kE];
-    const FftTwiddles<N, kE> tw = fft_twiddles<N, kE>(tid);
-    float2* const tab = tw16_table<N>(lds);
-    fft_tw16_table_fill(tab, tid, N / kE);
+    const auto tw = fft_twiddles_lds<N, kE>(tid, stride16_rows<N>(lds));
     // column sums of |profile| over the final rows of this chunk: kept in registers by the
     // final-row grid up to 4096 cells (above, its workgroup size leaves no room) and stored once,
     // otherwise accumulated in place (each location is read back only by the thread that wrote
@@ -506,21 +486,20 @@ __global__ __launch_bounds__(N / kE, PART == kUpdFinal && N <= 4096 ? 3 : 4) voi
     float arp[kArpInRegs ? kE : 1];
 #pragma unroll
     for (int e = 0; e < (kArpInRegs ? kE : 1); ++e) arp[e] = 0.0f;
+#pragma unroll 1
     for (int m = r0; m < r1; ++m) {
-        const double L = J.lagsum[static_cast<size_t>(f) * M + m] + lag;
-        load_row_shifted<N>(x, J, f, m, L, tid);
-        fft<N, kE, +1>(x, lds, tid, tw, tab);
+        load_row_shifted<N>(x, J, f, m, J.lagsum[static_cast<size_t>(f) * M + m], lag, tid);
+        fft_after_first<N, kE, +1>(x, lds, tid, tw);
 #pragma unroll
-        for (int e = 0; e < kE; ++e) acc[e] += cabs2(x[e]) * inv;
+        for (int e = 0; e < kE; ++e) acc[e] += cabs2(x[e]);
         if (final_rows) {   // S0 of row m was read before the transform's first barrier
             float2* st = J.st + (static_cast<size_t>(f) * M + m) * N;
             const int t = opaque(tid);
 #pragma unroll
             for (int e = 0; e < kE; ++e) {
-                const float2 v = cscale(x[e], invN);
-                const int pos = out_pos<N>(t, e);
-                elem_u32(st, pos) = v;
-                const float av = cabs_hw(v);
+                const int pos = row_pos<N>(t, e);
+                elem_u32(st, pos) = x[e];
+                const float av = cabs_hw(x[e]);
                 if constexpr (kArpInRegs) arp[e] += av;
                 else elem_u32(ap, pos) = (m == r0 ? 0.0f : elem_u32(ap, pos)) + av;
                 mx = fmaxf(mx, av);
@@ -531,7 +510,7 @@ __global__ __launch_bounds__(N / kE, PART == kUpdFinal && N <= 4096 ? 3 : 4) voi
         if constexpr (kArpInRegs) {
             const int t = opaque(tid);
 #pragma unroll
-            for (int e = 0; e < kE; ++e) elem_u32(ap, out_pos<N>(t, e)) = arp[e];
+            for (int e = 0; e < kE; ++e) elem_u32(ap, row_pos<N>(t, e)) = arp[e];
         }
         float* red = reinterpret_cast<float*>(lds + lds_padded_size(N));
         mx = block_max<N / kE>(mx, red);
@@ -541,7 +520,7 @@ __global__ __launch_bounds__(N / kE, PART == kUpdFinal && N <= 4096 ? 3 : 4) voi
     if (tid < r1 - r0) J.lagsum[static_cast<size_t>(f) * M + r0 + tid] += lag;
     float* dst = J.epart + (static_cast<size_t>(f) * M + r0) * N;
 #pragma unroll
-    for (int e = 0; e < kE; ++e) elem_u32(dst, out_pos<N>(tid, e)) = acc[e];
+    for (int e = 0; e < kE; ++e) elem_u32(dst, row_pos<N>(tid, e)) = acc[e];
 }
 
 // Range Hamming window 0.54 - 0.46 cos(2 pi n / (N - 1)) (genHammingVec, common.cu:260-266),
@@ -556,7 +535,7 @@ __global__ __launch_bounds__(256) void k_range_window(int N, float* win) {
 // ------------------------------------------------------------------------------------------
 namespace {
 template <int N>
-size_t ra_lds() { return lds_padded_size(N) * sizeof(float2) + 64 * sizeof(float) + 256 * sizeof(float2); }
+size_t ra_lds() { return row_words(N) * sizeof(float) + kFft16Bytes; }
 
 #define ISAR_RANGE_SWITCH(N, BODY)                     \
     switch (N) {                                       \
