@@ -190,8 +190,10 @@ ISAR_API int isar_session_dump(unsigned mask, const char* dir);
  * iterations in one launch: each workgroup keeps its bins in registers and the frame's
  * workgroups exchange their sums through memory after every iteration. Its waits are bounded;
  * a frame whose workgroups could not all be resident together gets status bit 2
- * (isar_get_trace) and no valid phase. AUTO (default) uses SPLIT for batches of at most 32
- * frames and FUSED above. All forms give the same phases bit for bit. */
+ * (isar_get_trace) and no valid phase. AUTO (default) uses RESIDENT for batches of at most 128
+ * frames, where a frame whose wait hits its bound is done over by one workgroup and reports
+ * nothing, and FUSED above; the groups of a sub-aperture plan, which run at the same time, SPLIT up
+ * to 32 windows and FUSED above. All forms give the same phases bit for bit. */
 enum isar_autofocus_mode {
     ISAR_AF_AUTO = 0,
     ISAR_AF_FUSED = 1,
@@ -201,7 +203,8 @@ enum isar_autofocus_mode {
 };
 ISAR_API int isar_set_autofocus_mode(isar_context* ctx, int mode);
 ISAR_API int isar_get_autofocus_mode(isar_context* ctx);
-/* Bound of each wait of the resident autofocus, in polls of about a microsecond (default 2^20);
+/* Bound of each wait of the resident autofocus, in polls of about a microsecond (default 2^20; in
+ * AUTO at most 2^16);
  * a negative bound makes every wait give up at once, which forces status bit 2 (for tests of the
  * fallback). */
 ISAR_API int isar_set_af_wait_polls(isar_context* ctx, int polls);

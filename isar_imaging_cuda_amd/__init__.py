@@ -260,7 +260,7 @@ class Imager:
         _check(L.isar_stage_dump(self._h, int(frame), mask, str(directory).encode()), "isar_stage_dump")
 
     def set_autofocus_mode(self, mode: int) -> None:
-        """AF_AUTO (split batches of at most 32 frames), AF_FUSED (one workgroup per frame),
+        """AF_AUTO (resident for at most 128 frames, fused above), AF_FUSED (one workgroup per frame),
         AF_SPLIT (several workgroups per frame, one launch per iteration), AF_SPLIT_PHASE (the
         same with a phase launch per iteration) or AF_RESIDENT (several workgroups per frame, all
         iterations in one launch); the phases are the same bit for bit."""

@@ -118,7 +118,7 @@ size_t carve_workspace(const isar_radar_params& p, int K_, char* base, Job* J, S
     j.colsum = static_cast<float2*>(frame(W * sizeof(float2)));
     j.delta = static_cast<float2*>(frame(W * sizeof(float2)));
     j.af_part = static_cast<float2*>(frame(4 * (W / 8) * M * sizeof(float2)));   // split: half; resident: all
-    j.af_sync = static_cast<unsigned*>(frame(2 * sizeof(unsigned)));
+    j.af_sync = static_cast<unsigned*>(frame(sizeof(unsigned)));
     SharedTables t{};
     t.czt_table = static_cast<float2*>(shared(W * F * sizeof(float2)));
     t.czt_pre = static_cast<float2*>(shared(W * M * sizeof(float2)));
@@ -391,12 +391,12 @@ int Context::enqueue(int frames, const void* echo, const double* velocity, const
         probed(ISAR_STAGE_PA_COLFFT, s, [&] { launch_pa_colfft(J, s); });
         probed(ISAR_STAGE_PA_SELECT, s, [&] { launch_pa_select(J, s); });
     }
-    // the resident form's exchange tags hold the iteration in 7 bits; above that it runs split
-    const bool af_resident = af_mode == ISAR_AF_RESIDENT && J.iterations <= 128;
-    const bool af_split = af_mode == ISAR_AF_SPLIT || af_mode == ISAR_AF_SPLIT_PHASE || af_mode == ISAR_AF_RESIDENT ||
-                          (af_mode == ISAR_AF_AUTO && frames <= kAfSplitFrames);
+    const bool af_auto = af_mode == ISAR_AF_AUTO;
+    const bool af_guarded = af_auto && af_auto_resident && frames <= kAfResidentFrames;
+    const bool af_split = af_mode == ISAR_AF_SPLIT || af_mode == ISAR_AF_SPLIT_PHASE || (af_auto && frames <= kAfSplitFrames);
+    if (af_guarded) J.af_wait_polls = std::min(J.af_wait_polls, kAfGuardedPolls);
     probed(ISAR_STAGE_AUTOFOCUS, s, [&] {
-        if (af_resident) launch_autofocus_resident(J, s);
+        if (af_guarded || af_mode == ISAR_AF_RESIDENT) launch_autofocus_resident(J, af_guarded, s);
         else if (af_split) launch_autofocus_split(J, af_mode != ISAR_AF_SPLIT_PHASE, s);
         else launch_autofocus(J, s);
     });

@@ -94,7 +94,8 @@ struct Context {
     int last_mode = -1;
     float2* stage_scratch = nullptr;
     float2* hrrp_out = nullptr;           // max_frames x M x N profiles written by if_hrrp runs, or null
-    int af_mode = ISAR_AF_AUTO;           // autofocus form: auto, one workgroup per frame, split
+    int af_mode = ISAR_AF_AUTO;           // autofocus form: auto, one workgroup per frame, split, resident
+    bool af_auto_resident = true;         // the resident form is among those auto chooses from
     float tuned_ms = 0.0f;                // time of one run in the configuration the autotuner kept
     float mode_ms[5] = {0, 0, 0, 0, 0};   // time of one run per autofocus form (index: isar_autofocus_mode)
     int ra_chunk = kRaChunkRowsDefault;   // tunable: rows per workgroup in the alignment update

@@ -153,6 +153,7 @@ ISAR_API int isar_sa_plan_create(const isar_radar_params* p, int dwell_pulses, i
         g->cost = static_cast<double>(M) * (static_cast<double>(wins.size()) + 16.0);
         isar_radar_params gp = *p;
         gp.echo_num = M;
+        g->ctx.af_auto_resident = false;   // groups run at the same time
         int rc = g->ctx.init(gp, static_cast<int>(wins.size()));
         if (rc) {
             delete plan;

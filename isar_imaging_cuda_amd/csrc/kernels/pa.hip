@@ -252,10 +252,8 @@ __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
     const int* sel = J.sel + static_cast<size_t>(f) * W;
     float2* su = J.su + static_cast<size_t>(f) * W * M;
     const float2* X = J.x + static_cast<size_t>(f) * M * W;
-    if (tid == 0) {   // the resident form's exchange epoch (the frame's run count) and hand-off counter
-        J.af_sync[2 * f] += 1;
-        J.af_sync[2 * f + 1] = 0;
-    }
+    if (J.af_redo && (J.dec[f].status & 2) == 0) return;   // the whole workgroup
+    if (PRE && tid == 0) J.af_sync[f] = 0;   // the resident form's hand-off counter
 
     // gather the selected bins, column-major (selectRangeBins, :335-346), scaled by 2^-e so that
     // the largest selected |S| lies in [1, 2): the update takes the unit phasor of sums cubic in
@@ -396,6 +394,7 @@ __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
         __syncthreads();
     }
     for (int m = tid; m < M; m += NT) J.phi[static_cast<size_t>(f) * M + m] = phi[m];
+    if (J.af_redo && tid == 0) J.dec[f].status &= ~2;
 }
 
 // Start of the split and resident forms with the frame's work spread over many workgroups (a
@@ -404,11 +403,26 @@ __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
 // workgroups per frame each taking a contiguous share of the (pulse, bin) elements; then
 // k_af_bin_doppler forms each pulse's Doppler product of the selected bins (:282) with the
 // products added in bin order as k_autofocus adds them, into rowdop, which is free once the bins
-// are selected; k_autofocus<M, true> then forms the start phase from it.
+// are selected; k_autofocus<M, true> then forms the start phase from it. For the resident form
+// k_af_gather also clears the frame's exchange words.
 constexpr int kAfGatherGroups = 32;
 
+// The resident form's exchange: up to 512 pulses in tagged words, above through a counter.
 template <int M>
-__global__ __launch_bounds__(256) void k_af_gather(Job J) {
+constexpr bool kAfTagged = M <= 512;
+
+// The exchange words of frame f in the resident form: per iteration parity, sub-chunk q < W/SUB
+// and pulse m, the real and the imaginary part of the sub-chunk's per-pulse sum as tagged words
+// (xwg_word). Frame f owns 4 (W/8) M words of af_part, the buffer being sized for it.
+template <int M>
+__device__ __forceinline__ uint64_t* af_words_of(const Job& J, int f, int it) {
+    const size_t nq = static_cast<size_t>(J.W / AfCfg<M>::SUB);
+    uint64_t* frame = reinterpret_cast<uint64_t*>(J.af_part) + static_cast<size_t>(f) * 4 * (J.W / 8) * M;
+    return frame + static_cast<size_t>(it & 1) * nq * M * 2;
+}
+
+template <int M>
+__global__ __launch_bounds__(256) void k_af_gather(Job J, int resident) {
     HIP_DYNAMIC_SHARED(int, lsel);                                 // W
     float* red = reinterpret_cast<float*>(lsel + J.W);             // 32
     const int f = blockIdx.y, tid = threadIdx.x;
@@ -421,6 +435,13 @@ __global__ __launch_bounds__(256) void k_af_gather(Job J) {
     const int e = af_scale_exponent(cm);
     for (int u = tid; u < U; u += 256) lsel[u] = sel[u];
     __syncthreads();
+    if (kAfTagged<M> && resident) {   // the words of the ceil(U / SUB) sub-chunks of both parities
+        const int words = (U + AfCfg<M>::SUB - 1) / AfCfg<M>::SUB * M * 2;
+        for (int i = blockIdx.x * 256 + tid; i < words; i += gridDim.x * 256) {
+            xwg_store(af_words_of<M>(J, f, 0) + i, 0);
+            xwg_store(af_words_of<M>(J, f, 1) + i, 0);
+        }
+    }
     const float2* X = J.x + static_cast<size_t>(f) * M * W;
     float2* su = J.su + static_cast<size_t>(f) * W * M;
     const int total = U * M, share = (total + gridDim.x - 1) / gridDim.x;
@@ -536,9 +557,22 @@ __device__ __forceinline__ void af_subchunk(const float2 (&s)[AfCfg<M>::E], cons
     __syncthreads();
     for (int m = tid; m < M; m += NTS) {
         float2 t = make_float2(0.0f, 0.0f);
-        for (int k = 0; k < ncol; ++k) t = cadd(t, bufs[k * lds_padded_size(M) + m]);
+        if (ncol == A::SUB) {
+#pragma unroll
+            for (int k = 0; k < A::SUB; ++k) t = cadd(t, bufs[k * lds_padded_size(M) + m]);
+        } else {
+            for (int k = 0; k < ncol; ++k) t = cadd(t, bufs[k * lds_padded_size(M) + m]);
+        }
         put(m, t);
     }
+}
+
+// The sub-chunk of workgroup blockIdx.x of frame f. Only nsub of a frame's gridDim.x (a multiple of 8)
+// workgroups have one, and consecutive workgroups go to the eight XCDs in turn, so the first nsub of
+// every frame would share the first XCDs: frame f's sub-chunks start f nsub workgroups on.
+__device__ __forceinline__ int af_subchunk_of(int f, int nsub) {
+    const unsigned G = gridDim.x;
+    return static_cast<int>((blockIdx.x + G - (static_cast<unsigned>(f) * static_cast<unsigned>(nsub)) % G) % G);
 }
 
 template <int M, bool FOLD>
@@ -547,9 +581,10 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_cols(Job J
     using C = ColCfg<M>;
     constexpr int E = A::E, TPF = A::TPF, SUB = A::SUB, NTS = SUB * TPF;
     HIP_DYNAMIC_SHARED(float2, bufs);   // SUB * lds_padded_size(M), then (FOLD) the phase (M)
-    const int j = blockIdx.x, f = blockIdx.y, tid = threadIdx.x;
+    const int f = blockIdx.y, tid = threadIdx.x;
     const int U = J.dec[f].unit2_num;
     const int nsub = (U + SUB - 1) / SUB;
+    const int j = af_subchunk_of(f, nsub);
     if (j >= nsub) return;   // the whole workgroup leaves before any barrier
     const int c0 = j * SUB;
     const int W = J.W;
@@ -570,16 +605,6 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_cols(Job J
     for (int e = 0; e < E; ++e) s[e] = valid ? col[C::in(lane, e)] : make_float2(0.0f, 0.0f);
     float2* part = af_part_of<M>(J, f, it) + static_cast<size_t>(j) * M;
     af_subchunk<M>(s, phi, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) { part[m] = t; });
-}
-
-// The exchange words of frame f in the resident form: per iteration parity, sub-chunk q < W/SUB
-// and pulse m, the real and the imaginary part of the sub-chunk's per-pulse sum as tagged words
-// (xwg_word). Frame f owns 4 (W/8) M words of af_part, the buffer being sized for it.
-template <int M>
-__device__ __forceinline__ uint64_t* af_words_of(const Job& J, int f, int it) {
-    const size_t nq = static_cast<size_t>(J.W / AfCfg<M>::SUB);
-    uint64_t* frame = reinterpret_cast<uint64_t*>(J.af_part) + static_cast<size_t>(f) * 4 * (J.W / 8) * M;
-    return frame + static_cast<size_t>(it & 1) * nq * M * 2;
 }
 
 // af_phase_from over tagged words (af_words_of): pulse m's sub-chunk sums are loaded eight at a
@@ -627,32 +652,35 @@ __device__ __forceinline__ float2 af_phase_tagged(const uint64_t* words, int nsu
 // the frame's other workgroups; every workgroup then forms the next phase from all nsub sums, in
 // sub-chunk order. The transforms, sums and phases are those of k_af_cols bit for bit.
 // Up to 512 pulses the sums travel as tagged words: each word is polled until it carries
-// iteration it's tag (epoch << 7) | it, where the epoch is the frame's run count that k_autofocus
-// advances before this launch, so words of an earlier run never pass (at most 128 iterations;
-// the host runs the split form above that). At 1024 pulses, where a frame has more sub-chunks and
+// iteration it's tag it + 1; k_af_gather has cleared the words, so those of an earlier run, or
+// whatever the memory held, never pass. At 1024 pulses, where a frame has more sub-chunks and
 // tagged words would double the bytes every workgroup reads per iteration, the sums travel as
 // plain 64-bit words: each thread waits for its stores to be acknowledged, the workgroup counts
 // itself in on the frame's counter (cleared by k_autofocus), and thread 0 polls the counter until
 // all nsub workgroups have counted in for the iteration.
 // Either way a workgroup writes iteration it + 2 into the words of iteration it only after it has
 // read every workgroup's iteration it + 1, which each wrote after reading iteration it.
-// All of a frame's workgroups must be resident together; the dispatcher places a grid's
-// workgroups in order, so every frame but the last one placed is complete, and that one
-// completes as earlier frames finish. A wait that exceeds J.af_wait_polls polls (about a second by
-// default; a negative bound gives up at once) sets status bit 2 of the frame and stops that
-// thread waiting; the frame's phase is then not valid. Workgroup 0 of each frame writes the final
-// phase to J.phi.
+// All of a frame's workgroups must be resident together; every XCD takes its share of a grid's
+// workgroups in order, so where the first incomplete frame lacks one, only complete frames are
+// ahead of it, and it completes as those finish. A wait that exceeds J.af_wait_polls polls (about a
+// second by default; a negative bound gives up at once) sets status bit 2 of the frame and stops
+// that thread waiting; the frame's phase is then not valid, and the default form does the frame
+// over with k_autofocus. Workgroup 0 of each frame writes the final phase to J.phi.
+// Bound by the latency of an iteration (two transforms by one wave per SIMD, the sums, the
+// exchange): 5.5 us at 256 pulses, 7.6 at 512, whether the frames are 1 or 40, as long as every
+// workgroup has a CU for itself and the XCDs share the work (af_subchunk_of; before, 32 frames
+// took 11.3 and 31 us an iteration).
 template <int M>
 __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(Job J) {
     using A = AfCfg<M>;
     using C = ColCfg<M>;
     constexpr int E = A::E, TPF = A::TPF, SUB = A::SUB, NTS = SUB * TPF;
-    constexpr bool kTagged = M <= 512;
     HIP_DYNAMIC_SHARED(float2, bufs);   // SUB * lds_padded_size(M), then the phase (M)
     float2* phi = bufs + SUB * lds_padded_size(M);
-    const int j = blockIdx.x, f = blockIdx.y, tid = threadIdx.x;
+    const int f = blockIdx.y, tid = threadIdx.x;
     const int U = J.dec[f].unit2_num;
     const int nsub = (U + SUB - 1) / SUB;
+    const int j = af_subchunk_of(f, nsub);
     if (j >= nsub) return;   // the whole workgroup leaves before any barrier
     const int c0 = j * SUB;
     const int W = J.W;
@@ -665,14 +693,13 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(J
     for (int e = 0; e < E; ++e) s[e] = valid ? col[C::in(lane, e)] : make_float2(0.0f, 0.0f);
     for (int m = tid; m < M; m += NTS) phi[m] = J.phi[static_cast<size_t>(f) * M + m];
     __syncthreads();
-    const unsigned epoch = J.af_sync[2 * f];
-    unsigned* const count = J.af_sync + 2 * f + 1;
+    unsigned* const count = J.af_sync + f;
     bool waiting = J.af_wait_polls >= 0;   // false once this thread's polls have hit their bound
     if (!waiting && tid == 0) atomicOr(&J.dec[f].status, 2);   // a negative bound: every wait gives up
     for (int it = 0; it < J.iterations; ++it) {
         uint64_t* words = af_words_of<M>(J, f, it);
-        if constexpr (kTagged) {
-            const unsigned tag = (epoch << 7) | static_cast<unsigned>(it);
+        if constexpr (kAfTagged<M>) {
+            const unsigned tag = static_cast<unsigned>(it) + 1;
             af_subchunk<M>(s, phi, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) {
                 uint64_t* w = words + (static_cast<size_t>(j) * M + m) * 2;
                 xwg_store(w, xwg_word(t.x, tag));
@@ -725,6 +752,17 @@ template <int M>
 size_t af_cols_lds(bool fold) {
     return (static_cast<size_t>(AfCfg<M>::SUB) * lds_padded_size(M) + (fold ? M : 0)) * sizeof(float2);
 }
+// LDS of a resident workgroup. The dispatcher puts two or more workgroups on a CU that has the LDS
+// for them while other CUs are idle, which then run an iteration in 7.4 instead of 5.6 us (32 frames
+// of 256 pulses); more than half of the CU's LDS keeps them apart. That holds back workgroups once
+// they outnumber the CUs: a frame commonly selects up to 64 bins, and with that the line lies at
+// three quarters of the CUs (of 256 pulses 40 frames take 0.57 instead of 0.75 ms, 64 frames 1.13
+// instead of 0.79).
+template <int M>
+size_t af_resident_lds(int frames) {
+    const size_t need = af_cols_lds<M>(true);
+    return frames * (64 / AfCfg<M>::SUB) <= 3 * kComputeUnits / 4 ? std::max(need, kLdsBytes / 2 + 1024) : need;
+}
 template <int M>
 size_t colfft_lds() {
     using C = ColCfg<M>;
@@ -771,7 +809,7 @@ hipError_t configure_pa_kernels() {
     set(reinterpret_cast<const void*>(&k_autofocus<MM, true>), autofocus_lds<MM>());   \
     set(reinterpret_cast<const void*>(&k_af_cols<MM, true>), af_cols_lds<MM>(true));   \
     set(reinterpret_cast<const void*>(&k_af_cols<MM, false>), af_cols_lds<MM>(false));   \
-    set(reinterpret_cast<const void*>(&k_af_resident<MM>), af_cols_lds<MM>(true));
+    set(reinterpret_cast<const void*>(&k_af_resident<MM>), af_resident_lds<MM>(1));
     ISAR_SET_PA(64) ISAR_SET_PA(128) ISAR_SET_PA(192) ISAR_SET_PA(256) ISAR_SET_PA(384) ISAR_SET_PA(512)
     ISAR_SET_PA(1024)
 #undef ISAR_SET_PA
@@ -794,8 +832,9 @@ namespace {
 // The start phase and the gathered bins of the split and resident forms (k_af_gather,
 // k_af_bin_doppler, k_autofocus<MM, true>).
 template <int MM>
-void autofocus_start_spread(const Job& J, hipStream_t s) {
-    ISAR_LAUNCH(k_af_gather<MM>, dim3(kAfGatherGroups, J.K), dim3(256), J.W * sizeof(int) + 32 * sizeof(float), s, J);
+void autofocus_start_spread(const Job& J, bool resident, hipStream_t s) {
+    ISAR_LAUNCH(k_af_gather<MM>, dim3(kAfGatherGroups, J.K), dim3(256), J.W * sizeof(int) + 32 * sizeof(float), s, J,
+                resident ? 1 : 0);
     if (!J.phi0_given) ISAR_LAUNCH(k_af_bin_doppler<MM>, dim3((MM - 1 + 255) / 256, J.K), dim3(256), 0, s, J);
     Job J0 = J;
     J0.iterations = 0;
@@ -804,7 +843,7 @@ void autofocus_start_spread(const Job& J, hipStream_t s) {
 
 template <int MM>
 void autofocus_split(const Job& J, bool fold, hipStream_t s) {
-    autofocus_start_spread<MM>(J, s);
+    autofocus_start_spread<MM>(J, false, s);
     constexpr int SUB = AfCfg<MM>::SUB;
     const dim3 cols_grid(J.W / SUB, J.K);
     const dim3 cols_block(SUB * AfCfg<MM>::TPF);
@@ -827,18 +866,23 @@ void launch_autofocus_split(const Job& J, bool fold, hipStream_t s) {
 
 namespace {
 template <int MM>
-void autofocus_resident(const Job& J, hipStream_t s) {
-    autofocus_start_spread<MM>(J, s);
+void autofocus_resident(const Job& J, bool guarded, hipStream_t s) {
+    autofocus_start_spread<MM>(J, true, s);
     if (J.iterations > 0) {
         constexpr int SUB = AfCfg<MM>::SUB;
-        ISAR_LAUNCH_RESIDENT(k_af_resident<MM>, dim3(J.W / SUB, J.K), dim3(SUB * AfCfg<MM>::TPF), af_cols_lds<MM>(true), s,
-                             J);
+        ISAR_LAUNCH_RESIDENT(k_af_resident<MM>, dim3(J.W / SUB, J.K), dim3(SUB * AfCfg<MM>::TPF), af_resident_lds<MM>(J.K),
+                             s, J);
+        if (guarded) {
+            Job redo = J;
+            redo.af_redo = 1;
+            ISAR_LAUNCH(k_autofocus<MM>, dim3(J.K), dim3(AfCfg<MM>::NT), autofocus_lds<MM>(), s, redo);
+        }
     }
 }
 }  // namespace
 
-void launch_autofocus_resident(const Job& J, hipStream_t s) {
-    ISAR_PULSE_SWITCH(J.M, autofocus_resident<MM>(J, s));
+void launch_autofocus_resident(const Job& J, bool guarded, hipStream_t s) {
+    ISAR_PULSE_SWITCH(J.M, autofocus_resident<MM>(J, guarded, s));
 }
 
 }  // namespace isar

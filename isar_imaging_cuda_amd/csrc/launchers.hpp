@@ -31,7 +31,9 @@ void launch_pa_select(const Job& J, hipStream_t s);
 void launch_autofocus(const Job& J, hipStream_t s);
 void launch_autofocus_split(const Job& J, bool fold, hipStream_t s);
 // all iterations in one launch, each frame over several workgroups that stay resident together
-void launch_autofocus_resident(const Job& J, hipStream_t s);
+// (guarded: a frame on which a wait hit its bound is done over by one workgroup, and its status
+// bit 2 cleared)
+void launch_autofocus_resident(const Job& J, bool guarded, hipStream_t s);
 
 // MTRC and azimuth compression (mtrc.cu:4-192, isar_main.cu:191-207)
 void launch_czt_table(int M, int W, int F, double c0, double posa, float2* table, hipStream_t s);

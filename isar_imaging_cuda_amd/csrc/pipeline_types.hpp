@@ -16,11 +16,25 @@
 
 namespace isar {
 
+constexpr int kComputeUnits = 256;    // of the GPU, in 8 XCDs
+constexpr size_t kLdsBytes = 160 * 1024;   // of a compute unit
 constexpr int kRangeCut = 512;        // RANGE_NUM_CUT (common.cuh:71)
 constexpr int kRangeNumIfdsPc = 4096; // RANGE_NUM_IFDS_PC (common.cuh:72)
 constexpr int kRaChunkRowsDefault = 8;   // rows per workgroup in the alignment update kernel
 constexpr int kCutBandRows = 16;      // rows per workgroup when cutting the range window
-constexpr int kAfSplitFrames = 32;    // batches of at most this many frames split the autofocus
+// Default autofocus form by batch size: several resident workgroups per frame up to this many frames,
+// one workgroup per frame above. The latter takes a CU per frame and leaves the others idle: at 64
+// selected bins 128 frames take 0.86 (resident) and 0.92 ms at 256 pulses, 2.5 and 2.8 at 512, 5.4
+// and 5.9 at 1024; 40 frames of 512 pulses 0.84 and 2.7. A batch that fills the CUs is the other way
+// round: 256 frames of 256 pulses 1.0 ms with one workgroup each, and more than that resident.
+constexpr int kAfResidentFrames = 128;
+// Bound of a resident wait in the default form, in polls of about a microsecond; a frame that
+// reaches it is done over by one workgroup. Frames of a full launch wait for earlier ones, at most a
+// few milliseconds.
+constexpr int kAfGuardedPolls = 1 << 16;
+// Sub-aperture plans run several groups at once; their default is the split form up to this many
+// windows, one workgroup per window above.
+constexpr int kAfSplitFrames = 32;
 // batches of at least this many echo cells (frames x pulses x range cells; 32 frames of 256 x 4096)
 // update the final rows of range alignment in a launch of their own
 constexpr long long kRaSplitCells = 1LL << 25;
@@ -53,6 +67,7 @@ struct Job {
     int ra_split;                 // alignment update grids per level: 0 by batch size, 1 one, 2 two
     int czt_threads;              // chirp-z workgroup width (256 or 512 threads)
     int af_wait_polls;            // bound of each resident-autofocus wait in polls (< 0: give up at once)
+    int af_redo;                  // k_autofocus: only the frames with status bit 2, which it clears
     double hpc_k;                 // HPC phase in half-turns = hpc_k * v * n^2
     double czt_c0, czt_posa;      // alpha_n = 1 - c0 + posa * n
     // inputs
@@ -87,7 +102,7 @@ struct Job {
     float2* czt;                  // K x M x W (chirp-z output)
     float2* colsum;               // K x W
     float2* af_part;              // K x 4 (W/8) M: per-pulse sums per sub-chunk of selected bins, by iteration parity (split autofocus: the first half; resident: all, as tagged words)
-    unsigned* af_sync;            // 2K: per frame the run count (the resident autofocus's exchange epoch, advanced by k_autofocus) and its hand-off counter (cleared there)
+    unsigned* af_sync;            // K: per frame the resident autofocus's hand-off counter, cleared by k_autofocus
     const float2* czt_table;      // W x F (FFT of the Bluestein chirp per range bin)
     const float2* czt_pre;        // W x M: exp(j pi a_n m (M - m) / M), the input chirp
     const float2* czt_post;       // W x M: exp(-j pi a_n k^2 / M) / F, the output chirp

@@ -218,6 +218,36 @@ def test_resident_wait_bound_sets_status():
         assert np.array_equal(phis[(isar.AF_SPLIT, False)][k], phis[(isar.AF_RESIDENT, False)][k])
 
 
+@pytest.mark.parametrize("M,N,frames,polls", [(64, 1024, 128, None), (192, 1024, 49, None), (256, 1024, 129, None),
+                                              (512, 1024, 40, None), (1024, 2048, 3, None), (128, 1024, 3, -1),
+                                              (1024, 2048, 3, -1)])
+def test_default_autofocus_form_equals_the_explicit_forms(M, N, frames, polls):
+    """AUTO takes the resident form up to 128 frames, with one workgroup per CU for the smaller batches,
+    and one workgroup per frame above; a frame whose wait gave up (negative bound) is done over. Phases
+    and images equal those of one workgroup per frame bit for bit and no frame reports status bit 2;
+    140 iterations, above the 128 that a 7-bit iteration tag would hold."""
+    cfgs = [synth.preset(1, echo_num=M, range_num=N, seed=320 + k) for k in range(3)]
+    data = [synth.frame(c) for c in cfgs]
+    radar = synth.radar_header(cfgs[0])
+    echo = np.stack([data[k % 3][0] for k in range(frames)])
+    vel = np.stack([data[k % 3][1] for k in range(frames)])
+    print(f"[case] default autofocus form M={M} N={N} frames={frames} polls={polls}", flush=True)
+    params = isar.RadarParams(M, N, radar["band_width"], radar["fc"], radar["Tp"], radar["Fs"])
+    out = {}
+    for mode in (isar.AF_AUTO, isar.AF_FUSED):
+        with isar.Imager(params, max_frames=frames) as im:
+            im.set_autofocus_mode(mode)
+            if polls is not None:
+                im.set_af_wait_polls(polls)
+            img = im.run_host(echo, vel, isar.Options(iterations=140))
+            out[mode] = (img, [im.trace(k) for k in range(frames)])
+    for k in range(frames):
+        a, b = out[isar.AF_AUTO][1][k], out[isar.AF_FUSED][1][k]
+        assert a.status & 2 == 0, f"frame {k}"
+        assert np.array_equal(a.phi, b.phi), f"frame {k}: phases differ"
+    assert np.array_equal(out[isar.AF_AUTO][0], out[isar.AF_FUSED][0])
+
+
 def test_batch_matches_single_frames():
     cfgs = [synth.preset(1, seed=100 + k) for k in range(3)]
     frames = [synth.frame(c) for c in cfgs]
