@@ -22,8 +22,8 @@ __device__ __forceinline__ short to_bf16(float f) {
     return static_cast<short>(u >> 16);
 }
 __device__ __forceinline__ __bf16 bits_bf16(short s) { return __builtin_bit_cast(__bf16, s); }
-__device__ __forceinline__ __bf16 load_bf16(const float* p) { return bits_bf16(to_bf16(*p)); }
-__device__ __forceinline__ __bf16 load_bf16(const uint16_t* p) { return bits_bf16(static_cast<short>(*p)); }
+__device__ __forceinline__ short as_bf16(float f) { return to_bf16(f); }
+__device__ __forceinline__ short as_bf16(uint16_t b) { return static_cast<short>(b); }
 
 // D = A B + C for one 16 x 16 x 32 tile. Lane l holds A[l % 16][8 (l / 16) + t] and
 // B[8 (l / 16) + t][l % 16] for t < 8, and D[4 (l / 16) + t][l % 16] for t < 4.
@@ -31,56 +31,99 @@ __device__ __forceinline__ f32x4 mfma16x32(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-constexpr int kGemmTile = 32;   // output rows and columns per wave (2 x 2 MFMA tiles)
+// Eight consecutive k of one row (or column) of an operand as they are in memory. VEC: they are
+// consecutive there and aligned to their size (16 bytes at most a load), and k is a multiple of 8.
+// Nothing outside the operand is read: where line >= lines or kk >= k the last one inside is, and the
+// values of kk >= k become zeros.
+template <typename T, bool VEC>
+struct Frag {
+    static constexpr int kWords = VEC ? static_cast<int>(8 * sizeof(T) / 16) : 8;
+    typename std::conditional<VEC, uint4, T>::type v[kWords];
+    __device__ __forceinline__ void load(const T* p, int line, int lines, long s_line, int kk, int k, long s_k) {
+        p += min(line, lines - 1) * s_line;
+        if constexpr (VEC) {
+            const uint4* q = reinterpret_cast<const uint4*>(p + min(kk, k - 8));
+#pragma unroll
+            for (int i = 0; i < kWords; ++i) v[i] = q[i];
+        } else {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) v[t] = p[min(kk + t, k - 1) * s_k];
+        }
+    }
+    __device__ __forceinline__ bf16x8 get(int kk, int k) const {
+        T e[8];
+        if constexpr (VEC) __builtin_memcpy(e, v, sizeof e);
+        else {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) e[t] = v[t];
+        }
+        bf16x8 r;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) r[t] = bits_bf16(kk + t < k ? as_bf16(e[t]) : static_cast<short>(0));
+        return r;
+    }
+};
 
 }  // namespace
 
 // C[m][n] = sum_k A(m, k) B(k, n) with A(m, k) = a[m sam + k sak], B(k, n) = b[k sbk + n sbn],
-// operands rounded to BF16, products accumulated in FP32. One wave per 32 x 32 block of C.
-// Epilogue: 0 store; 1 + bias[n], then max(0, .); 2 + bias[n]; 3 times (mask[m][n] > 0).
-template <typename TA, typename TB, int EPI>
+// operands rounded to BF16, products accumulated in FP32 in the order of k. One wave per block of
+// 16 T x 16 T of C. Epilogue: 0 store; 1 + bias[n], then max(0, .); 2 + bias[n]; 3 times (mask[m][n] > 0).
+// AV, BV: the operand's k are consecutive and aligned (Frag).
+//
+// Bound by the latency of its loads: the matrix work of a layer is under a microsecond, its
+// operands are in the L2, and the sums follow k, so that a wave has a serial chain over k. So the
+// loads of four steps of 32 k (two for T = 2) are issued together, 16 bytes each where the layout allows,
+// and small products take T = 1, four times as many waves (use_small_tiles). The first layer of the 256-pulse network,
+// 256 x 128 x 1024, takes 15 us (95 with a step's loads waited for one by one and 32 x 32 tiles),
+// the training step's products 80 instead of 406.
+template <typename TA, typename TB, int EPI, int T, bool AV, bool BV>
 __global__ __launch_bounds__(64) void k_gemm_bf16(int m, int n, int k, const TA* __restrict__ a, long sam, long sak,
                                                   const TB* __restrict__ b, long sbk, long sbn, float* __restrict__ c,
                                                   long scm, const float* __restrict__ bias,
                                                   const float* __restrict__ mask, long smm) {
+    constexpr int kTile = 16 * T, kSteps = T == 1 ? 4 : 2;
     const int l = threadIdx.x;
-    const int bm = blockIdx.y * kGemmTile, bn = blockIdx.x * kGemmTile;
+    const int bm = blockIdx.y * kTile, bn = blockIdx.x * kTile;
     const int li = l % 16, lk = 8 * (l / 16), lr = 4 * (l / 16);
-    f32x4 acc[2][2];
+    f32x4 acc[T][T];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < T; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const __bf16 zero = bits_bf16(0);
-    for (int k0 = 0; k0 < k; k0 += 32) {
-        bf16x8 fa[2], fb[2];
+        for (int j = 0; j < T; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k0 = 0; k0 < k; k0 += 32 * kSteps) {
+        Frag<TA, AV> fa[kSteps][T];
+        Frag<TB, BV> fb[kSteps][T];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int row = bm + 16 * i + li;
+        for (int q = 0; q < kSteps; ++q) {
+            const int kk = k0 + 32 * q + lk;
 #pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int kk = k0 + lk + t;
-                fa[i][t] = (row < m && kk < k) ? load_bf16(a + row * sam + kk * sak) : zero;
+            for (int i = 0; i < T; ++i) {
+                fa[q][i].load(a, bm + 16 * i + li, m, sam, kk, k, sak);
+                fb[q][i].load(b, bn + 16 * i + li, n, sbn, kk, k, sbk);
             }
         }
+        issue_point();
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int col = bn + 16 * j + li;
+        for (int q = 0; q < kSteps; ++q) {
+            const int kk = k0 + 32 * q + lk;
+            if (k0 + 32 * q >= k) break;
+            bf16x8 va[T], vb[T];
 #pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int kk = k0 + lk + t;
-                fb[j][t] = (col < n && kk < k) ? load_bf16(b + kk * sbk + col * sbn) : zero;
+            for (int i = 0; i < T; ++i) {
+                va[i] = fa[q][i].get(kk, k);
+                vb[i] = fb[q][i].get(kk, k);
             }
+#pragma unroll
+            for (int i = 0; i < T; ++i)
+#pragma unroll
+                for (int j = 0; j < T; ++j) acc[i][j] = mfma16x32(va[i], vb[j], acc[i][j]);
         }
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = mfma16x32(fa[i], fb[j], acc[i][j]);
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < T; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < T; ++j) {
             const int col = bn + 16 * j + li;
             if (col >= n) continue;
 #pragma unroll
@@ -96,13 +139,35 @@ __global__ __launch_bounds__(64) void k_gemm_bf16(int m, int n, int k, const TA*
         }
 }
 
-// bias gradient: db[j] = sum_b dz[b][j]
-__global__ void k_colsum(int rows, int cols, const float* __restrict__ dz, float* __restrict__ db) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= cols) return;
+// bias gradient: db[j] = sum_b dz[b][j]. A workgroup takes 64 columns, each wave a contiguous 16th of
+// the rows with sixteen loads in flight; the waves' sums are added in wave order. Bound by latency:
+// 256 rows take 2 to 4 us, with one thread per column and a load waited for per row they took 59.
+constexpr int kColsumWaves = 16;
+__global__ __launch_bounds__(64 * kColsumWaves) void k_colsum(int rows, int cols, const float* __restrict__ dz,
+                                                              float* __restrict__ db) {
+    __shared__ float part[kColsumWaves][64];
+    const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
+    const int j = blockIdx.x * 64 + lane;
+    const int share = (rows + kColsumWaves - 1) / kColsumWaves;
+    const int r0 = min(w * share, rows), r1 = min(r0 + share, rows);
+    const float* col = dz + min(j, cols - 1);
     float s = 0.0f;
-    for (int r = 0; r < rows; ++r) s += dz[static_cast<size_t>(r) * cols + j];
-    db[j] = s;
+    for (int r = r0; r < r1; r += 16) {
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = col[static_cast<size_t>(min(r + i, r1 - 1)) * cols];
+        issue_point();
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (r + i < r1) s += v[i];
+    }
+    part[w][lane] = s;
+    __syncthreads();
+    if (w != 0 || j >= cols) return;
+    float t = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kColsumWaves; ++i) t += part[i][lane];
+    db[j] = t;
 }
 
 // Adam (bias-corrected) on FP32 master parameters; the BF16 copy of each weight follows.
@@ -253,30 +318,59 @@ __global__ void k_image_entropy(int n, const float* __restrict__ img, double* __
 // host launchers
 // ------------------------------------------------------------------------------------------
 namespace {
-dim3 gemm_grid(int m, int n) { return dim3((n + kGemmTile - 1) / kGemmTile, (m + kGemmTile - 1) / kGemmTile); }
+// 16 x 16 tiles until 32 x 32 tiles give every SIMD a wave; above, the larger tiles read each operand
+// half as often. 1024 x 2048 x 128 (2048 tiles of 32 x 32) takes 9.9 us in the larger and 14.5 in the
+// smaller tiles, 2048 x 128 x 512 (256) 17.5 and 13.3, 1024 x 128 x 4096 (128) 84 and 52; at 512 tiles
+// it depends on k (31 and 36 us at k = 1024, 7.0 and 6.0 at 128).
+bool use_small_tiles(int m, int n) {
+    return static_cast<long long>((m + 31) / 32) * ((n + 31) / 32) < 4 * kComputeUnits;
+}
+
+// Whether the eight k of a fragment can be read as 16-byte words.
+template <typename T>
+bool vector_k(const T* p, long s_k, long s_line, int k) {
+    constexpr long per = 16 / static_cast<long>(sizeof(T));
+    return s_k == 1 && s_line % per == 0 && k % 8 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+}
+
+// AK, BK: the callers' layouts have consecutive k in that operand; both must be readable so, or
+// neither is.
+template <typename TA, typename TB, int EPI, bool AK, bool BK>
+void gemm_bf16(int m, int n, int k, const TA* a, long sam, long sak, const TB* b, long sbk, long sbn, float* c, long scm,
+               const float* bias, const float* mask, long smm, hipStream_t s) {
+    const bool small = use_small_tiles(m, n);
+    const bool vec = (AK || BK) && (!AK || vector_k(a, sak, sam, k)) && (!BK || vector_k(b, sbk, sbn, k));
+    const int tile = small ? 16 : 32;
+    const dim3 grid((n + tile - 1) / tile, (m + tile - 1) / tile);
+#define ISAR_GEMM(T, AV, BV)                                                                                           \
+    ISAR_LAUNCH((k_gemm_bf16<TA, TB, EPI, T, AV, BV>), grid, dim3(64), 0, s, m, n, k, a, sam, sak, b, sbk, sbn, c, scm, \
+                bias, mask, smm)
+    if (vec) {
+        if (small) ISAR_GEMM(1, AK, BK);
+        else ISAR_GEMM(2, AK, BK);
+    } else {
+        if (small) ISAR_GEMM(1, false, false);
+        else ISAR_GEMM(2, false, false);
+    }
+#undef ISAR_GEMM
+}
 }  // namespace
 
 void launch_gemm_f32_bf16w(int m, int n, int k, const float* a, long sam, long sak, const uint16_t* w, long sbk,
                            long sbn, float* c, long scm, const float* bias, int relu, hipStream_t s) {
-    if (relu)
-        ISAR_LAUNCH((k_gemm_bf16<float, uint16_t, 1>), gemm_grid(m, n), dim3(64), 0, s, m, n, k, a, sam, sak, w, sbk,
-                    sbn, c, scm, bias, static_cast<const float*>(nullptr), 0L);
-    else
-        ISAR_LAUNCH((k_gemm_bf16<float, uint16_t, 2>), gemm_grid(m, n), dim3(64), 0, s, m, n, k, a, sam, sak, w, sbk,
-                    sbn, c, scm, bias, static_cast<const float*>(nullptr), 0L);
+    if (relu) gemm_bf16<float, uint16_t, 1, true, false>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, bias, nullptr, 0L, s);
+    else gemm_bf16<float, uint16_t, 2, true, false>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, bias, nullptr, 0L, s);
 }
 void launch_gemm_f32_bf16w_masked(int m, int n, int k, const float* a, long sam, long sak, const uint16_t* w,
                                   long sbk, long sbn, float* c, long scm, const float* mask, long smm, hipStream_t s) {
-    ISAR_LAUNCH((k_gemm_bf16<float, uint16_t, 3>), gemm_grid(m, n), dim3(64), 0, s, m, n, k, a, sam, sak, w, sbk, sbn,
-                c, scm, static_cast<const float*>(nullptr), mask, smm);
+    gemm_bf16<float, uint16_t, 3, true, true>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, nullptr, mask, smm, s);
 }
 void launch_gemm_f32_f32(int m, int n, int k, const float* a, long sam, long sak, const float* b, long sbk, long sbn,
                          float* c, long scm, hipStream_t s) {
-    ISAR_LAUNCH((k_gemm_bf16<float, float, 0>), gemm_grid(m, n), dim3(64), 0, s, m, n, k, a, sam, sak, b, sbk, sbn, c,
-                scm, static_cast<const float*>(nullptr), static_cast<const float*>(nullptr), 0L);
+    gemm_bf16<float, float, 0, false, false>(m, n, k, a, sam, sak, b, sbk, sbn, c, scm, nullptr, nullptr, 0L, s);
 }
 void launch_colsum(int rows, int cols, const float* dz, float* db, hipStream_t s) {
-    ISAR_LAUNCH(k_colsum, dim3((cols + 255) / 256), dim3(256), 0, s, rows, cols, dz, db);
+    ISAR_LAUNCH(k_colsum, dim3((cols + 63) / 64), dim3(64 * kColsumWaves), 0, s, rows, cols, dz, db);
 }
 void launch_adam(int n, float* p, const float* g, float* m1, float* m2, uint16_t* pb, const int* bf_index, float lr,
                  float beta1, float beta2, float eps, float c1, float c2, hipStream_t s) {

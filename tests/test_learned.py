@@ -132,6 +132,29 @@ def test_network_forward_and_gradients_match_oracle(widths, batch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("widths,batch", [([8, 8], 1), ([13, 70], 5), ([136, 1030], 1030), ([24, 1024], 1024),
+                                          ([520, 17], 33)])
+def test_one_layer_products_at_tile_edges_match_oracle(widths, batch):
+    """Lengths that are and are not multiples of 8 (16-byte and single loads), of the 16 x 16 and
+    32 x 32 tiles and of the steps of 32 (issued four or two at a time), both tile sizes, and column sums
+    of fewer and more rows than waves. Both sides multiply the same BF16 operands, and a product of K
+    terms accumulated in FP32 is off by at most K 2^-23 times the sum of their magnitudes (an addition
+    by an ulp)."""
+    print(f"[case] one layer {widths} batch {batch}", flush=True)
+    net, params, x, y, out, grad_out, _ = _net_roundtrip(widths, batch, widths[1] + batch)
+    i, o = widths
+    w = MO.bf16_round(params[:i * o].reshape(i, o)).astype(np.float64)
+    xb, gb = MO.bf16_round(x).astype(np.float64), MO.bf16_round(grad_out).astype(np.float64)
+    b = params[i * o:].astype(np.float64)
+    eps = 2.0 ** -23
+    assert np.all(np.abs(out - (xb @ w + b)) <= (i + 1) * eps * (np.abs(xb) @ np.abs(w) + np.abs(b)) + 1e-30)
+    g = net.get_grads()
+    assert np.all(np.abs(g[:i * o].reshape(i, o) - xb.T @ gb) <= batch * eps * (np.abs(xb).T @ np.abs(gb)) + 1e-30)
+    go = grad_out.astype(np.float64)
+    assert np.all(np.abs(g[i * o:] - go.sum(0)) <= batch * eps * np.abs(go).sum(0) + 1e-30)
+
+
+@pytest.mark.gpu
 def test_adam_step_matches_oracle():
     torch = _torch()
     widths = [32, 16, 8]
