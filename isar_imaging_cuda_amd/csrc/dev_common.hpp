@@ -293,6 +293,13 @@ __device__ __forceinline__ float opaque(float v) {
     return v;
 }
 
+__device__ __forceinline__ double opaque(double v) {
+#ifndef ISAR_EMU
+    asm volatile("" : "+v"(v));
+#endif
+    return v;
+}
+
 __device__ __forceinline__ float2 opaque(float2 v) {
 #ifndef ISAR_EMU
     asm volatile("" : "+v"(v.x), "+v"(v.y));

@@ -237,6 +237,32 @@ def test_image_entropy_matches_oracle():
     assert e[2] == 0.0
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 1024, 8191, 8193, 40000])
+def test_image_entropy_lengths_and_scales(n):
+    """Fewer cells than threads, whole and broken groups of loads, and magnitudes whose squares leave
+    FP32's range. Both formulas are FP64: H = ln T - S / T is off by the rounding of two numbers of
+    the size of the largest |ln q| and of sums over n / 1024 + 26 additions."""
+    torch = _torch()
+    from isar_imaging_cuda_amd import learned as L
+    rng = np.random.default_rng(n)
+    scales = (1.0, 1e-18, 1e-44, 3e18, 4e37)
+    imgs = np.stack([np.abs(rng.standard_normal(n)) * s for s in scales]).astype(np.float32)
+    imgs[:, ::3] = 0.0
+    imgs[:, n - 1] = scales
+    d = torch.from_numpy(imgs).to("cuda:0")
+    out = torch.zeros(len(scales), dtype=torch.float64, device="cuda:0")
+    L.image_entropy(len(scales), n, d.data_ptr(), out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for k, e in enumerate(out.cpu().numpy()):
+        q = imgs[k].astype(np.longdouble) ** 2
+        q = q[q > 0] if np.any(q > 0) else np.ones(1, np.longdouble)
+        p = q / q.sum()
+        ref = float(-(p * np.log(p)).sum())
+        bound = (n / 1024 + 30) * 2.0 ** -52 * 2 * max(1.0, float(np.abs(np.log(q)).max()))
+        assert abs(e - ref) <= bound, (scales[k], e, ref)
+
+
 def _c4_batch(K, seed0):
     from isar_imaging_cuda_amd import learned as L
     echo, vel, h = L.synth_frames(4, list(range(seed0, seed0 + K)))
