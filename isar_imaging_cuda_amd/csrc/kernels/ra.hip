@@ -153,8 +153,23 @@ __device__ __forceinline__ void group_energy(float (&a)[kE], const Job& J, int f
         if (r0 < M) {
             const int r1 = min(r0 + s2, M);
             const int R = min(s2, J.ra_chunk);
-            for (int h = r0; h < r1; h += R) {
-                const float* pp = J.epart + (static_cast<size_t>(f) * M + h) * N;
+            const float* pp = J.epart + (static_cast<size_t>(f) * M + r0) * N;
+            const size_t step = static_cast<size_t>(R) * N;
+            int left = (r1 - r0 + R - 1) / R;
+            constexpr int kAtOnce = N >= 8192 ? 2 : 4;   // partial sums with their loads in flight together
+            for (; left >= kAtOnce; left -= kAtOnce, pp += kAtOnce * step) {
+                float v[kAtOnce][kE];
+#pragma unroll
+                for (int q = 0; q < kAtOnce; ++q)
+#pragma unroll
+                    for (int e = 0; e < kE; ++e) v[q][e] = elem_u32(pp + q * step, row_pos<N>(tid, e));
+                issue_point();
+#pragma unroll
+                for (int q = 0; q < kAtOnce; ++q)
+#pragma unroll
+                    for (int e = 0; e < kE; ++e) a[e] += v[q][e];
+            }
+            for (; left > 0; --left, pp += step) {
 #pragma unroll
                 for (int e = 0; e < kE; ++e) a[e] += elem_u32(pp, row_pos<N>(tid, e));
             }
@@ -523,6 +538,82 @@ __global__ __launch_bounds__(N / kE, PART == kUpdFinal && N <= 4096 ? 3 : 4) voi
     for (int e = 0; e < kE; ++e) elem_u32(dst, row_pos<N>(tid, e)) = acc[e];
 }
 
+// k_ra_upd (kUpdAll) for batches that leave the GPU idle with one row of each chunk at a time: a
+// workgroup takes G rows of its chunk at once, N / 16 threads each with a transform buffer of its
+// own. The rows' energies go through those buffers, and every thread adds 16 / G cells over the rows
+// in their order: the sums are k_ra_upd's bit for bit.
+// Bound by latency (a row's loads, ramp and transform, one after the other): a level of 13 frames of
+// 192 x 2048 in chunks of 8 takes 15 us instead of 36, of one frame of 256 x 4096 in chunks of 2 9
+// instead of 14; imaging 32 such frames in chunks of 8 1.39 ms instead of 1.48.
+template <int N, int G>
+__global__ __launch_bounds__(N / kE * G) void k_ra_upd_rows(Job J, int s, int pair_base) {
+    HIP_DYNAMIC_SHARED(float2, lds);   // G transform buffers, 64 floats of reductions, constants (rows_words)
+    constexpr int T = N / kE, B = lds_padded_size(N), C = kE / G;
+    const int b = blockIdx.x, f = blockIdx.y, g = threadIdx.x / T, tid = threadIdx.x % T;
+    const int M = J.M;
+    const int R = min(s, J.ra_chunk);
+    const int cpp = (s + R - 1) / R;
+    const int p = b / cpp, i = b % cpp;
+    const int gend = min((2 * p + 2) * s, M);
+    const int r0 = (2 * p + 1) * s + i * R;
+    const int r1 = min(r0 + R, gend);
+    if (r0 >= r1) return;
+    const double lag = uniform(J.lags[static_cast<size_t>(f) * (M - 1) + pair_base + p]);
+    const bool final_rows = p == 0;
+    float* const red = reinterpret_cast<float*>(lds + G * B);
+    const auto tw = fft_twiddles_lds<N, kE>(tid, reinterpret_cast<FftCT*>(red + 64));
+    float2* const buf = lds + g * B;
+    float acc[C], arp[C];
+    float mx = 0.0f;
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[c] = arp[c] = 0.0f;
+#pragma unroll 1
+    for (int m0 = r0; m0 < r1; m0 += G) {
+        const int m = min(m0 + g, r1 - 1);   // past the chunk's end: the last row, not used
+        float2 x[kE];
+        load_row_shifted<N>(x, J, f, m, J.lagsum[static_cast<size_t>(f) * M + m], lag, tid);
+        fft_after_first<N, kE, +1>(x, buf, tid, tw);
+        if (final_rows && m0 + g < r1) {   // S0 of the row was read before the transform's first barrier
+            float2* st = J.st + (static_cast<size_t>(f) * M + m) * N;
+            const int t = opaque(tid);
+#pragma unroll
+            for (int e = 0; e < kE; ++e) elem_u32(st, row_pos<N>(t, e)) = x[e];
+        }
+        __syncthreads();   // the transforms' last reads
+#pragma unroll
+        for (int e = 0; e < kE; ++e) reinterpret_cast<float*>(buf)[row_pos<N>(tid, e)] = cabs2(x[e]);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            if (m0 + q >= r1) break;
+            const float* row = reinterpret_cast<const float*>(lds + q * B) + threadIdx.x;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const float e = row[c * T * G];
+                acc[c] += e;
+                if (final_rows) {
+                    const float av = sqrt_hw(e);
+                    arp[c] += av;
+                    mx = fmaxf(mx, av);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    const size_t cell = threadIdx.x;
+    if (final_rows) {
+        float* ap = J.arp_part + (static_cast<size_t>(f) * (M / 2) + r0 / 2) * N + cell;
+#pragma unroll
+        for (int c = 0; c < C; ++c) ap[c * T * G] = arp[c];
+        mx = block_max<T * G>(mx, red);
+        if (threadIdx.x == 0) J.max_part[static_cast<size_t>(f) * (M / 2) + r0 / 2] = mx;
+    }
+    if (static_cast<int>(threadIdx.x) < r1 - r0) J.lagsum[static_cast<size_t>(f) * M + r0 + threadIdx.x] += lag;
+    float* dst = J.epart + (static_cast<size_t>(f) * M + r0) * N + cell;
+#pragma unroll
+    for (int c = 0; c < C; ++c) dst[c * T * G] = acc[c];
+}
+
 // Range Hamming window 0.54 - 0.46 cos(2 pi n / (N - 1)) (genHammingVec, common.cu:260-266),
 // evaluated in FP64 and rounded once to FP32.
 __global__ __launch_bounds__(256) void k_range_window(int N, float* win) {
@@ -536,6 +627,37 @@ __global__ __launch_bounds__(256) void k_range_window(int N, float* win) {
 namespace {
 template <int N>
 size_t ra_lds() { return row_words(N) * sizeof(float) + kFft16Bytes; }
+template <int N, int G>
+size_t ra_rows_lds() { return G * lds_padded_size(N) * sizeof(float2) + 64 * sizeof(float) + kFft16Bytes; }
+
+// The rows that k_ra_upd_rows may take at once: up to 8, in workgroups of at most 1024 threads.
+template <int N>
+constexpr int kRowsMax = N >= 16384 ? 1 : N == 8192 ? 2 : N == 4096 ? 4 : 8;
+
+// Rows at once of a level's chunks of R rows: doubled until the grid gives every SIMD four waves, which
+// is what fits beside each other; with that many, chunks row by row do as well without the exchange.
+template <int N>
+int rows_at_once(int frames, int nblocks, int R) {
+    const long long waves = static_cast<long long>(frames) * nblocks * (N / kE / 64);
+    int g = 1;
+    while (2 * g <= std::min(R, kRowsMax<N>) && waves * g < 4 * 4 * kComputeUnits) g *= 2;
+    return g;
+}
+
+template <int N, int G>
+void launch_upd_rows(const Job& J, int stride, int pair_base, int nblocks, hipStream_t s) {
+    if constexpr (G <= kRowsMax<N>)
+        ISAR_LAUNCH((k_ra_upd_rows<N, G>), dim3(nblocks, J.K), dim3(N / kE * G), (ra_rows_lds<N, G>()), s, J, stride, pair_base);
+}
+template <int N>
+bool upd_rows(const Job& J, int stride, int pair_base, int nblocks, int R, hipStream_t s) {
+    switch (rows_at_once<N>(J.K, nblocks, R)) {
+    case 2: launch_upd_rows<N, 2>(J, stride, pair_base, nblocks, s); return true;
+    case 4: launch_upd_rows<N, 4>(J, stride, pair_base, nblocks, s); return true;
+    case 8: launch_upd_rows<N, 8>(J, stride, pair_base, nblocks, s); return true;
+    default: return false;
+    }
+}
 
 #define ISAR_RANGE_SWITCH(N, BODY)                     \
     switch (N) {                                       \
@@ -572,6 +694,10 @@ hipError_t configure_ra_kernels() {
     set(reinterpret_cast<const void*>(&k_ra_upd<NN, kUpdRest>), ra_lds<NN>());
     ISAR_SET_RA(1024) ISAR_SET_RA(2048) ISAR_SET_RA(4096) ISAR_SET_RA(8192) ISAR_SET_RA(16384)
 #undef ISAR_SET_RA
+#define ISAR_SET_ROWS(NN, GG) set(reinterpret_cast<const void*>(&k_ra_upd_rows<NN, GG>), ra_rows_lds<NN, GG>());
+    ISAR_SET_ROWS(1024, 2) ISAR_SET_ROWS(1024, 4) ISAR_SET_ROWS(1024, 8) ISAR_SET_ROWS(2048, 2) ISAR_SET_ROWS(2048, 4)
+    ISAR_SET_ROWS(2048, 8) ISAR_SET_ROWS(4096, 2) ISAR_SET_ROWS(4096, 4) ISAR_SET_ROWS(8192, 2)
+#undef ISAR_SET_ROWS
 #endif
     return err;
 }
@@ -595,15 +721,21 @@ void launch_ra_corr(const Job& J, int stride, int pair_base, int nblocks, hipStr
                                        stride, pair_base));
 }
 void launch_ra_upd(const Job& J, int stride, int pair_base, int nblocks, hipStream_t s) {
-    // nblocks = pairs x chunks per pair. Large batches launch pair 0 (final rows) and the other
+    // nblocks = pairs x chunks per pair. Chunks that would leave SIMDs without work take several rows at
+    // once. Large batches launch pair 0 (final rows) and the other
     // pairs apart; small ones, where the second launch per level costs more than it saves, in one.
+    const int R = std::min(stride, J.ra_chunk), cpp = (stride + R - 1) / R;
+    if (J.ra_split == 0) {
+        bool done = false;
+        ISAR_RANGE_SWITCH(J.N, done = upd_rows<NN>(J, stride, pair_base, nblocks, R, s));
+        if (done) return;
+    }
     const bool split = J.ra_split == 2 || (J.ra_split == 0 && static_cast<long long>(J.K) * J.M * J.N >= kRaSplitCells);
     if (!split) {
         ISAR_RANGE_SWITCH(J.N, ISAR_LAUNCH((k_ra_upd<NN, kUpdAll>), dim3(nblocks, J.K), dim3(NN / kE), ra_lds<NN>(),
                                            s, J, stride, pair_base));
         return;
     }
-    const int R = std::min(stride, J.ra_chunk), cpp = (stride + R - 1) / R;
     const int rest = nblocks - cpp;
     ISAR_RANGE_SWITCH(J.N, ISAR_LAUNCH((k_ra_upd<NN, kUpdFinal>), dim3(cpp, J.K), dim3(NN / kE), ra_lds<NN>(), s, J,
                                        stride, pair_base));

@@ -280,6 +280,31 @@ def test_ra_update_launch_forms_agree(cid, over):
     assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("M,N,chunk,frames", [(64, 1024, 8, 1), (192, 1024, 16, 3), (128, 2048, 4, 2), (192, 2048, 2, 1),
+                                              (384, 4096, 8, 1), (64, 8192, 16, 2), (64, 16384, 8, 1), (256, 1024, 8, 40)])
+def test_ra_update_rows_at_once_agree(M, N, chunk, frames):
+    """Small batches update several rows of a chunk at once (2, 4 or 8 by length, chunk and batch; one at
+    a time for the longest rows and from about 40 frames of 256 x 1024): lags, phases and images equal the
+    row-by-row launches bit for bit, odd groups carried up a level (192 and 384 pulses) included."""
+    cfgs = [synth.preset(1, echo_num=M, range_num=N, seed=340 + k) for k in range(min(frames, 3))]
+    data = [synth.frame(c) for c in cfgs]
+    radar = synth.radar_header(cfgs[0])
+    echo = np.stack([data[k % len(data)][0] for k in range(frames)])
+    vel = np.stack([data[k % len(data)][1] for k in range(frames)])
+    print(f"[case] rows at once M={M} N={N} chunk={chunk} frames={frames}", flush=True)
+    params = isar.RadarParams(M, N, radar["band_width"], radar["fc"], radar["Tp"], radar["Fs"])
+    out = []
+    for split in (0, 1, 2):
+        with isar.Imager(params, max_frames=frames) as im:
+            im.set_ra_chunk(chunk)
+            im.set_ra_split(split)
+            out.append((im.run_host(echo, vel, isar.Options()), [im.trace(k) for k in range(frames)]))
+    for img, tr in out[1:]:
+        for k in range(frames):
+            assert np.array_equal(out[0][1][k].ra_lag, tr[k].ra_lag) and np.array_equal(out[0][1][k].phi, tr[k].phi)
+        assert np.array_equal(out[0][0], img)
+
+
 @pytest.mark.parametrize("M,N", [(64, 1024), (128, 1024), (192, 1024), (256, 2048), (384, 1024), (512, 1024),
                                  (1024, 2048)])
 def test_czt_lengths_and_tiles(M, N):
