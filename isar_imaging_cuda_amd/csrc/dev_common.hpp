@@ -58,19 +58,6 @@ __device__ __forceinline__ float2 expjpi_reduced(double t) {
     t -= 2.0 * rint(0.5 * t);
     return expjpi_twiddle(static_cast<float>(t));
 }
-// exp(j pi t) evaluated in FP64 and rounded once to FP32 (within half an ulp per component).
-__device__ __forceinline__ float2 expjpi_rounded(double t) {
-    double s, c;
-    sincospi(t, &s, &c);
-    return make_float2(static_cast<float>(c), static_cast<float>(s));
-}
-// exp(j pi t) for |t| small enough that FP32 holds it exactly (dyadic FFT twiddles).
-__device__ __forceinline__ float2 expjpi(float t) {
-    float s, c;
-    sincospif(t, &s, &c);
-    return make_float2(c, s);
-}
-
 // exp(j pi t) for t in [-2, 2] given exactly in FP32 (FFT twiddle arguments): octant reduction
 // t = q/4 + r, |r| <= 1/8, then Taylor polynomials of sin(pi r) (degree 9) and cos(pi r)
 // (degree 10), whose truncation errors (< 3e-11) are far below FP32 rounding, and a rotation by
@@ -155,6 +142,19 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     if (l == 0) red[w] = v;
     __syncthreads();
     float r = 0.f;
+#pragma unroll
+    for (int i = 0; i < NT / 64; ++i) r += red[i];
+    return r;
+}
+template <int NT>
+__device__ __forceinline__ long long block_sum_i64(long long v, long long* red) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    __syncthreads();
+    if (l == 0) red[w] = v;
+    __syncthreads();
+    long long r = 0;
 #pragma unroll
     for (int i = 0; i < NT / 64; ++i) r += red[i];
     return r;
@@ -349,25 +349,30 @@ __device__ __forceinline__ float2 group_sum2(float2 v) {
     return v;
 }
 
-// Inclusive prefix sum in FP64 of n values held as v[i] (i < n) in LDS, in place, by the
-// whole workgroup (NT threads). Each thread scans a contiguous segment sequentially.
+// Inclusive prefix sum in FP64 of n values held as v[i] (i < n) in LDS, in place, by the whole
+// workgroup (NT threads): every 64 consecutive values are scanned by a wave, then the sums of the
+// 64s before are added in their order, so that the result does not depend on NT. red: n / 64 slots.
+// (A serial pass over 1024 threads' partial sums took 11 us of a kernel's 16.)
 template <int NT>
 __device__ __forceinline__ void block_inclusive_scan_d(double* v, int n, double* red) {
-    const int tid = threadIdx.x;
-    const int seg = (n + NT - 1) / NT;
-    const int b = tid * seg, e = min(b + seg, n);
-    double run = 0.0;
-    for (int i = b; i < e; ++i) { run += v[i]; v[i] = run; }
-    __syncthreads();
-    red[tid] = run;
-    __syncthreads();
-    if (tid == 0) {
-        double acc = 0.0;
-        for (int i = 0; i < NT; ++i) { const double t = red[i]; red[i] = acc; acc += t; }
+    const int lane = threadIdx.x & 63;
+    for (int i0 = 0; i0 < n; i0 += NT) {   // every thread takes part in the shuffles
+        const int i = i0 + threadIdx.x;
+        double x = i < n ? v[i] : 0.0;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const double y = __shfl_up(x, o, 64);
+            x = lane >= o ? x + y : x;
+        }
+        if (i < n) v[i] = x;
+        if (lane == 63 && i - 63 < n) red[i >> 6] = x;
     }
     __syncthreads();
-    const double base = red[tid];
-    for (int i = b; i < e; ++i) v[i] += base;
+    for (int i = threadIdx.x; i < n; i += NT) {
+        double base = 0.0;
+        for (int k = 0; k < (i >> 6); ++k) base += red[k];
+        v[i] += base;
+    }
     __syncthreads();
 }
 

@@ -30,6 +30,7 @@
 
 struct float2 { float x, y; };
 struct float4 { float x, y, z, w; };
+struct alignas(16) uint4 { unsigned x, y, z, w; };
 struct double2 { double x, y; };
 struct int2 { int x, y; };
 inline float2 make_float2(float x, float y) { return float2{x, y}; }

@@ -112,38 +112,43 @@ __device__ void sort_arp(float* a, int n) {
 
 // Rows of arp_part / max_part holding partials, in summation order: row 0 (rows 0-1) and, at
 // every merge stride s >= 2, the chunks of min(s, ra_chunk) rows starting at s (the second group
-// of pair 0), stored at head row / 2. At most M/2 rows.
+// of pair 0), stored at head row / 2. At most M/2 rows. The NT threads fill them side by side (strides
+// and chunks are powers of two); every thread gets their number and a barrier follows.
+template <int NT>
 __device__ int arp_partial_rows(const Job& J, int* rows) {
-    int c = 0;
-    rows[c++] = 0;
-    for (int s = 2; s < J.M; s *= 2)
-        for (int h = s; h < min(2 * s, J.M); h += min(s, J.ra_chunk)) rows[c++] = h / 2;
+    int c = 1;
+    if (threadIdx.x == 0) rows[0] = 0;
+    for (int s = 2; s < J.M; s *= 2) {
+        const int R = min(s, J.ra_chunk), log_r = __builtin_ctz(R);
+        const int n = (min(s, J.M - s) + R - 1) >> log_r;
+        for (int i = threadIdx.x; i < n; i += NT) rows[c + i] = (s + (i << log_r)) / 2;
+        c += n;
+    }
+    __syncthreads();
     return c;
 }
 
 // Column sums of |S| over all M rows (the ARP numerator, range_alignment.cu:381-399) from the
 // partials range alignment wrote as rows finished moving, added in the order of their rows; one
-// thread per range cell, eight independent loads in flight. The sums go to the frame's first egrp
+// thread per range cell, sixteen independent loads in flight. The sums go to the frame's first egrp
 // row, free once range alignment has finished.
 __global__ __launch_bounds__(256) void k_arp(Job J) {
-    HIP_DYNAMIC_SHARED(int, rows);   // M/2 + 1
+    HIP_DYNAMIC_SHARED(int, rows);   // M/2
     const int f = blockIdx.y, n = blockIdx.x * 256 + threadIdx.x;
     const int M = J.M, N = J.N;
-    if (threadIdx.x == 0) rows[M / 2] = arp_partial_rows(J, rows);
-    __syncthreads();
+    const int P = arp_partial_rows<256>(J, rows);
     if (n >= N) return;
     const float* ap = J.arp_part + static_cast<size_t>(f) * (M / 2) * N + n;
-    const int P = rows[M / 2];
     float acc = 0.0f;
-    int i = 0;
-    for (; i + 8 <= P; i += 8) {
-        float v[8];
+    for (int i = 0; i < P; i += 16) {   // the last row again past the end, not used
+        float v[16];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) v[q] = ap[static_cast<size_t>(rows[i + q]) * N];
+        for (int q = 0; q < 16; ++q) v[q] = ap[static_cast<size_t>(rows[min(i + q, P - 1)]) * N];
+        issue_point();
 #pragma unroll
-        for (int q = 0; q < 8; ++q) acc += v[q];
+        for (int q = 0; q < 16; ++q)
+            if (i + q < P) acc += v[q];
     }
-    for (; i < P; ++i) acc += ap[static_cast<size_t>(rows[i]) * N];
     J.egrp[static_cast<size_t>(f) * M * N + n] = acc;
 }
 
@@ -157,17 +162,16 @@ __global__ __launch_bounds__(kCenterThreads) void k_center(Job J) {
     float* srt = sm + N;
     float* redv = srt + N;
     int* redi = reinterpret_cast<int*>(redv + 32);
-    int* rows = redi + 32;   // M/2 + 1
+    int* rows = redi + 32;   // M/2
     // max |S| arrives as partials per chunk of rows that finished moving (arp_partial_rows), the
     // column sums of |S| from k_arp
     const float* mp = J.max_part + static_cast<size_t>(f) * (M / 2);
     const float* colsum = J.egrp + static_cast<size_t>(f) * M * N;
-    if (tid == 0) rows[M / 2] = arp_partial_rows(J, rows);
-    __syncthreads();
+    const int partials = arp_partial_rows<NT>(J, rows);
 
     // H = |S| / max|S| ; ARP = column sums / M  (range_alignment.cu:381-399, all M rows)
     float gm = 0.0f;
-    for (int i = tid; i < rows[M / 2]; i += NT) gm = fmaxf(gm, mp[rows[i]]);
+    for (int i = tid; i < partials; i += NT) gm = fmaxf(gm, mp[rows[i]]);
     gm = block_max<NT>(gm, redv);
     const float inv = gm > 0.0f ? 1.0f / gm : 0.0f;
     const float invM = 1.0f / static_cast<float>(M);
@@ -218,12 +222,12 @@ __global__ __launch_bounds__(kCenterThreads) void k_center(Job J) {
             else keep_sum += n;
         }
     }
-    const int len1 = static_cast<int>(block_sum<NT>(static_cast<float>(c1), redv) + 0.5f);
-    const int len2 = static_cast<int>(block_sum<NT>(static_cast<float>(c2), redv) + 0.5f);
-    // the kept-index sum can exceed FP32 precision: reduce it as two exact halves
-    const float ks_hi = block_sum<NT>(static_cast<float>(keep_sum >> 12), redv);
-    const float ks_lo = block_sum<NT>(static_cast<float>(keep_sum & 4095), redv);
-    const long long ksum = (static_cast<long long>(ks_hi + 0.5f) << 12) + static_cast<long long>(ks_lo + 0.5f);
+    // both counts (at most 16384) and the sum of the kept indices (below 2^28) in one 64-bit sum; redv and
+    // redi, 32 words each, hold the waves' 16
+    long long sums = c1 | (static_cast<long long>(c2) << 16) | (keep_sum << 32);
+    sums = block_sum_i64<NT>(sums, reinterpret_cast<long long*>(redv));
+    const int len1 = static_cast<int>(sums & 0xffff), len2 = static_cast<int>((sums >> 16) & 0xffff);
+    const long long ksum = sums >> 32;
     int shift = 0, applied = 0;
     if (len2 != len1) {
         const int mean_idx = static_cast<int>(ksum / (len1 - len2));
@@ -260,9 +264,10 @@ __global__ __launch_bounds__(kCenterThreads) void k_center(Job J) {
 
 // Cut: X[m, j] = S[m, (off + j - shift) mod N] for a band of rows; column maxima of |X| per
 // band (fastEntropy :180-184) and the adjacent-pulse products sum_j conj(X[m,j]) X[m+1,j]
-// (dopplerTracking :12-20). Block = W threads, one per range bin of the window. Each wave's sum
-// of a row's products goes to LDS; one barrier after the band, then thread r adds row r's wave
-// sums in wave order.
+// (dopplerTracking :12-20). Block = W threads, one per range bin of the window. The band's rows and the
+// next are read together (a single frame's launch 9 us; 13 with a read waited for per row). Each
+// wave's sum of a row's products goes to LDS; one barrier after the band, then thread r adds row r's
+// wave sums in wave order.
 template <int W>
 __global__ __launch_bounds__(W) void k_cut(Job J) {
     HIP_DYNAMIC_SHARED(float2, wred);   // (W/64) x kCutBandRows wave sums
@@ -275,19 +280,18 @@ __global__ __launch_bounds__(W) void k_cut(Job J) {
     float2* xo = J.x + static_cast<size_t>(f) * M * W + j;
     const int m0 = band * kCutBandRows, m1 = min(m0 + kCutBandRows, M);
     float cmax = 0.0f;
-    float2 cur = src[static_cast<size_t>(m0) * N];
-    for (int m = m0; m < m1; ++m) {
-        xo[static_cast<size_t>(m) * W] = cur;
-        cmax = fmaxf(cmax, cabsf_(cur));
-        float2 prod = make_float2(0.0f, 0.0f);
-        float2 nxt = make_float2(0.0f, 0.0f);
-        if (m + 1 < M) {
-            nxt = src[static_cast<size_t>(m + 1) * N];
-            prod = cconjmul(cur, nxt);
-        }
-        const float2 sum = wave_sum2(prod);
-        if ((j & 63) == 0) wred[(j >> 6) * kCutBandRows + (m - m0)] = sum;
-        cur = nxt;
+    float2 v[kCutBandRows + 1];
+#pragma unroll
+    for (int r = 0; r <= kCutBandRows; ++r) v[r] = src[static_cast<size_t>(min(m0 + r, M - 1)) * N];
+    issue_point();
+#pragma unroll
+    for (int r = 0; r < kCutBandRows; ++r) {
+        const int m = m0 + r;
+        if (m >= m1) break;
+        xo[static_cast<size_t>(m) * W] = v[r];
+        cmax = fmaxf(cmax, cabsf_(v[r]));
+        const float2 sum = wave_sum2(m + 1 < M ? cconjmul(v[r], v[r + 1]) : make_float2(0.0f, 0.0f));
+        if ((j & 63) == 0) wred[(j >> 6) * kCutBandRows + r] = sum;
     }
     J.colmax_part[(static_cast<size_t>(f) * nbands + band) * W + j] = cmax;
     __syncthreads();
@@ -304,7 +308,7 @@ __global__ __launch_bounds__(W) void k_cut(Job J) {
 
 hipError_t configure_center_kernels() {
 #ifndef ISAR_EMU
-    const size_t bytes = (2 * 16384 + 64) * sizeof(float) + (1024 / 2 + 1) * sizeof(int);
+    const size_t bytes = (2 * 16384 + 64) * sizeof(float) + 1024 / 2 * sizeof(int);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_center), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        static_cast<int>(bytes));
     if (e != hipSuccess) report_config_error(__FILE__, bytes);
@@ -315,7 +319,7 @@ hipError_t configure_center_kernels() {
 }
 
 void launch_center(const Job& J, hipStream_t s) {
-    const size_t rows = (static_cast<size_t>(J.M) / 2 + 1) * sizeof(int);
+    const size_t rows = static_cast<size_t>(J.M) / 2 * sizeof(int);
     ISAR_LAUNCH(k_arp, dim3((J.N + 255) / 256, J.K), dim3(256), rows, s, J);
     const size_t lds = (2 * static_cast<size_t>(J.N) + 64) * sizeof(float) + rows;
     ISAR_LAUNCH(k_center, dim3(J.K), dim3(kCenterThreads), lds, s, J);

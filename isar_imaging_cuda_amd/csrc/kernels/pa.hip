@@ -24,55 +24,37 @@ __device__ void doppler_phase(const float2* r, int M, float2* phi, double* scrat
     __syncthreads();
 }
 
-// Ascending bitonic sort of NT (key, tag) pairs, one per thread, ties ordered by tag (stable for
-// unique tags), NaN keys last: stage (k, j) orders each pair i < i ^ j ascending where i & k == 0,
-// descending otherwise. The stages whose partner lies in the same wave (j < 64) exchange through
-// shuffles in registers; only those across waves go through LDS, with a barrier each (6 of the 45
-// stages at 512). key and tag are in LDS, filled before a barrier; every thread calls it.
-template <int NT>
-__device__ void bitonic_sort_kv(float* key, int* tag) {
-    static_assert(NT >= 64 && (NT & (NT - 1)) == 0, "one wave or more, a power of two");
-    const int t = threadIdx.x;
-    auto greater = [](float a, float b, int ta, int tb) { return (a > b) || (a == b && ta > tb) || (a != a && b == b); };
-    float kv = 0.0f;
-    int tv = 0;
-    bool in_regs = false;
-    for (int k = 2; k <= NT; k <<= 1) {
-        int j = k >> 1;
-        for (; j >= 64; j >>= 1) {   // partner in another wave
-            if (in_regs) {
-                key[t] = kv;
-                tag[t] = tv;
-                __syncthreads();
-                in_regs = false;
-            }
-            const int l = t ^ j;
-            if (l > t) {
-                const float a = key[t], b = key[l];
-                const int ta = tag[t], tb = tag[l];
-                if (greater(a, b, ta, tb) == ((t & k) == 0)) { key[t] = b; key[l] = a; tag[t] = tb; tag[l] = ta; }
-            }
-            __syncthreads();
+// A float's bits as an unsigned number in the order of the floats, both zeros alike and NaNs last.
+__device__ __forceinline__ unsigned order_key(float v) {
+    if (!(v == v)) return 0xffffffffu;
+    const unsigned b = __float_as_uint(v + 0.0f);
+    return b ^ ((b >> 31) ? 0xffffffffu : 0x80000000u);
+}
+
+// Rank of key[n] among key[0 ... count - 1] in LDS (ascending, equal keys by index), count at most W
+// and a multiple of 4: the keys before n's wave count where they are no larger, those after it
+// where they are smaller. All lanes of a wave read the same keys, four a load; a compare and an add
+// each, so 512 keys cost W waves' 1024 instructions, where a bitonic sort passes 45 barriers or
+// shuffles one after the other.
+template <int W>
+__device__ int rank_of(const unsigned* key, int count, int n) {
+    const unsigned own = key[n];
+    const int w0 = min(n & ~63, count), w1 = min(w0 + 64, count);
+    int rank = 0;
+    auto each = [&](int from, int to, auto before) {
+#pragma unroll 4
+        for (int k = from; k < to; k += 4) {
+            const uint4 q = *reinterpret_cast<const uint4*>(key + k);
+            rank += before(q.x, k) ? 1 : 0;
+            rank += before(q.y, k + 1) ? 1 : 0;
+            rank += before(q.z, k + 2) ? 1 : 0;
+            rank += before(q.w, k + 3) ? 1 : 0;
         }
-        if (!in_regs) {   // after the last LDS stage's barrier (or the caller's)
-            kv = key[t];
-            tv = tag[t];
-            in_regs = true;
-        }
-        for (; j >= 1; j >>= 1) {   // partner lane t ^ j of the same wave
-            const float pk = __shfl_xor(kv, j, 64);
-            const int pt = __shfl_xor(tv, j, 64);
-            const bool lower = (t & j) == 0;
-            const bool gt = lower ? greater(kv, pk, tv, pt) : greater(pk, kv, pt, tv);
-            if (gt == ((t & k) == 0)) {
-                kv = pk;
-                tv = pt;
-            }
-        }
-    }
-    key[t] = kv;   // the last stage (j = 1) left the pairs in registers
-    tag[t] = tv;
-    __syncthreads();
+    };
+    each(0, w0, [&](unsigned q, int) { return q <= own; });
+    each(w0, w1, [&](unsigned q, int k) { return q < own || (q == own && k < n); });
+    each(w1, count, [&](unsigned q, int) { return q < own; });
+    return rank;
 }
 
 }  // namespace
@@ -81,7 +63,7 @@ __device__ void bitonic_sort_kv(float* key, int* tag) {
 // adjacent-pulse products k_cut formed: once per frame, for every column tile of k_pa_colfft.
 template <int M>
 __global__ __launch_bounds__(256) void k_pa_doppler(Job J) {
-    HIP_DYNAMIC_SHARED(double, scr);   // M (scan) + 256 (scan partials)
+    HIP_DYNAMIC_SHARED(double, scr);   // M (scan) + 32 (its partial sums)
     const int f = blockIdx.x;
     doppler_phase<256>(J.rowdop + static_cast<size_t>(f) * M, M, J.dopphi + static_cast<size_t>(f) * M, scr,
                        scr + M);
@@ -145,18 +127,22 @@ __global__ __launch_bounds__(256) void k_pa_colfft(Job J) {
 // Bin selection (phase_adjustment.cu:186-264): int-truncated mean of the column maxima,
 // tgt_num bins above 1.48 * mean, the tgt_num most energetic (stable, descending), the
 // unit2_num = nextPow2(tgt_num / 2) of those with the lowest entropy (stable, ascending),
-// sorted by index. One workgroup of W threads per frame.
+// sorted by index. One workgroup of W threads per frame; the orders come from ranks (rank_of), the
+// final one from a prefix sum over the bins. 13 us for a single frame, with three bitonic sorts 27.
 template <int W>
 __global__ __launch_bounds__(W) void k_pa_select(Job J) {
-    HIP_DYNAMIC_SHARED(float, sm_sel);
-    float* key = sm_sel;                              // W
-    int* tag = reinterpret_cast<int*>(key + W);       // W
-    int* order1 = tag + W;                            // W
-    float* red = reinterpret_cast<float*>(order1 + W);   // 32
-    int* ired = reinterpret_cast<int*>(red + 32);        // 32
+    HIP_DYNAMIC_SHARED(uint4, sm_sel);
+    unsigned* key = reinterpret_cast<unsigned*>(sm_sel);   // W
+    int* order1 = reinterpret_cast<int*>(key + W);         // W
+    int* taken = order1 + W;                               // W
+    int* ired = taken + W;                                 // 32
     const int f = blockIdx.x, n = threadIdx.x;
     const float mx = J.colmax[static_cast<size_t>(f) * W + n];
     const float E = J.colE[static_cast<size_t>(f) * W + n];
+    const float H = J.colH[static_cast<size_t>(f) * W + n];
+    // energy descending, index ascending on ties, NaN last
+    key[n] = order_key((E == E) ? -E : __int_as_float(0x7f800000));
+    taken[n] = 0;
     // thrust::reduce(..., 0, plus<int>()) (phase_adjustment.cu:186) converts every maximum to int
     // as the device does (truncation, clamped) and adds them in 32-bit arithmetic, which wraps
     unsigned utot = 0;
@@ -170,27 +156,20 @@ __global__ __launch_bounds__(W) void k_pa_select(Job J) {
     int half = tgt / 2, U = 1;
     while (half >> 1) { U <<= 1; half >>= 1; }
     U <<= 1;   // nextPow2 (common.cu:521-529)
-    // sort 1: energy descending, index ascending on ties
-    key[n] = (E == E) ? -E : __int_as_float(0x7f800000);
-    tag[n] = n;
+    const int rank1 = rank_of<W>(key, W, n);
     __syncthreads();
-    bitonic_sort_kv<W>(key, tag);
-    order1[n] = tag[n];
+    // entropy ascending among the first tgt, rank ascending on ties
+    key[rank1] = rank1 < tgt ? order_key(H) : 0xffffffffu;
+    order1[rank1] = n;
     __syncthreads();
-    // sort 2: entropy ascending among the first tgt, rank ascending on ties
-    key[n] = n < tgt ? J.colH[static_cast<size_t>(f) * W + order1[n]] : __int_as_float(0x7f800000);
-    tag[n] = n < tgt ? n : W + n;
+    // the first U of them
+    if (n < tgt && rank_of<W>(key, (tgt + 3) & ~3, n) < U) taken[order1[n]] = 1;
     __syncthreads();
-    bitonic_sort_kv<W>(key, tag);
-    // first U of them (bin 0 fills positions beyond tgt, as std::vector growth does)
-    int bin = 0x7fffffff;
-    if (n < U) bin = (n < tgt) ? order1[tag[n]] : 0;
-    __syncthreads();
-    key[n] = static_cast<float>(bin == 0x7fffffff ? 1 << 30 : bin);
-    tag[n] = bin;
-    __syncthreads();
-    bitonic_sort_kv<W>(key, tag);
-    if (n < U) J.sel[static_cast<size_t>(f) * W + n] = tag[n];
+    // bin 0 fills positions beyond tgt, as std::vector growth does
+    const int times = taken[n] + (n == 0 ? max(U - tgt, 0) : 0);
+    int all = 0;
+    const int at = block_exclusive_scan<W>(times, ired, &all);
+    for (int i = 0; i < times; ++i) J.sel[static_cast<size_t>(f) * W + at + i] = n;
     if (n == 0) {
         J.dec[f].tgt_num = tgt;
         J.dec[f].unit2_num = U;
@@ -233,9 +212,7 @@ __device__ __forceinline__ int af_scale_exponent(float cm) {
     return cm > 0.0f && cm <= 3.40282347e38f ? ilogbf(cm) : 0;
 }
 
-// PRE = true: the selected bins are in su and their Doppler products in rowdop already
-// (k_af_gather, k_af_bin_doppler), and only the start phase is formed (no iterations).
-template <int M, bool PRE = false>
+template <int M>
 __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
     using A = AfCfg<M>;
     using C = ColCfg<M>;
@@ -253,44 +230,39 @@ __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
     float2* su = J.su + static_cast<size_t>(f) * W * M;
     const float2* X = J.x + static_cast<size_t>(f) * M * W;
     if (J.af_redo && (J.dec[f].status & 2) == 0) return;   // the whole workgroup
-    if (PRE && tid == 0) J.af_sync[f] = 0;   // the resident form's hand-off counter
 
     // gather the selected bins, column-major (selectRangeBins, :335-346), scaled by 2^-e so that
     // the largest selected |S| lies in [1, 2): the update takes the unit phasor of sums cubic in
     // S, and a power of two scales every product exactly, so the phases are those of the unscaled
     // bins while conj(S) IFFT(G |G|) stays far from FP32 overflow at any input level
-    if constexpr (!PRE) {
-        float cm = 0.0f;
-        for (int u = tid; u < U; u += NT) cm = fmaxf(cm, J.colmax[static_cast<size_t>(f) * W + sel[u]]);
-        cm = block_max<NT>(cm, reinterpret_cast<float*>(red));
-        const int e = af_scale_exponent(cm);
-        {   // the selected bins' indices in LDS (the transform buffers are free here), then the
-            // gather with eight loads in flight per thread
-            int* lsel = reinterpret_cast<int*>(bufs);
-            for (int u = tid; u < U; u += NT) lsel[u] = sel[u];
-            __syncthreads();
-            for (int idx0 = tid; idx0 < U * M; idx0 += 8 * NT) {
-                float2 v[8];
+    float cm = 0.0f;
+    for (int u = tid; u < U; u += NT) cm = fmaxf(cm, J.colmax[static_cast<size_t>(f) * W + sel[u]]);
+    cm = block_max<NT>(cm, reinterpret_cast<float*>(red));
+    const int e = af_scale_exponent(cm);
+    {   // the selected bins' indices in LDS (the transform buffers are free here), then the
+        // gather with eight loads in flight per thread
+        int* lsel = reinterpret_cast<int*>(bufs);
+        for (int u = tid; u < U; u += NT) lsel[u] = sel[u];
+        __syncthreads();
+        for (int idx0 = tid; idx0 < U * M; idx0 += 8 * NT) {
+            float2 v[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int idx = idx0 + i * NT;
-                    if (idx < U * M) v[i] = X[static_cast<size_t>(idx / U) * W + lsel[idx % U]];
-                }
+            for (int i = 0; i < 8; ++i) {
+                const int idx = idx0 + i * NT;
+                if (idx < U * M) v[i] = X[static_cast<size_t>(idx / U) * W + lsel[idx % U]];
+            }
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int idx = idx0 + i * NT;
-                    if (idx < U * M)
-                        su[static_cast<size_t>(idx % U) * M + idx / U] = make_float2(ldexpf(v[i].x, -e), ldexpf(v[i].y, -e));
-                }
+            for (int i = 0; i < 8; ++i) {
+                const int idx = idx0 + i * NT;
+                if (idx < U * M)
+                    su[static_cast<size_t>(idx % U) * M + idx / U] = make_float2(ldexpf(v[i].x, -e), ldexpf(v[i].y, -e));
             }
         }
-        __syncthreads();
     }
+    __syncthreads();
     if (J.phi0_given) {
         for (int m = tid; m < M; m += NT) phi[m] = J.phi0_in[static_cast<size_t>(f) * M + m];
         __syncthreads();
-    } else if constexpr (PRE) {
-        doppler_phase<NT>(J.rowdop + static_cast<size_t>(f) * M, M, phi, scr, red);
     } else {
         // Doppler tracking of the selected bins without compensation (:282), the products added
         // in bin order with eight bins' loads in flight
@@ -315,10 +287,6 @@ __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
         doppler_phase<NT>(rdop, M, phi, scr, red);
     }
     for (int m = tid; m < M; m += NT) J.phi0[static_cast<size_t>(f) * M + m] = phi[m];
-    if constexpr (PRE) {
-        for (int m = tid; m < M; m += NT) J.phi[static_cast<size_t>(f) * M + m] = phi[m];
-        return;
-    }
 
     const int g = tid / TPF, lane = tid % TPF;
     float2* buf = bufs + g * lds_padded_size(M);
@@ -403,8 +371,8 @@ __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
 // workgroups per frame each taking a contiguous share of the (pulse, bin) elements; then
 // k_af_bin_doppler forms each pulse's Doppler product of the selected bins (:282) with the
 // products added in bin order as k_autofocus adds them, into rowdop, which is free once the bins
-// are selected; k_autofocus<M, true> then forms the start phase from it. For the resident form
-// k_af_gather also clears the frame's exchange words.
+// are selected; k_af_start then forms the start phase from it. For the resident form
+// k_af_gather also clears the frame's exchange words, k_af_start its hand-off counter.
 constexpr int kAfGatherGroups = 32;
 
 // The resident form's exchange: up to 512 pulses in tagged words, above through a counter.
@@ -484,9 +452,27 @@ __global__ __launch_bounds__(256) void k_af_bin_doppler(Job J) {
     J.rowdop[static_cast<size_t>(f) * M + m] = acc;
 }
 
+template <int M>
+__global__ __launch_bounds__(256) void k_af_start(Job J) {
+    HIP_DYNAMIC_SHARED(double, scr);   // M (scan) + 32 (its partial sums), the phase (M float2)
+    const int f = blockIdx.x, tid = threadIdx.x;
+    float2* phi = reinterpret_cast<float2*>(scr + M + 32);
+    if (tid == 0) J.af_sync[f] = 0;
+    if (J.phi0_given) {
+        for (int m = tid; m < M; m += 256) phi[m] = J.phi0_in[static_cast<size_t>(f) * M + m];
+        __syncthreads();
+    } else {
+        doppler_phase<256>(J.rowdop + static_cast<size_t>(f) * M, M, phi, scr, scr + M);
+    }
+    for (int m = tid; m < M; m += 256) {
+        J.phi0[static_cast<size_t>(f) * M + m] = phi[m];
+        J.phi[static_cast<size_t>(f) * M + m] = phi[m];
+    }
+}
+
 // The same fixed-point update with a frame spread over several workgroups, for batches too small
-// to fill the GPU with one workgroup per frame. k_autofocus with no iterations gathers the
-// selected bins and forms the starting phase; then iteration `it` is a launch of k_af_cols:
+// to fill the GPU with one workgroup per frame. The start kernels gather the selected bins and form
+// the starting phase; then iteration `it` is a launch of k_af_cols:
 // workgroup (j, f) takes the frame's current phase, transforms sub-chunk j of the selected bins
 // and writes its per-pulse sums of conj(S) IFFT(G |G|) (/ M unless M is a power of two, af_term)
 // into the iteration's half of af_part.
@@ -774,7 +760,7 @@ size_t autofocus_lds() {
     using A = AfCfg<M>;
     return 2 * M * sizeof(float2) + (M + A::NT) * sizeof(double) + static_cast<size_t>(A::CF) * lds_padded_size(M) * sizeof(float2);
 }
-size_t select_lds(int W) { return 3 * W * sizeof(int) + 64 * sizeof(float); }
+size_t select_lds(int W) { return (3 * W + 32) * sizeof(int); }
 }  // namespace
 
 #define ISAR_PULSE_SWITCH(M, BODY)                       \
@@ -806,7 +792,6 @@ hipError_t configure_pa_kernels() {
 #define ISAR_SET_PA(MM)                                                          \
     set(reinterpret_cast<const void*>(&k_pa_colfft<MM>), colfft_lds<MM>());      \
     set(reinterpret_cast<const void*>(&k_autofocus<MM>), autofocus_lds<MM>());   \
-    set(reinterpret_cast<const void*>(&k_autofocus<MM, true>), autofocus_lds<MM>());   \
     set(reinterpret_cast<const void*>(&k_af_cols<MM, true>), af_cols_lds<MM>(true));   \
     set(reinterpret_cast<const void*>(&k_af_cols<MM, false>), af_cols_lds<MM>(false));   \
     set(reinterpret_cast<const void*>(&k_af_resident<MM>), af_resident_lds<MM>(1));
@@ -818,7 +803,7 @@ hipError_t configure_pa_kernels() {
 }
 
 void launch_pa_colfft(const Job& J, hipStream_t s) {
-    ISAR_PULSE_SWITCH(J.M, ISAR_LAUNCH(k_pa_doppler<MM>, dim3(J.K), dim3(256), (MM + 256) * sizeof(double), s, J));
+    ISAR_PULSE_SWITCH(J.M, ISAR_LAUNCH(k_pa_doppler<MM>, dim3(J.K), dim3(256), (MM + 32) * sizeof(double), s, J));
     ISAR_PULSE_SWITCH(J.M, ISAR_LAUNCH(k_pa_colfft<MM>, dim3(J.W / ColCfg<MM>::CT, J.K), dim3(ColCfg<MM>::NT),
                                        colfft_lds<MM>(), s, J));
 }
@@ -830,15 +815,13 @@ void launch_autofocus(const Job& J, hipStream_t s) {
 }
 namespace {
 // The start phase and the gathered bins of the split and resident forms (k_af_gather,
-// k_af_bin_doppler, k_autofocus<MM, true>).
+// k_af_bin_doppler, k_af_start).
 template <int MM>
 void autofocus_start_spread(const Job& J, bool resident, hipStream_t s) {
     ISAR_LAUNCH(k_af_gather<MM>, dim3(kAfGatherGroups, J.K), dim3(256), J.W * sizeof(int) + 32 * sizeof(float), s, J,
                 resident ? 1 : 0);
     if (!J.phi0_given) ISAR_LAUNCH(k_af_bin_doppler<MM>, dim3((MM - 1 + 255) / 256, J.K), dim3(256), 0, s, J);
-    Job J0 = J;
-    J0.iterations = 0;
-    ISAR_LAUNCH((k_autofocus<MM, true>), dim3(J.K), dim3(AfCfg<MM>::NT), autofocus_lds<MM>(), s, J0);
+    ISAR_LAUNCH(k_af_start<MM>, dim3(J.K), dim3(256), (MM + 32) * sizeof(double) + MM * sizeof(float2), s, J);
 }
 
 template <int MM>
