@@ -414,17 +414,21 @@ __device__ __forceinline__ void load_column_tile(const float2* src, int W, int n
 // Hand-off between the workgroups of one launch (the resident autofocus). Values pass through
 // memory as 64-bit words stored and loaded as agent-scope relaxed atomics: global accesses with
 // sc1 set, which are written through to the device's point of coherence and read from it, never
-// from a stale line of another XCD's L2. Either a word carries a 32-bit value and a 32-bit tag,
-// and a reader polls it until the tag is the one it expects, so value and tag arrive together;
-// or each writer waits for its stores to be acknowledged (s_waitcnt 0) before its workgroup
-// counts itself in on a counter, and readers poll the counter. Neither involves a fence, an L2
-// write-back or an invalidation.
+// from a stale line of another XCD's L2. A word is empty until its value is stored, and a reader
+// polls it until it is not, so nothing but the value itself has to arrive; a word that is used again
+// is emptied first, and that store waited for (s_waitcnt 0). No fence, L2 write-back or invalidation is involved.
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ uint64_t xwg_word(float v, unsigned tag) {
-    return (static_cast<uint64_t>(tag) << 32) | static_cast<uint64_t>(__float_as_uint(v));
+constexpr uint64_t kXwgEmpty = ~0ull;   // two NaNs
+__device__ __forceinline__ uint64_t xwg_word(float2 v) {
+    uint64_t w;
+    __builtin_memcpy(&w, &v, sizeof w);
+    return w == kXwgEmpty ? w - 1 : w;   // NaNs as well
 }
-__device__ __forceinline__ unsigned xwg_tag(uint64_t w) { return static_cast<unsigned>(w >> 32); }
-__device__ __forceinline__ float xwg_value(uint64_t w) { return __uint_as_float(static_cast<unsigned>(w)); }
+__device__ __forceinline__ float2 xwg_value(uint64_t w) {
+    float2 v;
+    __builtin_memcpy(&v, &w, sizeof v);
+    return v;
+}
 __device__ __forceinline__ void xwg_store(uint64_t* p, uint64_t w) {
 #ifdef ISAR_EMU
     __atomic_store_n(p, w, __ATOMIC_RELAXED);
@@ -444,14 +448,9 @@ __device__ __forceinline__ void xwg_stores_done() {
 #ifdef ISAR_EMU
     __atomic_thread_fence(__ATOMIC_SEQ_CST);
 #else
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0);
-#endif
-}
-__device__ __forceinline__ void xwg_arrive(unsigned* c) {
-#ifdef ISAR_EMU
-    __atomic_fetch_add(c, 1u, __ATOMIC_SEQ_CST);
-#else
-    __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::: "memory");
 #endif
 }
 __device__ __forceinline__ void xwg_pause() {
@@ -460,20 +459,6 @@ __device__ __forceinline__ void xwg_pause() {
 #else
     __builtin_amdgcn_s_sleep(2);
 #endif
-}
-// Polls *c until it reaches target; false when `limit` polls pass first, and at once when limit
-// is negative.
-__device__ __forceinline__ bool xwg_wait(const unsigned* c, unsigned target, int limit) {
-    if (limit < 0) return false;
-    for (int n = 0;; ++n) {
-#ifdef ISAR_EMU
-        if (__atomic_load_n(c, __ATOMIC_SEQ_CST) >= target) return true;
-#else
-        if (__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= target) return true;
-#endif
-        if (n >= limit) return false;
-        xwg_pause();
-    }
 }
 
 }  // namespace isar

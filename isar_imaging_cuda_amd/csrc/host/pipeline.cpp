@@ -118,7 +118,6 @@ size_t carve_workspace(const isar_radar_params& p, int K_, char* base, Job* J, S
     j.colsum = static_cast<float2*>(frame(W * sizeof(float2)));
     j.delta = static_cast<float2*>(frame(W * sizeof(float2)));
     j.af_part = static_cast<float2*>(frame(4 * (W / 8) * M * sizeof(float2)));   // split: half; resident: all
-    j.af_sync = static_cast<unsigned*>(frame(sizeof(unsigned)));
     SharedTables t{};
     t.czt_table = static_cast<float2*>(shared(W * F * sizeof(float2)));
     t.czt_pre = static_cast<float2*>(shared(W * M * sizeof(float2)));

@@ -372,21 +372,17 @@ __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
 // k_af_bin_doppler forms each pulse's Doppler product of the selected bins (:282) with the
 // products added in bin order as k_autofocus adds them, into rowdop, which is free once the bins
 // are selected; k_af_start then forms the start phase from it. For the resident form
-// k_af_gather also clears the frame's exchange words, k_af_start its hand-off counter.
+// k_af_gather also empties the frame's exchange words.
 constexpr int kAfGatherGroups = 32;
 
-// The resident form's exchange: up to 512 pulses in tagged words, above through a counter.
-template <int M>
-constexpr bool kAfTagged = M <= 512;
-
-// The exchange words of frame f in the resident form: per iteration parity, sub-chunk q < W/SUB
-// and pulse m, the real and the imaginary part of the sub-chunk's per-pulse sum as tagged words
-// (xwg_word). Frame f owns 4 (W/8) M words of af_part, the buffer being sized for it.
+// The exchange words of frame f in the resident form (xwg_word): for iterations 0, 1, 2 modulo 3,
+// sub-chunk q < W/SUB and pulse m, the sub-chunk's per-pulse sum. Frame f owns 4 (W/8) M words of
+// af_part, the buffer being sized for it.
 template <int M>
 __device__ __forceinline__ uint64_t* af_words_of(const Job& J, int f, int it) {
     const size_t nq = static_cast<size_t>(J.W / AfCfg<M>::SUB);
     uint64_t* frame = reinterpret_cast<uint64_t*>(J.af_part) + static_cast<size_t>(f) * 4 * (J.W / 8) * M;
-    return frame + static_cast<size_t>(it & 1) * nq * M * 2;
+    return frame + static_cast<size_t>(it % 3) * nq * M;
 }
 
 template <int M>
@@ -403,12 +399,10 @@ __global__ __launch_bounds__(256) void k_af_gather(Job J, int resident) {
     const int e = af_scale_exponent(cm);
     for (int u = tid; u < U; u += 256) lsel[u] = sel[u];
     __syncthreads();
-    if (kAfTagged<M> && resident) {   // the words of the ceil(U / SUB) sub-chunks of both parities
-        const int words = (U + AfCfg<M>::SUB - 1) / AfCfg<M>::SUB * M * 2;
-        for (int i = blockIdx.x * 256 + tid; i < words; i += gridDim.x * 256) {
-            xwg_store(af_words_of<M>(J, f, 0) + i, 0);
-            xwg_store(af_words_of<M>(J, f, 1) + i, 0);
-        }
+    if (resident) {   // the words of the ceil(U / SUB) sub-chunks
+        const int words = (U + AfCfg<M>::SUB - 1) / AfCfg<M>::SUB * M;
+        for (int i = blockIdx.x * 256 + tid; i < words; i += gridDim.x * 256)
+            for (int it = 0; it < 3; ++it) xwg_store(af_words_of<M>(J, f, it) + i, kXwgEmpty);
     }
     const float2* X = J.x + static_cast<size_t>(f) * M * W;
     float2* su = J.su + static_cast<size_t>(f) * W * M;
@@ -457,7 +451,6 @@ __global__ __launch_bounds__(256) void k_af_start(Job J) {
     HIP_DYNAMIC_SHARED(double, scr);   // M (scan) + 32 (its partial sums), the phase (M float2)
     const int f = blockIdx.x, tid = threadIdx.x;
     float2* phi = reinterpret_cast<float2*>(scr + M + 32);
-    if (tid == 0) J.af_sync[f] = 0;
     if (J.phi0_given) {
         for (int m = tid; m < M; m += 256) phi[m] = J.phi0_in[static_cast<size_t>(f) * M + m];
         __syncthreads();
@@ -480,26 +473,21 @@ __global__ __launch_bounds__(256) void k_af_start(Job J) {
 // (FOLD: one launch per iteration) or read from J.phi, which k_af_phase writes after each
 // iteration (two launches per iteration, no repeated work). The transforms and the summation
 // order are those of k_autofocus, so the phases agree bit for bit.
-// Unit phasor of pulse m's sum over the nsub sub-chunk sums part[q M + m], added in order;
-// load(p) reads one sum.
-template <int M, typename Load>
-__device__ __forceinline__ float2 af_phase_from(const float2* part, int nsub, int m, Load load) {
+// Unit phasor of pulse m's sum over the nsub sub-chunk sums part[q M + m], added in order.
+template <int M>
+__device__ __forceinline__ float2 af_phase_from(const float2* part, int nsub, int m) {
     float2 acc = make_float2(0.0f, 0.0f);
     for (int q = 0; q < nsub; q += 8) {   // up to eight loads in flight, added in order
         float2 v[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-            if (q + i < nsub) v[i] = load(part + static_cast<size_t>(q + i) * M + m);
+            if (q + i < nsub) v[i] = part[static_cast<size_t>(q + i) * M + m];
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             if (q + i < nsub) acc = cadd(acc, v[i]);
     }
     const float a = cabsf_(acc);
     return a > 0.0f ? cscale(acc, 1.0f / a) : make_float2(0.0f, 0.0f);
-}
-template <int M>
-__device__ __forceinline__ float2 af_phase_from(const float2* part, int nsub, int m) {
-    return af_phase_from<M>(part, nsub, m, [](const float2* p) { return *p; });
 }
 
 // the half of af_part that iteration `it` writes; frame f's sub-chunk sums in it
@@ -593,42 +581,48 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_cols(Job J
     af_subchunk<M>(s, phi, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) { part[m] = t; });
 }
 
-// af_phase_from over tagged words (af_words_of): pulse m's sub-chunk sums are loaded eight at a
-// time, each word polled until it carries `tag`, and added in sub-chunk order, so the phase is
-// af_phase_from's bit for bit. A thread that has polled more than `limit` times gives up for the
-// rest of the launch (waiting = false) and sets status bit 2.
-template <int M>
-__device__ __forceinline__ float2 af_phase_tagged(const uint64_t* words, int nsub, int m, unsigned tag, int limit,
-                                                  bool& waiting, int32_t& status) {
-    float2 acc = make_float2(0.0f, 0.0f);
-    int polls = 0;
-    for (int q0 = 0; q0 < nsub; q0 += 8) {
-        uint64_t re[8], im[8];
+// Adds n sub-chunk sums of pulse m to acc in order, from exchange words M apart. They are loaded
+// together, and all again until none is empty. A thread that has polled more than `limit` times in a row gives
+// up for the rest of the launch (waiting = false) and sets status bit 2.
+template <int M, int n>
+__device__ __forceinline__ void af_add_words(float2& acc, const uint64_t* w, int limit, bool& waiting, int32_t& status) {
+    uint64_t v[n];
+    for (int polls = 0;; ++polls) {
+        bool all = true;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            if (q0 + i < nsub) {
-                const uint64_t* w = words + (static_cast<size_t>(q0 + i) * M + m) * 2;
-                re[i] = xwg_load(w);
-                im[i] = xwg_load(w + 1);
-            }
-        }
+        for (int i = 0; i < n; ++i) v[i] = xwg_load(w + i * M);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            if (q0 + i >= nsub) break;
-            const uint64_t* w = words + (static_cast<size_t>(q0 + i) * M + m) * 2;
-            while (waiting && (xwg_tag(re[i]) != tag || xwg_tag(im[i]) != tag)) {
-                if (polls++ >= limit) {
-                    waiting = false;
-                    atomicOr(&status, 2);
-                    break;
-                }
-                xwg_pause();
-                re[i] = xwg_load(w);
-                im[i] = xwg_load(w + 1);
-            }
-            acc = cadd(acc, make_float2(xwg_value(re[i]), xwg_value(im[i])));
+        for (int i = 0; i < n; ++i) all = all && v[i] != kXwgEmpty;
+        if (all || !waiting) break;
+        if (polls >= limit) {
+            waiting = false;
+            atomicOr(&status, 2);
+            break;
         }
+        xwg_pause();
     }
+#pragma unroll
+    for (int i = 0; i < n; ++i) acc = cadd(acc, xwg_value(v[i]));
+}
+
+// af_phase_from over exchange words, bit for bit. nsub is a power of two, or 1 (the selected bins are
+// a power of two of them).
+template <int M>
+__device__ __forceinline__ float2 af_phase_from_words(const uint64_t* words, int nsub, int m, int limit, bool& waiting,
+                                                      int32_t& status) {
+    float2 acc = make_float2(0.0f, 0.0f);
+    const uint64_t* w = words + m;
+    int q = 0;
+    // the other workgroups' sums come about now: a first round that is too early costs its whole latency
+    // (with several workgroups on a CU 3 to 8 percent of an iteration)
+    xwg_pause();
+    xwg_pause();
+    for (; q + 4 <= nsub; q += 4) af_add_words<M, 4>(acc, w + static_cast<size_t>(q) * M, limit, waiting, status);
+    if (q + 2 <= nsub) {
+        af_add_words<M, 2>(acc, w + static_cast<size_t>(q) * M, limit, waiting, status);
+        q += 2;
+    }
+    if (q < nsub) af_add_words<M, 1>(acc, w + static_cast<size_t>(q) * M, limit, waiting, status);
     const float a = cabsf_(acc);
     return a > 0.0f ? cscale(acc, 1.0f / a) : make_float2(0.0f, 0.0f);
 }
@@ -637,15 +631,14 @@ __device__ __forceinline__ float2 af_phase_tagged(const uint64_t* words, int nsu
 // j of frame f's selected bins in registers for every iteration and hands its per-pulse sums to
 // the frame's other workgroups; every workgroup then forms the next phase from all nsub sums, in
 // sub-chunk order. The transforms, sums and phases are those of k_af_cols bit for bit.
-// Up to 512 pulses the sums travel as tagged words: each word is polled until it carries
-// iteration it's tag it + 1; k_af_gather has cleared the words, so those of an earlier run, or
-// whatever the memory held, never pass. At 1024 pulses, where a frame has more sub-chunks and
-// tagged words would double the bytes every workgroup reads per iteration, the sums travel as
-// plain 64-bit words: each thread waits for its stores to be acknowledged, the workgroup counts
-// itself in on the frame's counter (cleared by k_autofocus), and thread 0 polls the counter until
-// all nsub workgroups have counted in for the iteration.
-// Either way a workgroup writes iteration it + 2 into the words of iteration it only after it has
-// read every workgroup's iteration it + 1, which each wrote after reading iteration it.
+// The sums travel as 64-bit words that are empty (kXwgEmpty) until they are written, in three buffers
+// by iteration modulo 3, all empty at the start (k_af_gather). The thread of pulse m, having read all
+// of iteration it, empties its workgroup's word of iteration it - 1, which it + 2 takes next:
+// - every reader is done with it: a workgroup writes iteration it only after its barrier behind all
+//   reads of it - 1;
+// - every reader of it + 2 finds it emptied: it reads there only after this thread's word of it + 1,
+//   before whose store the thread has waited for the emptying to be acknowledged (a transform
+//   later, so that wait costs nothing).
 // All of a frame's workgroups must be resident together; every XCD takes its share of a grid's
 // workgroups in order, so where the first incomplete frame lacks one, only complete frames are
 // ahead of it, and it completes as those finish. A wait that exceeds J.af_wait_polls polls (about a
@@ -653,9 +646,10 @@ __device__ __forceinline__ float2 af_phase_tagged(const uint64_t* words, int nsu
 // that thread waiting; the frame's phase is then not valid, and the default form does the frame
 // over with k_autofocus. Workgroup 0 of each frame writes the final phase to J.phi.
 // Bound by the latency of an iteration (two transforms by one wave per SIMD, the sums, the
-// exchange): 5.5 us at 256 pulses, 7.6 at 512, whether the frames are 1 or 40, as long as every
-// workgroup has a CU for itself and the XCDs share the work (af_subchunk_of; before, 32 frames
-// took 11.3 and 31 us an iteration).
+// exchange): 3.6 us at 256 pulses, 6.1 at 512, whether the frames are 1 or 40, as long as every
+// workgroup has a CU for itself and the XCDs share the work (af_subchunk_of). At 256 pulses the
+// transforms and products take 5500 cycles, the sums 700 and the exchange, which the number of load
+// instructions decides, 1700; with a tag in every word, so twice as many loads, 2500.
 template <int M>
 __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(Job J) {
     using A = AfCfg<M>;
@@ -679,43 +673,18 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(J
     for (int e = 0; e < E; ++e) s[e] = valid ? col[C::in(lane, e)] : make_float2(0.0f, 0.0f);
     for (int m = tid; m < M; m += NTS) phi[m] = J.phi[static_cast<size_t>(f) * M + m];
     __syncthreads();
-    unsigned* const count = J.af_sync + f;
     bool waiting = J.af_wait_polls >= 0;   // false once this thread's polls have hit their bound
     if (!waiting && tid == 0) atomicOr(&J.dec[f].status, 2);   // a negative bound: every wait gives up
     for (int it = 0; it < J.iterations; ++it) {
-        uint64_t* words = af_words_of<M>(J, f, it);
-        if constexpr (kAfTagged<M>) {
-            const unsigned tag = static_cast<unsigned>(it) + 1;
-            af_subchunk<M>(s, phi, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) {
-                uint64_t* w = words + (static_cast<size_t>(j) * M + m) * 2;
-                xwg_store(w, xwg_word(t.x, tag));
-                xwg_store(w + 1, xwg_word(t.y, tag));
-            });
-            for (int m = tid; m < M; m += NTS)
-                phi[m] = af_phase_tagged<M>(words, nsub, m, tag, J.af_wait_polls, waiting, J.dec[f].status);
-        } else {
-            af_subchunk<M>(s, phi, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) {
-                uint64_t v;
-                __builtin_memcpy(&v, &t, sizeof v);
-                xwg_store(words + static_cast<size_t>(j) * M + m, v);
-            });
-            xwg_stores_done();
-            __syncthreads();
-            if (tid == 0) {
-                xwg_arrive(count);
-                if (waiting && !xwg_wait(count, static_cast<unsigned>(it + 1) * static_cast<unsigned>(nsub), J.af_wait_polls)) {
-                    waiting = false;
-                    atomicOr(&J.dec[f].status, 2);
-                }
-            }
-            __syncthreads();
-            for (int m = tid; m < M; m += NTS)
-                phi[m] = af_phase_from<M>(reinterpret_cast<const float2*>(words), nsub, m, [](const float2* p) {
-                    const uint64_t v = xwg_load(reinterpret_cast<const uint64_t*>(p));
-                    float2 t;
-                    __builtin_memcpy(&t, &v, sizeof t);
-                    return t;
-                });
+        uint64_t* const words = af_words_of<M>(J, f, it);
+        uint64_t* const old = af_words_of<M>(J, f, it + 2) + static_cast<size_t>(j) * M;   // iteration it - 1
+        af_subchunk<M>(s, phi, min(SUB, U - c0), bufs, tid, tw, [&](int m, float2 t) {
+            if (m == tid) xwg_stores_done();   // the words emptied an iteration ago
+            xwg_store(words + static_cast<size_t>(j) * M + m, xwg_word(t));
+        });
+        for (int m = tid; m < M; m += NTS) {
+            phi[m] = af_phase_from_words<M>(words, nsub, m, J.af_wait_polls, waiting, J.dec[f].status);
+            xwg_store(old + m, kXwgEmpty);
         }
         __syncthreads();
     }
@@ -738,16 +707,17 @@ template <int M>
 size_t af_cols_lds(bool fold) {
     return (static_cast<size_t>(AfCfg<M>::SUB) * lds_padded_size(M) + (fold ? M : 0)) * sizeof(float2);
 }
-// LDS of a resident workgroup. The dispatcher puts two or more workgroups on a CU that has the LDS
-// for them while other CUs are idle, which then run an iteration in 7.4 instead of 5.6 us (32 frames
-// of 256 pulses); more than half of the CU's LDS keeps them apart. That holds back workgroups once
-// they outnumber the CUs: a frame commonly selects up to 64 bins, and with that the line lies at
-// three quarters of the CUs (of 256 pulses 40 frames take 0.57 instead of 0.75 ms, 64 frames 1.13
-// instead of 0.79).
+// LDS of a resident workgroup. The dispatcher fills a CU that has the LDS for another workgroup while
+// other CUs are idle, and the fullest CU sets the pace of every iteration. So a workgroup asks for
+// so much LDS that a CU takes only its share of them, with a quarter of the places to spare; a
+// frame commonly selects up to 64 bins, more only run in more rounds. Of 256 pulses 40 frames take 0.51 ms
+// with the share, 0.78 with the LDS needed, 64 frames 0.57 and 0.81, 128 frames 0.76 and 0.86; of
+// 512 pulses 40 frames 0.74 and 1.10.
 template <int M>
 size_t af_resident_lds(int frames) {
-    const size_t need = af_cols_lds<M>(true);
-    return frames * (64 / AfCfg<M>::SUB) <= 3 * kComputeUnits / 4 ? std::max(need, kLdsBytes / 2 + 1024) : need;
+    const int groups = frames * (64 / AfCfg<M>::SUB);
+    const size_t per_cu = (4 * groups + 3 * kComputeUnits - 1) / (3 * kComputeUnits);
+    return std::max(af_cols_lds<M>(true), kLdsBytes / (per_cu + 1) + 1024);
 }
 template <int M>
 size_t colfft_lds() {

@@ -24,9 +24,9 @@ constexpr int kRaChunkRowsDefault = 8;   // rows per workgroup in the alignment 
 constexpr int kCutBandRows = 16;      // rows per workgroup when cutting the range window
 // Default autofocus form by batch size: several resident workgroups per frame up to this many frames,
 // one workgroup per frame above. The latter takes a CU per frame and leaves the others idle: at 64
-// selected bins 128 frames take 0.86 (resident) and 0.92 ms at 256 pulses, 2.5 and 2.8 at 512, 5.4
-// and 5.9 at 1024; 40 frames of 512 pulses 0.84 and 2.7. A batch that fills the CUs is the other way
-// round: 256 frames of 256 pulses 1.0 ms with one workgroup each, and more than that resident.
+// selected bins 128 frames take 0.76 (resident) and 0.94 ms at 256 pulses, 2.0 and 3.0 at 512, 4.0
+// and 6.0 at 1024; 40 frames of 512 pulses 0.74 and 2.98. A batch that fills the CUs is the other
+// way round: 256 frames of 256 pulses 1.0 ms with one workgroup each, and more than that resident.
 constexpr int kAfResidentFrames = 128;
 // Bound of a resident wait in the default form, in polls of about a microsecond; a frame that
 // reaches it is done over by one workgroup. Frames of a full launch wait for earlier ones, at most a
@@ -101,8 +101,7 @@ struct Job {
     float2* stm;                  // K x M x W (MTRC range-frequency rows)
     float2* czt;                  // K x M x W (chirp-z output)
     float2* colsum;               // K x W
-    float2* af_part;              // K x 4 (W/8) M: per-pulse sums per sub-chunk of selected bins, by iteration parity (split autofocus: the first half; resident: all, as tagged words)
-    unsigned* af_sync;            // K: per frame the resident autofocus's hand-off counter, cleared by k_autofocus
+    float2* af_part;              // K x 4 (W/8) M: per-pulse sums per sub-chunk of selected bins, by iteration parity (split autofocus: the first half; resident: up to three quarters, by iteration modulo 3)
     const float2* czt_table;      // W x F (FFT of the Bluestein chirp per range bin)
     const float2* czt_pre;        // W x M: exp(j pi a_n m (M - m) / M), the input chirp
     const float2* czt_post;       // W x M: exp(-j pi a_n k^2 / M) / F, the output chirp

@@ -222,7 +222,7 @@ def test_resident_wait_bound_sets_status():
                                               (512, 1024, 40, None), (1024, 2048, 3, None), (128, 1024, 3, -1),
                                               (1024, 2048, 3, -1)])
 def test_default_autofocus_form_equals_the_explicit_forms(M, N, frames, polls):
-    """AUTO takes the resident form up to 128 frames, with one workgroup per CU for the smaller batches,
+    """AUTO takes the resident form up to 128 frames, with as few workgroups on a CU as the batch allows,
     and one workgroup per frame above; a frame whose wait gave up (negative bound) is done over. Phases
     and images equal those of one workgroup per frame bit for bit and no frame reports status bit 2;
     140 iterations, above the 128 that a 7-bit iteration tag would hold."""
