@@ -374,8 +374,7 @@ int Context::enqueue(int frames, const void* echo, const double* velocity, const
     // a family launches at most log2(M) + 1 times per run; drain the ring only when it could overflow
     if (probe_stage >= 0 && probe_used + 16 > static_cast<int>(probe_events.size()) / 2) probe_collect();
     if (mode != ISAR_RUN_BACK) {
-        if (J.data_type == 1) probed(ISAR_STAGE_IFDS_PRE, s, [&] { launch_ifds_pre(J, s); });
-        else if (J.hrrp) probed(ISAR_STAGE_HRRP, s, [&] { launch_hrrp(J, s); });
+        if (J.hrrp && J.data_type == 2) probed(ISAR_STAGE_HRRP, s, [&] { launch_hrrp(J, s); });
         probed(ISAR_STAGE_RA_PAIR0, s, [&] { launch_ra_pair0(J, s); });
         int pair_base = M / 2;
         for (int st = 2; st < M; st *= 2) {

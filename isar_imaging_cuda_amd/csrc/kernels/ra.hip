@@ -48,7 +48,12 @@ __device__ __forceinline__ FftCT* stride16_rows(float2* lds) {
 //
 // The row's samples and window values are loaded first (RowSamples::load), together, and turned into
 // the spectrum later (spectrum), every element times `scale`, a power of two.
-template <int N, bool ONE_WINDOW = false>
+//
+// IFDS: the rows pass the pre-stage first (isar_main.cu:15-27: ifftshift, IFFT / N, ifftshift). Both
+// shifts by N / 2 are by eight register slots, so that transform runs where the row is
+// (prestage) instead of in a kernel of its own with a pass over memory each way: for 96 frames of
+// 256 x 4096 that took 305 us beside pair 0's 456, together they take 550.
+template <int N, bool ONE_WINDOW = false, bool IFDS = false>
 struct RowSamples {
     static_assert(FftPlan<N, kE>::R[0] == 16, "factorised phase assumes a radix-16 first pass");
     float2 v[kE];
@@ -58,20 +63,38 @@ struct RowSamples {
     __device__ __forceinline__ void load(const Job& J, int f, int m, int tid_) {
         const int tid = opaque(tid_);
         const long long erow = echo_first_row(J, f) + m;
-        const float2* row = J.data_type == 1 ? J.pre + (static_cast<size_t>(f) * J.M + m) * N
-                                             : J.echo + static_cast<size_t>(erow) * N;
-        velocity = J.if_hpc && J.data_type == 2 ? J.velocity[erow] : 0.0;
+        const float2* row = J.echo + static_cast<size_t>(erow) * N;
+        velocity = !IFDS && J.if_hpc ? J.velocity[erow] : 0.0;
 #pragma unroll
-        for (int e = 0; e < kE; ++e) v[e] = elem_u32(row + e * (N / kE), tid);
+        for (int e = 0; e < kE; ++e) v[e] = elem_u32(row + (IFDS ? e ^ 8 : e) * (N / kE), tid);
 #pragma unroll
         for (int e = 0; e < kE; ++e) w[e] = elem_u32(J.win_range + e * (N / kE), tid);
         issue_point();
     }
 
+    // The IFDS pre-stage of the loaded row but for its 1 / N. getHRRP for IFDS (common.cu:546-558) undoes
+    // the stage, ifftshift(FFT(ifftshift(pre))) = the input row, so the profile is the row itself.
+    __device__ __forceinline__ void prestage(const Job& J, int f, int m, float2* lds, int tid_,
+                                             const FftTwiddlesLds<N, kE>& tw) {
+        if (J.hrrp) {
+            const int tid = opaque(tid_);
+            float2* dst = J.hrrp + (static_cast<size_t>(f) * J.M + m) * N;
+#pragma unroll
+            for (int e = 0; e < kE; ++e) elem_u32(dst + (e ^ 8) * (N / kE), tid) = v[e];
+        }
+        fft<N, kE, +1>(v, lds, tid_, tw);
+#pragma unroll
+        for (int e = 0; e < kE / 2; ++e) {
+            const float2 t = v[e];
+            v[e] = v[e + 8];
+            v[e + 8] = t;
+        }
+    }
+
     __device__ __forceinline__ void spectrum(float2 (&x)[kE], const Job& J, int tid_, float scale) const {
         const int tid = opaque(tid_);
-        const bool hpc = J.if_hpc && J.data_type == 2;
-        const bool hrrp_window = !ONE_WINDOW && J.if_hrrp && J.data_type == 2;
+        const bool hpc = !IFDS && J.if_hpc;
+        const bool hrrp_window = !IFDS && !ONE_WINDOW && J.if_hrrp;
         // N/16 is even, so the sign (-1)^n is that of the thread
         const float sign = (tid & 1) ? -1.0f : 1.0f;
         auto window = [&](int e) { return sign * (hrrp_window ? w[e] * w[e] : w[e]); };
@@ -306,7 +329,8 @@ __device__ double parabola_lag(const float (&a)[kE], const float (&b)[kE], int b
 
 }  // namespace
 
-// IFDS pre-stage (isar_main.cu:15-27): ifftshift, IFFT / N, ifftshift of every row.
+// IFDS pre-stage (isar_main.cu:15-27): ifftshift, IFFT / N, ifftshift of every row, for stage reads (a
+// run does it in k_ra_pair0).
 template <int N>
 __global__ __launch_bounds__(N / kE) void k_ifds_pre(Job J) {
     HIP_DYNAMIC_SHARED(float2, lds);
@@ -316,12 +340,6 @@ __global__ __launch_bounds__(N / kE) void k_ifds_pre(Job J) {
     float2 x[kE];
 #pragma unroll
     for (int e = 0; e < kE; ++e) x[e] = src[(row_pos<N>(tid, e) + N / 2) & (N - 1)];
-    // getHRRP for IFDS (common.cu:546-558) undoes this stage, ifftshift(FFT(ifftshift(pre))) =
-    // the input row, so the profile is the row itself
-    if (J.hrrp) {
-#pragma unroll
-        for (int e = 0; e < kE; ++e) J.hrrp[off + ((row_pos<N>(tid, e) + N / 2) & (N - 1))] = x[e];
-    }
     fft<N, kE, +1>(x, lds, tid);
     const float inv = 1.0f / N;
 #pragma unroll
@@ -350,7 +368,10 @@ __global__ __launch_bounds__(N / kE) void k_hrrp(Job J) {
 // merged level-1 energy. Rows 0 and 1 never move again: their aligned profiles and column sums
 // are written here. The spectra carry the inverse transforms' 1 / N (a power of two), so no
 // profile or energy is scaled later.
-template <int N>
+// Bound by memory and by FP32 and FP64 issue alike: 1024 frames of 256 x 4096 take 5.5 ms, of which
+// the 23.6 GB read and written would take 5.0 at a copy's 4.7 TB/s and the instructions 4.1. (S0 of row
+// 2p+1 kept in registers instead of read again saves 4.3 GB, but the fourth wave of a SIMD does not fit then: 5.7 ms.)
+template <int N, bool IFDS>
 __global__ __launch_bounds__(N / kE, 4) void k_ra_pair0(Job J) {
     HIP_DYNAMIC_SHARED(float2, lds);
     constexpr int NT = N / kE;
@@ -365,16 +386,18 @@ __global__ __launch_bounds__(N / kE, 4) void k_ra_pair0(Job J) {
     float2* s0b = J.pre + (static_cast<size_t>(f) * M + rb) * N;
     float* dst = J.egrp + (static_cast<size_t>(f) * M + ra) * N;
     float* ap = J.arp_part + static_cast<size_t>(f) * (M / 2) * N;
-    RowSamples<N> row;
+    RowSamples<N, false, IFDS> row;
     row.load(J, f, ra, tid);
     const auto tw = fft_twiddles_lds<N, kE>(tid, stride16_rows<N>(lds));
     float2 x[kE];
     float ea[kE], eb[kE];
+    constexpr float scale = IFDS ? invN * invN : invN;
     float mx = 0.0f;
     // Every global location below is re-read only by the thread that wrote it, and the stores
     // into the S0 rows (which st aliases) are ordered by the barriers inside each transform.
     // row 2p: S0, profile, energy (kept in registers as the first term of the merged energy)
-    row.spectrum(x, J, tid, invN);
+    if constexpr (IFDS) row.prestage(J, f, ra, lds, tid, tw);
+    row.spectrum(x, J, tid, scale);
     {
         const int t = opaque(tid);
 #pragma unroll
@@ -396,7 +419,8 @@ __global__ __launch_bounds__(N / kE, 4) void k_ra_pair0(Job J) {
     for (int e = 0; e < kE; ++e) ea[e] = cabs2(x[e]);
     // row 2p+1: S0 and energy
     row.load(J, f, rb, tid);
-    row.spectrum(x, J, tid, invN);
+    if constexpr (IFDS) row.prestage(J, f, rb, lds, tid, tw);
+    row.spectrum(x, J, tid, scale);
     {
         const int t = opaque(tid);
 #pragma unroll
@@ -687,7 +711,8 @@ hipError_t configure_ra_kernels() {
 #define ISAR_SET_RA(NN)                                                        \
     set(reinterpret_cast<const void*>(&k_ifds_pre<NN>), ra_lds<NN>());         \
     set(reinterpret_cast<const void*>(&k_hrrp<NN>), ra_lds<NN>());             \
-    set(reinterpret_cast<const void*>(&k_ra_pair0<NN>), ra_lds<NN>());         \
+    set(reinterpret_cast<const void*>(&k_ra_pair0<NN, false>), ra_lds<NN>());  \
+    set(reinterpret_cast<const void*>(&k_ra_pair0<NN, true>), ra_lds<NN>());   \
     set(reinterpret_cast<const void*>(&k_ra_corr<NN>), ra_lds<NN>());          \
     set(reinterpret_cast<const void*>(&k_ra_upd<NN, kUpdAll>), ra_lds<NN>());   \
     set(reinterpret_cast<const void*>(&k_ra_upd<NN, kUpdFinal>), ra_lds<NN>()); \
@@ -714,7 +739,11 @@ void launch_hrrp(const Job& J, hipStream_t s) {
     ISAR_RANGE_SWITCH(J.N, ISAR_LAUNCH(k_hrrp<NN>, dim3(J.M, J.K), dim3(NN / kE), ra_lds<NN>(), s, J));
 }
 void launch_ra_pair0(const Job& J, hipStream_t s) {
-    ISAR_RANGE_SWITCH(J.N, ISAR_LAUNCH(k_ra_pair0<NN>, dim3(J.M / 2, J.K), dim3(NN / kE), ra_lds<NN>(), s, J));
+    if (J.data_type == 1) {
+        ISAR_RANGE_SWITCH(J.N, ISAR_LAUNCH((k_ra_pair0<NN, true>), dim3(J.M / 2, J.K), dim3(NN / kE), ra_lds<NN>(), s, J));
+    } else {
+        ISAR_RANGE_SWITCH(J.N, ISAR_LAUNCH((k_ra_pair0<NN, false>), dim3(J.M / 2, J.K), dim3(NN / kE), ra_lds<NN>(), s, J));
+    }
 }
 void launch_ra_corr(const Job& J, int stride, int pair_base, int nblocks, hipStream_t s) {
     ISAR_RANGE_SWITCH(J.N, ISAR_LAUNCH(k_ra_corr<NN>, dim3(nblocks, J.K), dim3(NN / kE), ra_lds<NN>(), s, J,

@@ -161,6 +161,21 @@ def test_pipeline_variants(name, dev, orc):
     assert rep.ok(), str(rep)
 
 
+@pytest.mark.parametrize("N", [1024, 2048, 4096, 8192, 16384])
+def test_ifds_prestage_at_every_row_length(N):
+    """The IFDS pre-stage runs inside the first alignment kernel, its two half-row shifts as an exchange
+    of register slots: every row length against the oracle, a batch of two frames."""
+    data = [_frame(1, echo_num=64, range_num=N, seed=360 + k) for k in range(2)]
+    radar = data[0][3]
+    print(f"[case] ifds pre-stage N={N}", flush=True)
+    img, tr = _run_device(np.stack([d[1] for d in data]), np.stack([d[2] for d in data]), radar, 64, N,
+                          isar.Options(data_type=1), frames=2)
+    for k in range(2):
+        img_o, tro = oracle_run(data[k][1], data[k][2], radar, 64, N, data_type=1)
+        rep = compare(img[k], tr[k], img_o, tro, 64)
+        assert rep.ok(), f"frame {k}: {rep}"
+
+
 @pytest.mark.parametrize("M,N", [(64, 1024), (128, 1024), (192, 1024), (256, 2048), (384, 1024), (512, 1024),
                                  (1024, 2048)])
 def test_autofocus_forms_agree(M, N):
