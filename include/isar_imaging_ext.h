@@ -220,9 +220,10 @@ ISAR_API int isar_set_graph_mode(isar_context* ctx, int on);
 ISAR_API int isar_set_ra_chunk(isar_context* ctx, int rows);
 ISAR_API int isar_get_ra_chunk(isar_context* ctx);
 /* Grids of the range-alignment update per merge level: 0 (default) by batch size, one grid below
- * 2^25 echo cells per batch and two from there (the rows of pair 0, which move for the last time
- * and carry the aligned-profile output, apart from the other pairs); 1 always one grid; 2 always
- * two. All give the same results bit for bit; the setting exists so that both launch forms can
+ * 192 frames per batch and two from there (the rows of pair 0, which move for the last time
+ * and carry the aligned-profile output, apart from the other pairs), with several rows of a chunk at
+ * once where a batch leaves the GPU idle otherwise; 1 always one grid; 2 always two, both row by
+ * row. All give the same results bit for bit; the setting exists so that both launch forms can
  * be exercised on small frames. */
 ISAR_API int isar_set_ra_split(isar_context* ctx, int mode);
 ISAR_API int isar_get_ra_split(isar_context* ctx);

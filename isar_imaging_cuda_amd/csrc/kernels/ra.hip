@@ -492,12 +492,12 @@ __global__ __launch_bounds__(N / kE, 4) void k_ra_corr(Job J, int s, int pair_ba
 // their column sums feed HRRP centring.
 // PART selects the grid: kUpdAll, the chunks of every pair (final rows where p = 0, one launch
 // per level); kUpdFinal, the chunks of pair 0 only; kUpdRest, those of pairs 1, 2, ... Apart
-// from the final-row work the three run the same code; split into kUpdFinal + kUpdRest, the
-// other pairs, most of the rows, do not carry that work's registers, at the cost of a second
-// launch per level.
+// from the final-row work the three run the same code.
+// Bound by memory: 1024 frames of 256 x 4096 read S0 of half the rows at each of seven levels and write
+// all profiles once, 41.6 GB in 8.3 ms.
 constexpr int kUpdAll = 0, kUpdFinal = 1, kUpdRest = 2;
 template <int N, int PART>
-__global__ __launch_bounds__(N / kE, PART == kUpdFinal && N <= 4096 ? 3 : 4) void k_ra_upd(Job J, int s, int pair_base) {
+__global__ __launch_bounds__(N / kE, 4) void k_ra_upd(Job J, int s, int pair_base) {
     HIP_DYNAMIC_SHARED(float2, lds);
     const int b = blockIdx.x, f = blockIdx.y, tid = threadIdx.x;
     const int M = J.M;
@@ -516,15 +516,13 @@ __global__ __launch_bounds__(N / kE, PART == kUpdFinal && N <= 4096 ? 3 : 4) voi
     for (int e = 0; e < kE; ++e) acc[e] = 0.0f;
     float2 x[kE];
     const auto tw = fft_twiddles_lds<N, kE>(tid, stride16_rows<N>(lds));
-    // column sums of |profile| over the final rows of this chunk: kept in registers by the
-    // final-row grid up to 4096 cells (above, its workgroup size leaves no room) and stored once,
-    // otherwise accumulated in place (each location is read back only by the thread that wrote
-    // it); the same additions in the same order either way
-    constexpr bool kArpInRegs = PART == kUpdFinal && N <= 4096;
+    // column sums of |profile| over the final rows of this chunk, in registers (added in place in memory
+    // they cost a final row as many bytes again: 40 frames of 512 x 8192 took 2.16 instead of 1.75 ms)
+    constexpr bool kFinal = PART != kUpdRest;
     float* ap = J.arp_part + (static_cast<size_t>(f) * (M / 2) + r0 / 2) * N;
-    float arp[kArpInRegs ? kE : 1];
+    float arp[kFinal ? kE : 1];
 #pragma unroll
-    for (int e = 0; e < (kArpInRegs ? kE : 1); ++e) arp[e] = 0.0f;
+    for (int e = 0; e < (kFinal ? kE : 1); ++e) arp[e] = 0.0f;
 #pragma unroll 1
     for (int m = r0; m < r1; ++m) {
         load_row_shifted<N>(x, J, f, m, J.lagsum[static_cast<size_t>(f) * M + m], lag, tid);
@@ -539,14 +537,13 @@ __global__ __launch_bounds__(N / kE, PART == kUpdFinal && N <= 4096 ? 3 : 4) voi
                 const int pos = row_pos<N>(t, e);
                 elem_u32(st, pos) = x[e];
                 const float av = cabs_hw(x[e]);
-                if constexpr (kArpInRegs) arp[e] += av;
-                else elem_u32(ap, pos) = (m == r0 ? 0.0f : elem_u32(ap, pos)) + av;
+                if constexpr (kFinal) arp[e] += av;
                 mx = fmaxf(mx, av);
             }
         }
     }
     if (final_rows) {
-        if constexpr (kArpInRegs) {
+        if constexpr (kFinal) {
             const int t = opaque(tid);
 #pragma unroll
             for (int e = 0; e < kE; ++e) elem_u32(ap, row_pos<N>(t, e)) = arp[e];
@@ -751,15 +748,14 @@ void launch_ra_corr(const Job& J, int stride, int pair_base, int nblocks, hipStr
 }
 void launch_ra_upd(const Job& J, int stride, int pair_base, int nblocks, hipStream_t s) {
     // nblocks = pairs x chunks per pair. Chunks that would leave SIMDs without work take several rows at
-    // once. Large batches launch pair 0 (final rows) and the other
-    // pairs apart; small ones, where the second launch per level costs more than it saves, in one.
+    // once. Batches of many frames launch pair 0 (final rows) and the other pairs apart, others together.
     const int R = std::min(stride, J.ra_chunk), cpp = (stride + R - 1) / R;
     if (J.ra_split == 0) {
         bool done = false;
         ISAR_RANGE_SWITCH(J.N, done = upd_rows<NN>(J, stride, pair_base, nblocks, R, s));
         if (done) return;
     }
-    const bool split = J.ra_split == 2 || (J.ra_split == 0 && static_cast<long long>(J.K) * J.M * J.N >= kRaSplitCells);
+    const bool split = J.ra_split == 2 || (J.ra_split == 0 && J.K >= kRaSplitFrames);
     if (!split) {
         ISAR_RANGE_SWITCH(J.N, ISAR_LAUNCH((k_ra_upd<NN, kUpdAll>), dim3(nblocks, J.K), dim3(NN / kE), ra_lds<NN>(),
                                            s, J, stride, pair_base));

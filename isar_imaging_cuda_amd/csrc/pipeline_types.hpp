@@ -35,9 +35,13 @@ constexpr int kAfGuardedPolls = 1 << 16;
 // Sub-aperture plans run several groups at once; their default is the split form up to this many
 // windows, one workgroup per window above.
 constexpr int kAfSplitFrames = 32;
-// batches of at least this many echo cells (frames x pulses x range cells; 32 frames of 256 x 4096)
-// update the final rows of range alignment in a launch of their own
-constexpr long long kRaSplitCells = 1LL << 25;
+// Batches of at least this many frames update the final rows of range alignment in a launch of their
+// own, since then it fills the GPU by itself: all levels of 1024 frames of 256 x 4096 take 8.3 instead
+// of 9.3 ms, of 256 such frames 2.26 and 2.35, of 512 frames of 128 x 1024 0.53 and 0.58. With fewer
+// frames the launches, one after the other, leave it idle between them: 40 frames of 512 x 8192 1.89
+// (apart) and 1.75 ms (together), 8 of 1024 x 16384 2.14 and 1.77, 96 of 256 x 4096 0.93 and 0.91,
+// 160 about alike.
+constexpr int kRaSplitFrames = 192;
 
 // Per-frame scalar decisions written by the device (one record per frame).
 struct FrameDecisions {
