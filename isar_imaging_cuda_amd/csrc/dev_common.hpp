@@ -84,52 +84,97 @@ __device__ __forceinline__ float2 expjpi_twiddle(float t) {
 }
 
 // ------------------------------------------------------------------------------------------
+// exchange between the lanes of a wave
+// ------------------------------------------------------------------------------------------
+// v of lane (lane ^ MASK), a power of two below 64: by DPP moves within a row of 16 lanes and by the
+// swap instructions between rows, so no trip through the LDS crossbar (about 100 cycles a step in
+// the one-workgroup kernels, whose chains of such steps nothing else covers).
+template <int MASK>
+__device__ __forceinline__ unsigned lane_xor_bits(unsigned v) {
+#ifdef ISAR_EMU
+    return __shfl_xor(v, MASK, 64);
+#else
+    static_assert(MASK == 1 || MASK == 2 || MASK == 4 || MASK == 8 || MASK == 16 || MASK == 32, "one bit of the lane");
+    const int b = static_cast<int>(v);
+    if constexpr (MASK == 1) return __builtin_amdgcn_mov_dpp(b, 0xB1, 0xf, 0xf, true);        // quad_perm 1 0 3 2
+    else if constexpr (MASK == 2) return __builtin_amdgcn_mov_dpp(b, 0x4E, 0xf, 0xf, true);   // quad_perm 2 3 0 1
+    else if constexpr (MASK == 4)   // half-row mirror (lane ^ 7), then quad_perm 3 2 1 0 (lane ^ 3)
+        return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(b, 0x141, 0xf, 0xf, true), 0x1B, 0xf, 0xf, true);
+    else if constexpr (MASK == 8) return __builtin_amdgcn_mov_dpp(b, 0x128, 0xf, 0xf, true);  // row rotate by 8
+    else if constexpr (MASK == 16) {   // odd rows of the first with even rows of the second
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return (threadIdx.x & 16) ? r[0] : r[1];
+    } else {                           // upper half of the first with lower half of the second
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return (threadIdx.x & 32) ? r[0] : r[1];
+    }
+#endif
+}
+template <int MASK>
+__device__ __forceinline__ int lane_xor(int v) { return static_cast<int>(lane_xor_bits<MASK>(static_cast<unsigned>(v))); }
+template <int MASK>
+__device__ __forceinline__ float lane_xor(float v) { return __uint_as_float(lane_xor_bits<MASK>(__float_as_uint(v))); }
+template <int MASK, typename T>
+__device__ __forceinline__ T lane_xor_64(T v) {
+    uint64_t b;
+    __builtin_memcpy(&b, &v, sizeof b);
+    b = (static_cast<uint64_t>(lane_xor_bits<MASK>(static_cast<unsigned>(b >> 32))) << 32) |
+        lane_xor_bits<MASK>(static_cast<unsigned>(b));
+    __builtin_memcpy(&v, &b, sizeof b);
+    return v;
+}
+template <int MASK>
+__device__ __forceinline__ double lane_xor(double v) { return lane_xor_64<MASK>(v); }
+template <int MASK>
+__device__ __forceinline__ long long lane_xor(long long v) { return lane_xor_64<MASK>(v); }
+template <int MASK>
+__device__ __forceinline__ float2 lane_xor(float2 v) { return make_float2(lane_xor<MASK>(v.x), lane_xor<MASK>(v.y)); }
+
+// v combined over groups of WIDTH lanes (a power of two up to 64) by steps v = step(v, v of lane ^ WIDTH / 2,
+// ... ^ 1)
+template <int WIDTH, typename T, typename F>
+__device__ __forceinline__ T group_combine(T v, F step) {
+    if constexpr (WIDTH >= 64) v = step(v, lane_xor<32>(v));
+    if constexpr (WIDTH >= 32) v = step(v, lane_xor<16>(v));
+    if constexpr (WIDTH >= 16) v = step(v, lane_xor<8>(v));
+    if constexpr (WIDTH >= 8) v = step(v, lane_xor<4>(v));
+    if constexpr (WIDTH >= 4) v = step(v, lane_xor<2>(v));
+    if constexpr (WIDTH >= 2) v = step(v, lane_xor<1>(v));
+    return v;
+}
+
+// ------------------------------------------------------------------------------------------
 // reductions
 // ------------------------------------------------------------------------------------------
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return group_combine<64>(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ double wave_sum_d(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return group_combine<64>(v, [](double a, double b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+    return group_combine<64>(v, [](float a, float b) { return fmaxf(a, b); });
 }
 __device__ __forceinline__ float2 wave_sum2(float2 v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        v.x += __shfl_xor(v.x, o, 64);
-        v.y += __shfl_xor(v.y, o, 64);
-    }
-    return v;
+    return group_combine<64>(v, [](float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); });
 }
-// (value, index) argmax with lowest index on ties
-__device__ __forceinline__ void wave_argmax(float& v, int& i) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(v, o, 64);
-        const int oi = __shfl_xor(i, o, 64);
-        const bool take = (ov > v) | ((ov == v) & (oi < i));
-        v = take ? ov : v;
-        i = take ? oi : i;
-    }
+// (value, index) argmax and argmin with the lowest index on ties: LESS = true takes the smaller value
+template <bool LESS, int MASK>
+__device__ __forceinline__ void wave_arg_step(float& v, int& i) {
+    const float ov = lane_xor<MASK>(v);
+    const int oi = lane_xor<MASK>(i);
+    const bool take = (LESS ? ov < v : ov > v) | ((ov == v) & (oi < i));
+    v = take ? ov : v;
+    i = take ? oi : i;
 }
-// (value, index) argmin with lowest index on ties
-__device__ __forceinline__ void wave_argmin(float& v, int& i) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(v, o, 64);
-        const int oi = __shfl_xor(i, o, 64);
-        const bool take = (ov < v) | ((ov == v) & (oi < i));
-        v = take ? ov : v;
-        i = take ? oi : i;
-    }
+template <bool LESS>
+__device__ __forceinline__ void wave_arg(float& v, int& i) {
+    wave_arg_step<LESS, 32>(v, i);
+    wave_arg_step<LESS, 16>(v, i);
+    wave_arg_step<LESS, 8>(v, i);
+    wave_arg_step<LESS, 4>(v, i);
+    wave_arg_step<LESS, 2>(v, i);
+    wave_arg_step<LESS, 1>(v, i);
 }
 
 // Workgroup-wide reductions through a small LDS scratch (>= 16 slots). All threads get the
@@ -148,8 +193,7 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 }
 template <int NT>
 __device__ __forceinline__ long long block_sum_i64(long long v, long long* red) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    v = group_combine<64>(v, [](long long a, long long b) { return a + b; });
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     __syncthreads();
     if (l == 0) red[w] = v;
@@ -173,7 +217,7 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 }
 template <int NT>
 __device__ __forceinline__ void block_argmax(float& v, int& i, float* redv, int* redi) {
-    wave_argmax(v, i);
+    wave_arg<false>(v, i);
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     __syncthreads();
     if (l == 0) { redv[w] = v; redi[w] = i; }
@@ -191,7 +235,7 @@ __device__ __forceinline__ void block_argmax(float& v, int& i, float* redv, int*
 }
 template <int NT>
 __device__ __forceinline__ void block_argmin(float& v, int& i, float* redv, int* redi) {
-    wave_argmin(v, i);
+    wave_arg<true>(v, i);
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     __syncthreads();
     if (l == 0) { redv[w] = v; redi[w] = i; }
@@ -334,19 +378,12 @@ namespace isar {
 template <int WIDTH>
 __device__ __forceinline__ float group_sum(float v) {
     static_assert(WIDTH <= 64, "shuffle groups cannot span waves");
-#pragma unroll
-    for (int o = WIDTH / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WIDTH);
-    return v;
+    return group_combine<WIDTH>(v, [](float a, float b) { return a + b; });
 }
 template <int WIDTH>
 __device__ __forceinline__ float2 group_sum2(float2 v) {
     static_assert(WIDTH <= 64, "shuffle groups cannot span waves");
-#pragma unroll
-    for (int o = WIDTH / 2; o > 0; o >>= 1) {
-        v.x += __shfl_xor(v.x, o, WIDTH);
-        v.y += __shfl_xor(v.y, o, WIDTH);
-    }
-    return v;
+    return group_combine<WIDTH>(v, [](float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); });
 }
 
 // Inclusive prefix sum in FP64 of n values held as v[i] (i < n) in LDS, in place, by the whole

@@ -28,11 +28,27 @@ __device__ void bitonic_sort_f(float* a, int n) {
     }
 }
 
+// Stage (k, j) of a thread's elements i0 ... i0 + E - 1 against those of the partner thread, which
+// partner(v) reads.
+template <int E, typename F>
+__device__ __forceinline__ void bitonic_partner_step(float (&v)[E], int i0, int j, int k, F partner) {
+    const bool lower = (i0 & j) == 0;
+    const bool up = (i0 & k) == 0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const float p = partner(v[e]);
+        // x = the lower index's value, y = the higher one's
+        const float x = lower ? v[e] : p, y = lower ? p : v[e];
+        const bool sw = (x > y) == up;
+        v[e] = sw ? p : v[e];
+    }
+}
+
 // The same compare-exchange network (stage (k, j) orders each pair i < i ^ j ascending where
 // i & k == 0, descending otherwise, swapping when (a[i] > a[i ^ j]) == ascending), with the stages
 // inside a wave taken out of LDS: thread t holds elements t E ... t E + E - 1 in registers, stages
 // j < E exchange within the thread, stages E <= j < 64 E with the partner thread t ^ (j / E) of
-// the same wave by shuffles, and only the stages j >= 64 E go through LDS with a barrier each
+// the same wave (lane_xor or shuffles), and only the stages j >= 64 E go through LDS with a barrier each
 // (10 of the 105 stages at 16384 elements). Every pair meets the same comparator in the same
 // stage as in bitonic_sort_f, so the sorted array is the same bit for bit, NaNs included.
 // n = NT E; every thread of the workgroup calls it, with a in LDS and a barrier after its fill.
@@ -67,15 +83,20 @@ __device__ void bitonic_sort_f_waves(float* a) {
             in_regs = true;
         }
         for (; j >= E; j >>= 1) {   // partner thread t ^ (j / E) of the same wave
-            const bool lower = (i0 & j) == 0;
-            const bool up = (i0 & k) == 0;
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const float p = __shfl_xor(v[e], j / E, 64);
-                // x = the lower index's value, y = the higher one's
-                const float x = lower ? v[e] : p, y = lower ? p : v[e];
-                const bool sw = (x > y) == up;
-                v[e] = sw ? p : v[e];
+            // From 8 elements on by lane_xor with the code of each step apart: 16384 cells take 101 instead
+            // of 113 us. With 4 (4096 cells) fetching that code, which runs once, costs more than
+            // the shuffles: 32 instead of 29 us.
+            if constexpr (E >= 8) {
+                switch (j / E) {
+                case 32: bitonic_partner_step(v, i0, j, k, [](float a) { return lane_xor<32>(a); }); break;
+                case 16: bitonic_partner_step(v, i0, j, k, [](float a) { return lane_xor<16>(a); }); break;
+                case 8: bitonic_partner_step(v, i0, j, k, [](float a) { return lane_xor<8>(a); }); break;
+                case 4: bitonic_partner_step(v, i0, j, k, [](float a) { return lane_xor<4>(a); }); break;
+                case 2: bitonic_partner_step(v, i0, j, k, [](float a) { return lane_xor<2>(a); }); break;
+                default: bitonic_partner_step(v, i0, j, k, [](float a) { return lane_xor<1>(a); }); break;
+                }
+            } else {
+                bitonic_partner_step(v, i0, j, k, [j](float a) { return __shfl_xor(a, j / E, 64); });
             }
         }
 #pragma unroll
