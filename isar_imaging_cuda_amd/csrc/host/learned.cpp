@@ -155,13 +155,14 @@ ISAR_API int isar_mlp_forward(isar_mlp* net, int batch, const float* d_in, float
     const float* a = d_in;
     for (int l = 0; l < L; ++l) {
         const int in = net->widths[l], o = net->widths[l + 1];
-        float* z = net->act[l + 1];
+        // the last layer writes the caller's buffer, unless it reads the caller's input as well, which may be the same
+        float* z = l + 1 == L && l > 0 ? d_out : net->act[l + 1];
         isar::launch_gemm_f32_bf16w(batch, o, in, a, in, 1, net->wbf + net->wb_off[l], o, 1, z, o,
                                     net->params + net->b_off[l], l + 1 < L ? 1 : 0, s);
         a = z;
     }
     const size_t bytes = static_cast<size_t>(batch) * net->widths[L] * sizeof(float);
-    if (hipMemcpyAsync(d_out, net->act[L], bytes, hipMemcpyDeviceToDevice, s) != hipSuccess)
+    if (L == 1 && hipMemcpyAsync(d_out, net->act[L], bytes, hipMemcpyDeviceToDevice, s) != hipSuccess)
         return fail(ISAR_ERR_DEVICE, "isar_mlp_forward: output copy failed");
     if (hipGetLastError() != hipSuccess) return fail(ISAR_ERR_DEVICE, "isar_mlp_forward: launch failed");
     net->input = d_in;
@@ -181,8 +182,8 @@ ISAR_API int isar_mlp_backward(isar_mlp* net, int batch, const float* d_grad_out
         const int in = net->widths[l], o = net->widths[l + 1];
         const float* a_prev = l == 0 ? net->input : net->act[l];
         // dW = A_prev^T dZ (in x o), db = column sums of dZ
-        isar::launch_gemm_f32_f32(in, o, batch, a_prev, 1, in, dz, o, 1, net->grads + net->w_off[l], o, s);
-        isar::launch_colsum(batch, o, dz, net->grads + net->b_off[l], s);
+        isar::launch_gemm_f32_f32(in, o, batch, a_prev, 1, in, dz, o, 1, net->grads + net->w_off[l], o,
+                                  net->grads + net->b_off[l], s);
         if (l > 0) {
             // dA_prev = dZ W^T, then through the ReLU of layer l - 1 (its output is A_prev)
             float* next = net->dz[ping];

@@ -50,6 +50,14 @@ struct Frag {
             for (int t = 0; t < 8; ++t) v[t] = p[min(kk + t, k - 1) * s_k];
         }
     }
+    // the eight added in order, those of kk >= k left out
+    __device__ __forceinline__ float sum(int kk, int k) const {
+        static_assert(!VEC, "single loads");
+        float s = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) s += kk + t < k ? v[t] : 0.0f;
+        return s;
+    }
     __device__ __forceinline__ bf16x8 get(int kk, int k) const {
         T e[8];
         if constexpr (VEC) __builtin_memcpy(e, v, sizeof e);
@@ -69,6 +77,9 @@ struct Frag {
 // C[m][n] = sum_k A(m, k) B(k, n) with A(m, k) = a[m sam + k sak], B(k, n) = b[k sbk + n sbn],
 // operands rounded to BF16, products accumulated in FP32 in the order of k. One wave per block of
 // 16 T x 16 T of C. Epilogue: 0 store; 1 + bias[n], then max(0, .); 2 + bias[n]; 3 times (mask[m][n] > 0).
+// With EPI = 0 the waves of the first row of blocks also add B's columns before rounding, colsum[n] =
+// sum_k B(k, n): of the weight gradient's operand dZ that is the bias gradient, which took a launch of its own
+// and another pass over dZ (14 of a training step's 159 us).
 // AV, BV: the operand's k are consecutive and aligned (Frag).
 //
 // Bound by the latency of its loads: the matrix work of a layer is under a microsecond, its
@@ -81,7 +92,8 @@ template <typename TA, typename TB, int EPI, int T, bool AV, bool BV>
 __global__ __launch_bounds__(64) void k_gemm_bf16(int m, int n, int k, const TA* __restrict__ a, long sam, long sak,
                                                   const TB* __restrict__ b, long sbk, long sbn, float* __restrict__ c,
                                                   long scm, const float* __restrict__ bias,
-                                                  const float* __restrict__ mask, long smm) {
+                                                  const float* __restrict__ mask, long smm,
+                                                  float* __restrict__ colsum) {
     constexpr int kTile = 16 * T, kSteps = T == 1 ? 4 : 2;
     const int l = threadIdx.x;
     const int bm = blockIdx.y * kTile, bn = blockIdx.x * kTile;
@@ -91,6 +103,9 @@ __global__ __launch_bounds__(64) void k_gemm_bf16(int m, int n, int k, const TA*
     for (int i = 0; i < T; ++i)
 #pragma unroll
         for (int j = 0; j < T; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    float cs[T];
+#pragma unroll
+    for (int i = 0; i < T; ++i) cs[i] = 0.0f;
     for (int k0 = 0; k0 < k; k0 += 32 * kSteps) {
         Frag<TA, AV> fa[kSteps][T];
         Frag<TB, BV> fb[kSteps][T];
@@ -113,6 +128,7 @@ __global__ __launch_bounds__(64) void k_gemm_bf16(int m, int n, int k, const TA*
             for (int i = 0; i < T; ++i) {
                 va[i] = fa[q][i].get(kk, k);
                 vb[i] = fb[q][i].get(kk, k);
+                if constexpr (EPI == 0) cs[i] += fb[q][i].sum(kk, k);
             }
 #pragma unroll
             for (int i = 0; i < T; ++i)
@@ -137,37 +153,17 @@ __global__ __launch_bounds__(64) void k_gemm_bf16(int m, int n, int k, const TA*
                 c[row * scm + col] = v;
             }
         }
-}
-
-// bias gradient: db[j] = sum_b dz[b][j]. A workgroup takes 64 columns, each wave a contiguous 16th of
-// the rows with sixteen loads in flight; the waves' sums are added in wave order. Bound by latency:
-// 256 rows take 2 to 4 us, with one thread per column and a load waited for per row they took 59.
-constexpr int kColsumWaves = 16;
-__global__ __launch_bounds__(64 * kColsumWaves) void k_colsum(int rows, int cols, const float* __restrict__ dz,
-                                                              float* __restrict__ db) {
-    __shared__ float part[kColsumWaves][64];
-    const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
-    const int j = blockIdx.x * 64 + lane;
-    const int share = (rows + kColsumWaves - 1) / kColsumWaves;
-    const int r0 = min(w * share, rows), r1 = min(r0 + share, rows);
-    const float* col = dz + min(j, cols - 1);
-    float s = 0.0f;
-    for (int r = r0; r < r1; r += 16) {
-        float v[16];
+    if constexpr (EPI == 0) {
+        if (blockIdx.y == 0) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = col[static_cast<size_t>(min(r + i, r1 - 1)) * cols];
-        issue_point();
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if (r + i < r1) s += v[i];
+            for (int i = 0; i < T; ++i) {   // the four groups of 16 lanes hold every fourth eight of k
+                cs[i] += lane_xor<32>(cs[i]);
+                cs[i] += lane_xor<16>(cs[i]);
+                const int col = bn + 16 * i + li;
+                if (l < 16 && col < n) colsum[col] = cs[i];
+            }
+        }
     }
-    part[w][lane] = s;
-    __syncthreads();
-    if (w != 0 || j >= cols) return;
-    float t = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kColsumWaves; ++i) t += part[i][lane];
-    db[j] = t;
 }
 
 // Adam (bias-corrected) on FP32 master parameters; the BF16 copy of each weight follows.
@@ -403,14 +399,14 @@ bool vector_k(const T* p, long s_k, long s_line, int k) {
 // neither is.
 template <typename TA, typename TB, int EPI, bool AK, bool BK>
 void gemm_bf16(int m, int n, int k, const TA* a, long sam, long sak, const TB* b, long sbk, long sbn, float* c, long scm,
-               const float* bias, const float* mask, long smm, hipStream_t s) {
+               const float* bias, const float* mask, long smm, float* colsum, hipStream_t s) {
     const bool small = use_small_tiles(m, n);
     const bool vec = (AK || BK) && (!AK || vector_k(a, sak, sam, k)) && (!BK || vector_k(b, sbk, sbn, k));
     const int tile = small ? 16 : 32;
     const dim3 grid((n + tile - 1) / tile, (m + tile - 1) / tile);
 #define ISAR_GEMM(T, AV, BV)                                                                                           \
     ISAR_LAUNCH((k_gemm_bf16<TA, TB, EPI, T, AV, BV>), grid, dim3(64), 0, s, m, n, k, a, sam, sak, b, sbk, sbn, c, scm, \
-                bias, mask, smm)
+                bias, mask, smm, colsum)
     if (vec) {
         if (small) ISAR_GEMM(1, AK, BK);
         else ISAR_GEMM(2, AK, BK);
@@ -424,19 +420,16 @@ void gemm_bf16(int m, int n, int k, const TA* a, long sam, long sak, const TB* b
 
 void launch_gemm_f32_bf16w(int m, int n, int k, const float* a, long sam, long sak, const uint16_t* w, long sbk,
                            long sbn, float* c, long scm, const float* bias, int relu, hipStream_t s) {
-    if (relu) gemm_bf16<float, uint16_t, 1, true, false>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, bias, nullptr, 0L, s);
-    else gemm_bf16<float, uint16_t, 2, true, false>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, bias, nullptr, 0L, s);
+    if (relu) gemm_bf16<float, uint16_t, 1, true, false>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, bias, nullptr, 0L, nullptr, s);
+    else gemm_bf16<float, uint16_t, 2, true, false>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, bias, nullptr, 0L, nullptr, s);
 }
 void launch_gemm_f32_bf16w_masked(int m, int n, int k, const float* a, long sam, long sak, const uint16_t* w,
                                   long sbk, long sbn, float* c, long scm, const float* mask, long smm, hipStream_t s) {
-    gemm_bf16<float, uint16_t, 3, true, true>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, nullptr, mask, smm, s);
+    gemm_bf16<float, uint16_t, 3, true, true>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, nullptr, mask, smm, nullptr, s);
 }
 void launch_gemm_f32_f32(int m, int n, int k, const float* a, long sam, long sak, const float* b, long sbk, long sbn,
-                         float* c, long scm, hipStream_t s) {
-    gemm_bf16<float, float, 0, false, false>(m, n, k, a, sam, sak, b, sbk, sbn, c, scm, nullptr, nullptr, 0L, s);
-}
-void launch_colsum(int rows, int cols, const float* dz, float* db, hipStream_t s) {
-    ISAR_LAUNCH(k_colsum, dim3((cols + 63) / 64), dim3(64 * kColsumWaves), 0, s, rows, cols, dz, db);
+                         float* c, long scm, float* colsum, hipStream_t s) {
+    gemm_bf16<float, float, 0, false, false>(m, n, k, a, sam, sak, b, sbk, sbn, c, scm, nullptr, nullptr, 0L, colsum, s);
 }
 void launch_adam(int n, float* p, const float* g, float* m1, float* m2, uint16_t* pb, const int* bf_index, float lr,
                  float beta1, float beta2, float eps, float c1, float c2, hipStream_t s) {

@@ -56,8 +56,7 @@ void launch_gemm_f32_bf16w(int m, int n, int k, const float* a, long sam, long s
 void launch_gemm_f32_bf16w_masked(int m, int n, int k, const float* a, long sam, long sak, const uint16_t* w,
                                   long sbk, long sbn, float* c, long scm, const float* mask, long smm, hipStream_t s);
 void launch_gemm_f32_f32(int m, int n, int k, const float* a, long sam, long sak, const float* b, long sbk, long sbn,
-                         float* c, long scm, hipStream_t s);
-void launch_colsum(int rows, int cols, const float* dz, float* db, hipStream_t s);
+                         float* c, long scm, float* colsum, hipStream_t s);
 void launch_adam(int n, float* p, const float* g, float* m1, float* m2, uint16_t* pb, const int* bf_index, float lr,
                  float beta1, float beta2, float eps, float c1, float c2, hipStream_t s);
 void launch_to_bf16(int n, const float* p, uint16_t* pb, const int* bf_index, hipStream_t s);
