@@ -268,7 +268,8 @@ __device__ double parabola_lag(const float (&a)[kE], const float (&b)[kE], int b
                                double* lag_out, int32_t* imax_out) {
     constexpr int NT = N / kE;
     // cl[i] = c[i - N/2] and c[l] = sum_n gA[n] gB[n - l] (mod N): the samples at bi - 1, bi,
-    // bi + 1 are lags l0 - 1, l0, l0 + 1 with l0 = bi - N/2. gB goes to LDS by range cell (N
+    // bi + 1 are lags l0 - 1, l0, l0 + 1 with l0 = bi - N/2. gB goes to LDS by range cell, its first
+    // two cells once more behind the last, so that the three cells of a product follow each other (N + 2
     // doubles fit the transform's padded N float2); each thread sums over its own cells. The
     // per-wave sums follow gB in LDS and are added in wave order, so the result does not depend
     // on scheduling.
@@ -277,20 +278,24 @@ __device__ double parabola_lag(const float (&a)[kE], const float (&b)[kE], int b
     // opaque() so that the roots are not shared with the transform input above and kept live
     // across its transforms.
     double* gb = reinterpret_cast<double*>(lds);
-    double* red = gb + N;
+    double* red = gb + N + 2;
     auto pos = [&](int e) { return row_pos<N>(tid, e); };
 #pragma unroll
-    for (int e = 0; e < kE; ++e) gb[pos(e)] = sqrt_refined(opaque(b[e]));
+    for (int e = 0; e < kE; ++e) {
+        const double g = sqrt_refined(opaque(b[e]));
+        gb[pos(e)] = g;
+        if (e == 0 && tid < 2) gb[N + tid] = g;
+    }
     __syncthreads();
     const int l0 = bi - N / 2;
     double s1 = 0.0, s2 = 0.0, s3 = 0.0;
 #pragma unroll
     for (int e = 0; e < kE; ++e) {
-        const int n = pos(e);
         const double ga = sqrt_refined(opaque(a[e]));
-        s1 = fma(ga, gb[(n - l0 + 1) & (N - 1)], s1);
-        s2 = fma(ga, gb[(n - l0) & (N - 1)], s2);
-        s3 = fma(ga, gb[(n - l0 - 1) & (N - 1)], s3);
+        const double* g = gb + ((pos(e) - l0 - 1) & (N - 1));
+        s1 = fma(ga, g[2], s1);
+        s2 = fma(ga, g[1], s2);
+        s3 = fma(ga, g[0], s3);
     }
     s1 = wave_sum_d(s1);
     s2 = wave_sum_d(s2);
