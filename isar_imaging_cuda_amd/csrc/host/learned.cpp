@@ -155,10 +155,11 @@ ISAR_API int isar_mlp_forward(isar_mlp* net, int batch, const float* d_in, float
     const float* a = d_in;
     for (int l = 0; l < L; ++l) {
         const int in = net->widths[l], o = net->widths[l + 1];
-        // the last layer writes the caller's buffer, unless it reads the caller's input as well, which may be the same
+        // the last layer writes the caller's buffer, unless it reads the caller's input as well, which
+        // may be the same
         float* z = l + 1 == L && l > 0 ? d_out : net->act[l + 1];
-        isar::launch_gemm_f32_bf16w(batch, o, in, a, in, 1, net->wbf + net->wb_off[l], o, 1, z, o,
-                                    net->params + net->b_off[l], l + 1 < L ? 1 : 0, s);
+        isar::launch_dense_forward(batch, in, o, a, net->wbf + net->wb_off[l], net->params + net->b_off[l], z,
+                                   l + 1 < L ? 1 : 0, s);
         a = z;
     }
     const size_t bytes = static_cast<size_t>(batch) * net->widths[L] * sizeof(float);
@@ -181,17 +182,13 @@ ISAR_API int isar_mlp_backward(isar_mlp* net, int batch, const float* d_grad_out
     for (int l = L - 1; l >= 0; --l) {
         const int in = net->widths[l], o = net->widths[l + 1];
         const float* a_prev = l == 0 ? net->input : net->act[l];
-        // dW = A_prev^T dZ (in x o), db = column sums of dZ
-        isar::launch_gemm_f32_f32(in, o, batch, a_prev, 1, in, dz, o, 1, net->grads + net->w_off[l], o,
-                                  net->grads + net->b_off[l], s);
-        if (l > 0) {
-            // dA_prev = dZ W^T, then through the ReLU of layer l - 1 (its output is A_prev)
-            float* next = net->dz[ping];
-            isar::launch_gemm_f32_bf16w_masked(batch, in, o, dz, o, 1, net->wbf + net->wb_off[l], 1, o, next, in,
-                                               a_prev, in, s);
-            dz = next;
-            ping ^= 1;
-        }
+        // the weight and bias gradients, and for l > 0 dA_prev = dZ W^T through the ReLU of layer l - 1
+        // (its output is A_prev)
+        float* next = l > 0 ? net->dz[ping] : nullptr;
+        isar::launch_dense_backward(batch, in, o, a_prev, dz, net->wbf + net->wb_off[l], net->grads + net->w_off[l],
+                                    net->grads + net->b_off[l], next, s);
+        dz = next;
+        ping ^= 1;
     }
     if (hipGetLastError() != hipSuccess) return fail(ISAR_ERR_DEVICE, "isar_mlp_backward: launch failed");
     return ISAR_OK;

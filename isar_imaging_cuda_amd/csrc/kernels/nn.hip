@@ -72,14 +72,27 @@ struct Frag {
     }
 };
 
-}  // namespace
+template <typename TA, typename TB>
+struct GemmArgs {
+    int m, n, k;
+    const TA* a;
+    long sam, sak;
+    const TB* b;
+    long sbk, sbn;
+    float* c;
+    long scm;
+    const float* bias;
+    const float* mask;
+    long smm;
+    float* colsum;
+};
 
 // C[m][n] = sum_k A(m, k) B(k, n) with A(m, k) = a[m sam + k sak], B(k, n) = b[k sbk + n sbn],
 // operands rounded to BF16, products accumulated in FP32 in the order of k. One wave per block of
 // 16 T x 16 T of C. Epilogue: 0 store; 1 + bias[n], then max(0, .); 2 + bias[n]; 3 times (mask[m][n] > 0).
 // With EPI = 0 the waves of the first row of blocks also add B's columns before rounding, colsum[n] =
-// sum_k B(k, n): of the weight gradient's operand dZ that is the bias gradient, which took a launch of its own
-// and another pass over dZ (14 of a training step's 159 us).
+// sum_k B(k, n): of the weight gradient's operand dZ that is the bias gradient, which took a launch of
+// its own and another pass over dZ (14 of a training step's 159 us).
 // AV, BV: the operand's k are consecutive and aligned (Frag).
 //
 // Bound by the latency of its loads: the matrix work of a layer is under a microsecond, its
@@ -87,16 +100,13 @@ struct Frag {
 // loads of four steps of 32 k (two for T = 2) are issued together, 16 bytes each where the layout allows,
 // and small products take T = 1, four times as many waves (use_small_tiles). The first layer of the 256-pulse network,
 // 256 x 128 x 1024, takes 15 us (95 with a step's loads waited for one by one and 32 x 32 tiles),
-// the training step's products 80 instead of 406.
+// the training step's products 61 instead of 406.
 template <typename TA, typename TB, int EPI, int T, bool AV, bool BV>
-__global__ __launch_bounds__(64) void k_gemm_bf16(int m, int n, int k, const TA* __restrict__ a, long sam, long sak,
-                                                  const TB* __restrict__ b, long sbk, long sbn, float* __restrict__ c,
-                                                  long scm, const float* __restrict__ bias,
-                                                  const float* __restrict__ mask, long smm,
-                                                  float* __restrict__ colsum) {
+__device__ __forceinline__ void gemm_block(const GemmArgs<TA, TB>& G, int bx, int by) {
+    const int m = G.m, n = G.n, k = G.k;
     constexpr int kTile = 16 * T, kSteps = T == 1 ? 4 : 2;
     const int l = threadIdx.x;
-    const int bm = blockIdx.y * kTile, bn = blockIdx.x * kTile;
+    const int bm = by * kTile, bn = bx * kTile;
     const int li = l % 16, lk = 8 * (l / 16), lr = 4 * (l / 16);
     f32x4 acc[T][T];
 #pragma unroll
@@ -114,8 +124,8 @@ __global__ __launch_bounds__(64) void k_gemm_bf16(int m, int n, int k, const TA*
             const int kk = k0 + 32 * q + lk;
 #pragma unroll
             for (int i = 0; i < T; ++i) {
-                fa[q][i].load(a, bm + 16 * i + li, m, sam, kk, k, sak);
-                fb[q][i].load(b, bn + 16 * i + li, n, sbn, kk, k, sbk);
+                fa[q][i].load(G.a, bm + 16 * i + li, m, G.sam, kk, k, G.sak);
+                fb[q][i].load(G.b, bn + 16 * i + li, n, G.sbn, kk, k, G.sbk);
             }
         }
         issue_point();
@@ -147,23 +157,41 @@ __global__ __launch_bounds__(64) void k_gemm_bf16(int m, int n, int k, const TA*
                 const int row = bm + 16 * i + lr + t;
                 if (row >= m) continue;
                 float v = acc[i][j][t];
-                if constexpr (EPI == 1) v = fmaxf(v + bias[col], 0.0f);
-                if constexpr (EPI == 2) v += bias[col];
-                if constexpr (EPI == 3) v = mask[row * smm + col] > 0.0f ? v : 0.0f;
-                c[row * scm + col] = v;
+                if constexpr (EPI == 1) v = fmaxf(v + G.bias[col], 0.0f);
+                if constexpr (EPI == 2) v += G.bias[col];
+                if constexpr (EPI == 3) v = G.mask[row * G.smm + col] > 0.0f ? v : 0.0f;
+                G.c[row * G.scm + col] = v;
             }
         }
     if constexpr (EPI == 0) {
-        if (blockIdx.y == 0) {
+        if (by == 0) {
 #pragma unroll
             for (int i = 0; i < T; ++i) {   // the four groups of 16 lanes hold every fourth eight of k
                 cs[i] += lane_xor<32>(cs[i]);
                 cs[i] += lane_xor<16>(cs[i]);
                 const int col = bn + 16 * i + li;
-                if (l < 16 && col < n) colsum[col] = cs[i];
+                if (l < 16 && col < n) G.colsum[col] = cs[i];
             }
         }
     }
+}
+
+}  // namespace
+
+template <typename TA, typename TB, int EPI, int T, bool AV, bool BV>
+__global__ __launch_bounds__(64) void k_gemm_bf16(GemmArgs<TA, TB> G) {
+    gemm_block<TA, TB, EPI, T, AV, BV>(G, blockIdx.x, blockIdx.y);
+}
+
+// The two products of a layer's backward pass that read dZ and do not depend on each other, in one
+// launch: the first `first` workgroups form the weight (and bias) gradient, across_dw to a row of
+// blocks, the rest dZ W^T.
+template <bool VEC>
+__global__ __launch_bounds__(64) void k_gemm_backward(GemmArgs<float, float> dw, GemmArgs<float, uint16_t> dx, int first,
+                                                      int across_dw, int across_dx) {
+    const int b = blockIdx.x;
+    if (b < first) gemm_block<float, float, 0, 1, false, false>(dw, b % across_dw, b / across_dw);
+    else gemm_block<float, uint16_t, 3, 1, VEC, VEC>(dx, (b - first) % across_dx, (b - first) / across_dx);
 }
 
 // Adam (bias-corrected) on FP32 master parameters; the BF16 copy of each weight follows.
@@ -397,16 +425,16 @@ bool vector_k(const T* p, long s_k, long s_line, int k) {
 
 // AK, BK: the callers' layouts have consecutive k in that operand; both must be readable so, or
 // neither is.
+template <bool AK, bool BK, typename TA, typename TB>
+bool vector_both(const GemmArgs<TA, TB>& G) {
+    return (AK || BK) && (!AK || vector_k(G.a, G.sak, G.sam, G.k)) && (!BK || vector_k(G.b, G.sbk, G.sbn, G.k));
+}
 template <typename TA, typename TB, int EPI, bool AK, bool BK>
-void gemm_bf16(int m, int n, int k, const TA* a, long sam, long sak, const TB* b, long sbk, long sbn, float* c, long scm,
-               const float* bias, const float* mask, long smm, float* colsum, hipStream_t s) {
-    const bool small = use_small_tiles(m, n);
-    const bool vec = (AK || BK) && (!AK || vector_k(a, sak, sam, k)) && (!BK || vector_k(b, sbk, sbn, k));
+void gemm_bf16(const GemmArgs<TA, TB>& G, hipStream_t s) {
+    const bool small = use_small_tiles(G.m, G.n), vec = vector_both<AK, BK>(G);
     const int tile = small ? 16 : 32;
-    const dim3 grid((n + tile - 1) / tile, (m + tile - 1) / tile);
-#define ISAR_GEMM(T, AV, BV)                                                                                           \
-    ISAR_LAUNCH((k_gemm_bf16<TA, TB, EPI, T, AV, BV>), grid, dim3(64), 0, s, m, n, k, a, sam, sak, b, sbk, sbn, c, scm, \
-                bias, mask, smm, colsum)
+    const dim3 grid((G.n + tile - 1) / tile, (G.m + tile - 1) / tile);
+#define ISAR_GEMM(T, AV, BV) ISAR_LAUNCH((k_gemm_bf16<TA, TB, EPI, T, AV, BV>), grid, dim3(64), 0, s, G)
     if (vec) {
         if (small) ISAR_GEMM(1, AK, BK);
         else ISAR_GEMM(2, AK, BK);
@@ -418,18 +446,34 @@ void gemm_bf16(int m, int n, int k, const TA* a, long sam, long sak, const TB* b
 }
 }  // namespace
 
-void launch_gemm_f32_bf16w(int m, int n, int k, const float* a, long sam, long sak, const uint16_t* w, long sbk,
-                           long sbn, float* c, long scm, const float* bias, int relu, hipStream_t s) {
-    if (relu) gemm_bf16<float, uint16_t, 1, true, false>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, bias, nullptr, 0L, nullptr, s);
-    else gemm_bf16<float, uint16_t, 2, true, false>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, bias, nullptr, 0L, nullptr, s);
+void launch_dense_forward(int batch, int in, int out, const float* a, const uint16_t* w, const float* bias, float* z,
+                          int relu, hipStream_t s) {
+    const GemmArgs<float, uint16_t> G{batch, out, in, a, in, 1, w, out, 1, z, out, bias, nullptr, 0, nullptr};
+    if (relu) gemm_bf16<float, uint16_t, 1, true, false>(G, s);
+    else gemm_bf16<float, uint16_t, 2, true, false>(G, s);
 }
-void launch_gemm_f32_bf16w_masked(int m, int n, int k, const float* a, long sam, long sak, const uint16_t* w,
-                                  long sbk, long sbn, float* c, long scm, const float* mask, long smm, hipStream_t s) {
-    gemm_bf16<float, uint16_t, 3, true, true>(m, n, k, a, sam, sak, w, sbk, sbn, c, scm, nullptr, mask, smm, nullptr, s);
-}
-void launch_gemm_f32_f32(int m, int n, int k, const float* a, long sam, long sak, const float* b, long sbk, long sbn,
-                         float* c, long scm, float* colsum, hipStream_t s) {
-    gemm_bf16<float, float, 0, false, false>(m, n, k, a, sam, sak, b, sbk, sbn, c, scm, nullptr, nullptr, 0L, colsum, s);
+void launch_dense_backward(int batch, int in, int out, const float* a, const float* dz, const uint16_t* w, float* dw,
+                           float* db, float* da, hipStream_t s) {
+    // dW = A^T dZ (in x out), db = column sums of dZ; dA = dZ W^T where A > 0
+    const GemmArgs<float, float> W{in, out, batch, a, 1, in, dz, out, 1, dw, out, nullptr, nullptr, 0, db};
+    if (!da) {
+        gemm_bf16<float, float, 0, false, false>(W, s);
+        return;
+    }
+    const GemmArgs<float, uint16_t> A{batch, in, out, dz, out, 1, w, 1, out, da, in, nullptr, a, in, nullptr};
+    // One launch while both take 16 x 16 tiles: a layer of the 256-pulse network at batch 256 takes 6.5 us, two
+    // launches took 10.5.
+    if (use_small_tiles(W.m, W.n) && use_small_tiles(A.m, A.n)) {
+        const int xw = (W.n + 15) / 16, xa = (A.n + 15) / 16;
+        const int first = xw * ((W.m + 15) / 16), rest = xa * ((A.m + 15) / 16);
+        if (vector_both<true, true>(A))
+            ISAR_LAUNCH(k_gemm_backward<true>, dim3(first + rest), dim3(64), 0, s, W, A, first, xw, xa);
+        else
+            ISAR_LAUNCH(k_gemm_backward<false>, dim3(first + rest), dim3(64), 0, s, W, A, first, xw, xa);
+        return;
+    }
+    gemm_bf16<float, float, 0, false, false>(W, s);
+    gemm_bf16<float, uint16_t, 3, true, true>(A, s);
 }
 void launch_adam(int n, float* p, const float* g, float* m1, float* m2, uint16_t* pb, const int* bf_index, float lr,
                  float beta1, float beta2, float eps, float c1, float c2, hipStream_t s) {

@@ -51,12 +51,10 @@ bool pulse_compress_supported(int nfft);
 void launch_pulse_compress(const PcJob& P, int nfft, hipStream_t s);
 
 // learned warm start: BF16 matrix-core GEMMs with FP32 accumulation and their helpers
-void launch_gemm_f32_bf16w(int m, int n, int k, const float* a, long sam, long sak, const uint16_t* w, long sbk,
-                           long sbn, float* c, long scm, const float* bias, int relu, hipStream_t s);
-void launch_gemm_f32_bf16w_masked(int m, int n, int k, const float* a, long sam, long sak, const uint16_t* w,
-                                  long sbk, long sbn, float* c, long scm, const float* mask, long smm, hipStream_t s);
-void launch_gemm_f32_f32(int m, int n, int k, const float* a, long sam, long sak, const float* b, long sbk, long sbn,
-                         float* c, long scm, float* colsum, hipStream_t s);
+void launch_dense_forward(int batch, int in, int out, const float* a, const uint16_t* w, const float* bias, float* z,
+                          int relu, hipStream_t s);
+void launch_dense_backward(int batch, int in, int out, const float* a, const float* dz, const uint16_t* w, float* dw,
+                           float* db, float* da, hipStream_t s);   // da: null for the first layer
 void launch_adam(int n, float* p, const float* g, float* m1, float* m2, uint16_t* pb, const int* bf_index, float lr,
                  float beta1, float beta2, float eps, float c1, float c2, hipStream_t s);
 void launch_to_bf16(int n, const float* p, uint16_t* pb, const int* bf_index, hipStream_t s);

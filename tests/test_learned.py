@@ -132,6 +132,15 @@ def test_network_forward_and_gradients_match_oracle(widths, batch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("widths,batch", [([21, 13, 30, 9], 19), ([16, 1024, 1024], 130)])
+def test_backward_launch_forms_match_oracle(widths, batch):
+    """A layer's two backward products in one launch with single loads (odd widths), and in launches of
+    their own where one of them takes the larger tiles (1024 x 1024 weights), to the bounds of
+    test_network_forward_and_gradients_match_oracle."""
+    test_network_forward_and_gradients_match_oracle(widths, batch)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("widths,batch", [([8, 8], 1), ([13, 70], 5), ([136, 1030], 1030), ([24, 1024], 1024),
                                           ([520, 17], 33)])
 def test_one_layer_products_at_tile_edges_match_oracle(widths, batch):
