@@ -180,18 +180,6 @@ __device__ __forceinline__ void wave_arg(float& v, int& i) {
 // Workgroup-wide reductions through a small LDS scratch (>= 16 slots). All threads get the
 // result. Must be called by every thread of the workgroup.
 template <int NT>
-__device__ __forceinline__ float block_sum(float v, float* red) {
-    v = wave_sum(v);
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    __syncthreads();
-    if (l == 0) red[w] = v;
-    __syncthreads();
-    float r = 0.f;
-#pragma unroll
-    for (int i = 0; i < NT / 64; ++i) r += red[i];
-    return r;
-}
-template <int NT>
 __device__ __forceinline__ long long block_sum_i64(long long v, long long* red) {
     v = group_combine<64>(v, [](long long a, long long b) { return a + b; });
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -425,9 +413,10 @@ struct ColCfg {
     __device__ static int out(int lane, int e) { return fft_out_pos<M, E>(lane, e); }
 };
 
-// Copies columns n0 ... n0 + CT - 1 of rows 0 ... M - 1 of a row-major matrix of W columns into LDS, element
-// (m, c) at sm[m (CT + 1) + c], by NT threads with eight loads of a thread in flight: the column kernels wait for
-// this tile before anything else, and with a load at a time that wait was most of their time.
+// Copies columns n0 ... n0 + CT - 1 of rows 0 ... M - 1 of a row-major matrix of W columns into LDS,
+// element (m, c) at sm[m (CT + 1) + c], by NT threads with eight loads of a thread in flight: the
+// column kernels wait for this tile before anything else, and with a load at a time that wait was
+// most of their time.
 template <int NT, int CT>
 __device__ __forceinline__ void load_column_tile(const float2* src, int W, int n0, int M, float2* sm, int tid) {
     const int total = M * CT;
@@ -453,7 +442,8 @@ __device__ __forceinline__ void load_column_tile(const float2* src, int W, int n
 // sc1 set, which are written through to the device's point of coherence and read from it, never
 // from a stale line of another XCD's L2. A word is empty until its value is stored, and a reader
 // polls it until it is not, so nothing but the value itself has to arrive; a word that is used again
-// is emptied first, and that store waited for (s_waitcnt 0). No fence, L2 write-back or invalidation is involved.
+// is emptied first, and that store waited for (s_waitcnt 0). No fence, L2 write-back or invalidation
+// is involved.
 // ------------------------------------------------------------------------------------------
 constexpr uint64_t kXwgEmpty = ~0ull;   // two NaNs
 __device__ __forceinline__ uint64_t xwg_word(float2 v) {

@@ -98,8 +98,8 @@ struct GemmArgs {
 // Bound by the latency of its loads: the matrix work of a layer is under a microsecond, its
 // operands are in the L2, and the sums follow k, so that a wave has a serial chain over k. So the
 // loads of four steps of 32 k (two for T = 2) are issued together, 16 bytes each where the layout allows,
-// and small products take T = 1, four times as many waves (use_small_tiles). The first layer of the 256-pulse network,
-// 256 x 128 x 1024, takes 15 us (95 with a step's loads waited for one by one and 32 x 32 tiles),
+// and small products take T = 1, four times as many waves (use_small_tiles). The first layer of the
+// 256-pulse network, 256 x 128 x 1024, takes 15 us (95 with a step's loads waited for one by one and 32 x 32 tiles),
 // the training step's products 61 instead of 406.
 template <typename TA, typename TB, int EPI, int T, bool AV, bool BV>
 __device__ __forceinline__ void gemm_block(const GemmArgs<TA, TB>& G, int bx, int by) {

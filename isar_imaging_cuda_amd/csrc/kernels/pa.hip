@@ -582,8 +582,8 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_cols(Job J
 }
 
 // Adds n sub-chunk sums of pulse m to acc in order, from exchange words M apart. They are loaded
-// together, and all again until none is empty. A thread that has polled more than `limit` times in a row gives
-// up for the rest of the launch (waiting = false) and sets status bit 2.
+// together, and all again until none is empty. A thread that has polled more than `limit` times in a
+// row gives up for the rest of the launch (waiting = false) and sets status bit 2.
 template <int M, int n>
 __device__ __forceinline__ void af_add_words(float2& acc, const uint64_t* w, int limit, bool& waiting, int32_t& status) {
     uint64_t v[n];

@@ -248,7 +248,8 @@ __device__ int correlation_argmax(const float (&a)[kE], const float (&b)[kE], fl
 
 // sqrt(x) to about 1e-14 relative for x >= 0: the hardware FP32 root (within 1 ulp) refined by one
 // Newton step in FP64, s + (x - s^2) / (2 s); the step's own factor 1 / (2 s) needs only the
-// hardware reciprocal's accuracy (1 ulp). A few FP64 operations instead of the long correctly rounded FP64 square root.
+// hardware reciprocal's accuracy (1 ulp). A few FP64 operations instead of the long correctly rounded
+// FP64 square root.
 __device__ __forceinline__ double sqrt_refined(float x) {
     const float s = sqrt_hw(x);
     const double sd = static_cast<double>(s);
@@ -261,8 +262,9 @@ __device__ __forceinline__ double sqrt_refined(float x) {
 // not read from the FP32 transform: near a broad peak the second
 // difference f1 + f3 - 2 f2 cancels most of its digits, and the transform's rounding alone moved
 // the vertex by up to 2.4e-4 cell at 1024 x 16384, which 120 autofocus iterations amplify into a
-// 1e-3 image difference. The vertex and the lag are FP64. a, b: the two energy profiles. Must follow correlation_argmax (its barriers end the LDS use). Thread 0 records
-// the lag and argmax; every thread gets the lag.
+// 1e-3 image difference. The vertex and the lag are FP64. a, b: the two energy profiles. Must follow
+// correlation_argmax (its barriers end the LDS use). Thread 0 records the lag and argmax; every thread
+// gets the lag.
 template <int N>
 __device__ double parabola_lag(const float (&a)[kE], const float (&b)[kE], int bi, float2* lds, int tid,
                                double* lag_out, int32_t* imax_out) {
@@ -352,7 +354,7 @@ __global__ __launch_bounds__(N / kE) void k_ifds_pre(Job J) {
 }
 
 // getHRRP for STRETCH (common.cu:561-571): ifftshift(FFT(hamming_N * row)) of the compensated
-// rows, one workgroup per row. The ifftshift is the (-1)^n modulation load_row_raw applies.
+// rows, one workgroup per row. The ifftshift is the (-1)^n modulation RowSamples applies.
 template <int N>
 __global__ __launch_bounds__(N / kE) void k_hrrp(Job J) {
     HIP_DYNAMIC_SHARED(float2, lds);
