@@ -308,9 +308,9 @@ __global__ void k_half_phase(int frames, int M, const float2* __restrict__ phi_a
     out[i] = cmul(a, h);
 }
 
-// ln of a positive normal double to about 2e-16 (absolute, beside the rounding of the result) by
-// table and series: with the mantissa in [1, 2) cut into 128 intervals, c_j about the reciprocal of
-// interval j's centre and r = mantissa c_j - 1, at most 1/256 in magnitude,
+// ln(q / 2^(k - 1023)) of a positive normal double to about 2e-16 (absolute, beside the rounding of the
+// result) by table and series: with the mantissa in [1, 2) cut into 128 intervals, c_j about the
+// reciprocal of interval j's centre and r = mantissa c_j - 1, at most 1/256 in magnitude,
 // ln q = e ln 2 - ln c_j + ln(1 + r). (P. T. P. Tang, "Table-driven implementation of the logarithm
 // function in IEEE floating-point arithmetic", 1990.)
 struct LogRow {
@@ -334,43 +334,59 @@ struct LogTable {
 };
 __constant__ const LogTable kLogTable{};
 
-__device__ __forceinline__ double log_by_table(double q, const LogRow* rows) {
+constexpr double kLn2 = 0.69314718055994530942;
+__device__ __forceinline__ int biased_exponent(double q) {   // q >= 0
+    return static_cast<int>(__builtin_bit_cast(uint64_t, q) >> 52);
+}
+__device__ __forceinline__ double log_by_table(double q, int k, const LogRow* rows) {
     const uint64_t bits = __builtin_bit_cast(uint64_t, q);
     const unsigned hi = static_cast<unsigned>(bits >> 32);
     const LogRow t = rows[(hi >> 13) & 127];
     const uint64_t mb = (static_cast<uint64_t>((hi & 0x000fffffu) | 0x3ff00000u) << 32) | (bits & 0xffffffffu);
     const double r = fma(__builtin_bit_cast(double, mb), t.c, -1.0);
-    const double e = static_cast<double>(static_cast<int>(hi >> 20) - 1023);
+    const double e = static_cast<double>(static_cast<int>(hi >> 20) - k);
     double y = fma(r, 1.0 / 7.0, -1.0 / 6.0);
     y = fma(y, r, 1.0 / 5.0);
     y = fma(y, r, -1.0 / 4.0);
     y = fma(y, r, 1.0 / 3.0);
     y = fma(y, r, -0.5);
     y = fma(y * r, r, r);
-    return fma(e, 0.69314718055994530942, t.ln_c) + y;
+    return fma(e, kLn2, t.ln_c) + y;
 }
 
-// Image entropy -sum p ln p, p = q / T, q = img^2, T = sum q, one workgroup per image, FP64 sums:
-// (T ln T - sum q ln q) / T, one pass over the image. A single bright cell gives 0 exactly, as both
-// terms are then the same product. Bound by the loads' latency and FP64 issue: 256 images of
-// 256 x 512 take 38 us (3.6 TB/s); with two passes, the library's logarithm and 256 threads an image
-// they took 475.
+// Image entropy -sum p ln p, p = q / T, q = img^2, T = sum q, one workgroup per image, FP64 sums, one pass
+// over the image: (T ln(T / r) - sum q ln(q / r)) / T for any r. With r = 1 both terms grow with ln T and
+// nearly cancel (amplitudes of 1e4: off by 7e-15, where -sum p ln p is off by 6e-16). So r is the power
+// of two of the largest q so far, per thread and then for all: raising it by 2^d takes T d ln 2 from the
+// second sum, and the terms that count have q near r. Off by as much as -sum p ln p or less
+// (131072 cells, amplitudes 1e-15 to 1e15), and the same bits for an image scaled by a power of two.
+// A single bright cell gives 0 exactly, as both terms are then the same product. Bound by the loads'
+// latency and FP64 issue: 256 images of 256 x 512 take 32 us (4.2 TB/s); 31 with r = 1, and 390 in two
+// passes with the library's logarithm and 256 threads an image.
+struct EntropySums {
+    double total, s;
+    int k;   // biased exponent of r; 0: no q yet
+    __device__ __forceinline__ void raise(int to) {
+        s = fma(total, static_cast<double>(k - to) * kLn2, s);
+        k = to;
+    }
+    __device__ __forceinline__ void add(double q, const LogRow* rows) {   // q is a float's square: normal or 0
+        total += q;
+        s = fma(q, log_by_table(q, k, rows), s);   // 0 where q = 0: the logarithm is finite there
+    }
+};
 constexpr int kEntropyThreads = 1024;
 __global__ __launch_bounds__(kEntropyThreads) void k_image_entropy(int n, const float* __restrict__ img,
                                                                    double* __restrict__ out) {
     constexpr int NT = kEntropyThreads;
     __shared__ LogRow rows[128];
-    __shared__ double red[2][NT / 64];
+    __shared__ EntropySums red[NT / 64];
     const int f = blockIdx.x, tid = threadIdx.x;
     const float* x = img + static_cast<size_t>(f) * n;
     if (tid < 128) rows[tid] = kLogTable.row[tid];
     __syncthreads();
-    double total = 0.0, s = 0.0;
-    auto add = [&](float v) {
-        const double q = static_cast<double>(v) * v;   // normal or 0 for any float
-        total += q;
-        s = fma(q, log_by_table(q, rows), s);          // 0 where q = 0: the logarithm is finite there
-    };
+    EntropySums a{0.0, 0.0, 0};
+    auto square = [](float v) { return static_cast<double>(v) * v; };
     constexpr int kLoads = 8;
     int i = tid;
     for (; i + (kLoads - 1) * NT < n; i += kLoads * NT) {
@@ -378,29 +394,38 @@ __global__ __launch_bounds__(kEntropyThreads) void k_image_entropy(int n, const 
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) v[u] = x[i + u * NT];
         issue_point();
+        int top = a.k;
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u) add(v[u]);
+        for (int u = 0; u < kLoads; ++u) top = max(top, biased_exponent(square(v[u])));
+        a.raise(top);
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) a.add(square(v[u]), rows);
     }
-    for (; i < n; i += NT) add(x[i]);
-    total = wave_sum_d(total);
-    s = wave_sum_d(s);
-    if (tid % 64 == 0) {
-        red[0][tid / 64] = total;
-        red[1][tid / 64] = s;
+    for (; i < n; i += NT) {
+        const double q = square(x[i]);
+        a.raise(max(a.k, biased_exponent(q)));
+        a.add(q, rows);
     }
+    a.raise(group_combine<64>(a.k, [](int p, int q) { return max(p, q); }));
+    a.total = wave_sum_d(a.total);
+    a.s = wave_sum_d(a.s);
+    if (tid % 64 == 0) red[tid / 64] = a;
     __syncthreads();
     if (tid == 0) {
-        total = 0.0;
-        s = 0.0;
+        int k = 0;
+        for (int w = 0; w < NT / 64; ++w) k = max(k, red[w].k);
+        EntropySums all{0.0, 0.0, 0};
         for (int w = 0; w < NT / 64; ++w) {
-            total += red[0][w];
-            s += red[1][w];
+            EntropySums p = red[w];
+            p.raise(k);
+            all.total += p.total;
+            all.s += p.s;
         }
         // no entropy where the image is all zero, or its energy infinite or NaN; the difference's
         // rounding may leave a hair below 0
-        const bool any = total > 0.0 && total <= 1.7976931348623157e308;
-        const double tl = opaque(total * log_by_table(total, rows));   // rounded by itself, as s is
-        out[f] = any ? fmax((tl - s) / total, 0.0) : 0.0;
+        const bool any = all.total > 0.0 && all.total <= 1.7976931348623157e308;
+        const double tl = opaque(all.total * log_by_table(all.total, k, rows));   // rounded by itself, as s is
+        out[f] = any ? fmax((tl - all.s) / all.total, 0.0) : 0.0;
     }
 }
 

@@ -272,6 +272,33 @@ def test_image_entropy_lengths_and_scales(n):
         assert abs(e - ref) <= bound, (scales[k], e, ref)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 300, 8191, 8193, 131072])
+def test_image_entropy_keeps_its_bits_under_scaling(n):
+    """-sum p ln p with p = q / sum q does not change at all when an image is multiplied by a power of two:
+    every product, sum and quotient scales exactly. So the entropy's rounding may not depend on the
+    level of the image, and at any level it is that of numbers of the size of H."""
+    torch = _torch()
+    from isar_imaging_cuda_amd import learned as L
+    rng = np.random.default_rng(n)
+    base = np.abs(rng.standard_normal(n)).astype(np.float32)
+    base[::97] += 300.0   # bright points
+    exponents = (0, 1, 13, -13, 27, 40, -60, 100)
+    imgs = np.stack([np.ldexp(base, e).astype(np.float32) for e in exponents])
+    d = torch.from_numpy(imgs).to("cuda:0")
+    out = torch.zeros(len(exponents), dtype=torch.float64, device="cuda:0")
+    L.image_entropy(len(exponents), n, d.data_ptr(), out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    e = out.cpu().numpy()
+    q = base.astype(np.longdouble) ** 2
+    p = q / q.sum()
+    ref = float(-(p * np.log(p)).sum())
+    assert np.all(e == e[0]), dict(zip(exponents, e - e[0]))
+    # two terms below H + ln 4n each, rounded, and sums of n / 1024 + 26 additions of non-negative parts
+    bound = (n / 1024 + 30) * 2.0 ** -53 * 2 * (ref + float(np.log(4.0 * n)))
+    assert abs(e[0] - ref) <= bound, (e[0], ref)
+
+
 def _c4_batch(K, seed0):
     from isar_imaging_cuda_amd import learned as L
     echo, vel, h = L.synth_frames(4, list(range(seed0, seed0 + K)))
