@@ -361,12 +361,14 @@ __device__ __forceinline__ double log_by_table(double q, int k, const LogRow* ro
 // second sum, and the terms that count have q near r. Off by as much as -sum p ln p or less
 // (131072 cells, amplitudes 1e-15 to 1e15), and the same bits for an image scaled by a power of two.
 // A single bright cell gives 0 exactly, as both terms are then the same product. Bound by the loads'
-// latency and FP64 issue: 256 images of 256 x 512 take 32 us (4.2 TB/s); 31 with r = 1, and 390 in two
-// passes with the library's logarithm and 256 threads an image.
+// latency and FP64 issue: 256 images of 256 x 512 take 34 us (3.9 TB/s), 1024 of them 121; 32 and 112
+// with r = 1; 34 and 132 with the registers left free, as a CU then holds one workgroup; 390 the 256 in
+// two passes with the library's logarithm.
 struct EntropySums {
     double total, s;
     int k;   // biased exponent of r; 0: no q yet
     __device__ __forceinline__ void raise(int to) {
+        if (to <= k) return;
         s = fma(total, static_cast<double>(k - to) * kLn2, s);
         k = to;
     }
@@ -375,12 +377,11 @@ struct EntropySums {
         s = fma(q, log_by_table(q, k, rows), s);   // 0 where q = 0: the logarithm is finite there
     }
 };
-constexpr int kEntropyThreads = 1024;
-__global__ __launch_bounds__(kEntropyThreads) void k_image_entropy(int n, const float* __restrict__ img,
-                                                                   double* __restrict__ out) {
-    constexpr int NT = kEntropyThreads;
+template <int NT>
+__global__ __launch_bounds__(NT, 8) void k_image_entropy(int n, const float* __restrict__ img, double* __restrict__ out) {
+    constexpr int WAVES = NT / 64;
     __shared__ LogRow rows[128];
-    __shared__ EntropySums red[NT / 64];
+    __shared__ EntropySums red[WAVES];
     const int f = blockIdx.x, tid = threadIdx.x;
     const float* x = img + static_cast<size_t>(f) * n;
     if (tid < 128) rows[tid] = kLogTable.row[tid];
@@ -394,38 +395,35 @@ __global__ __launch_bounds__(kEntropyThreads) void k_image_entropy(int n, const 
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) v[u] = x[i + u * NT];
         issue_point();
-        int top = a.k;
+        float top = 0.0f;
 #pragma unroll
-        for (int u = 0; u < kLoads; ++u) top = max(top, biased_exponent(square(v[u])));
-        a.raise(top);
+        for (int u = 0; u < kLoads; ++u) top = fmaxf(top, fabsf(v[u]));
+        a.raise(biased_exponent(square(top)));
 #pragma unroll
         for (int u = 0; u < kLoads; ++u) a.add(square(v[u]), rows);
     }
     for (; i < n; i += NT) {
         const double q = square(x[i]);
-        a.raise(max(a.k, biased_exponent(q)));
+        a.raise(biased_exponent(q));
         a.add(q, rows);
     }
-    a.raise(group_combine<64>(a.k, [](int p, int q) { return max(p, q); }));
-    a.total = wave_sum_d(a.total);
-    a.s = wave_sum_d(a.s);
+    auto combine = [&]<int WIDTH>() {
+        a.raise(group_combine<WIDTH>(a.k, [](int p, int q) { return max(p, q); }));
+        a.total = group_combine<WIDTH>(a.total, [](double p, double q) { return p + q; });
+        a.s = group_combine<WIDTH>(a.s, [](double p, double q) { return p + q; });
+    };
+    combine.template operator()<64>();
     if (tid % 64 == 0) red[tid / 64] = a;
     __syncthreads();
+    if (tid >= 64) return;
+    a = red[tid % WAVES];
+    combine.template operator()<WAVES>();
     if (tid == 0) {
-        int k = 0;
-        for (int w = 0; w < NT / 64; ++w) k = max(k, red[w].k);
-        EntropySums all{0.0, 0.0, 0};
-        for (int w = 0; w < NT / 64; ++w) {
-            EntropySums p = red[w];
-            p.raise(k);
-            all.total += p.total;
-            all.s += p.s;
-        }
         // no entropy where the image is all zero, or its energy infinite or NaN; the difference's
         // rounding may leave a hair below 0
-        const bool any = all.total > 0.0 && all.total <= 1.7976931348623157e308;
-        const double tl = opaque(all.total * log_by_table(all.total, k, rows));   // rounded by itself, as s is
-        out[f] = any ? fmax((tl - all.s) / all.total, 0.0) : 0.0;
+        const bool any = a.total > 0.0 && a.total <= 1.7976931348623157e308;
+        const double tl = opaque(a.total * log_by_table(a.total, a.k, rows));   // rounded by itself, as s is
+        out[f] = any ? fmax((tl - a.s) / a.total, 0.0) : 0.0;
     }
 }
 
@@ -531,8 +529,13 @@ void launch_accept_image(int frames, int n, const float* img_a, const double* en
     ISAR_LAUNCH(k_accept_image, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, s, frames, n, img_a,
                 ent_a, img_b, ent_b, rel_tol, out, accepted);
 }
+// 1024 threads an image from 8192 cells on, where every thread has a whole group of loads, 256 below:
+// 2000 images of 100 cells take 4.5 us (10.4 with 1024 threads), 1024 of 1000 cells 4.3 (6.1), of 8192
+// cells 10.1 (11.3); but one image of 16384 cells 7.0 (5.5), 256 of 32768 14 (10).
+constexpr int kEntropyWideCells = 8192;
 void launch_image_entropy(int frames, int n, const float* img, double* out, hipStream_t s) {
-    ISAR_LAUNCH(k_image_entropy, dim3(frames), dim3(kEntropyThreads), 0, s, n, img, out);
+    if (n < kEntropyWideCells) ISAR_LAUNCH(k_image_entropy<256>, dim3(frames), dim3(256), 0, s, n, img, out);
+    else ISAR_LAUNCH(k_image_entropy<1024>, dim3(frames), dim3(1024), 0, s, n, img, out);
 }
 
 }  // namespace isar
