@@ -471,6 +471,13 @@ __device__ __forceinline__ uint64_t xwg_load(const uint64_t* p) {
 #endif
 }
 // Waits until this thread's stores are acknowledged.
+__device__ __forceinline__ int32_t xwg_load(const int32_t* p) {
+#ifdef ISAR_EMU
+    return __atomic_load_n(p, __ATOMIC_SEQ_CST);
+#else
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#endif
+}
 __device__ __forceinline__ void xwg_stores_done() {
 #ifdef ISAR_EMU
     __atomic_thread_fence(__ATOMIC_SEQ_CST);
@@ -482,6 +489,7 @@ __device__ __forceinline__ void xwg_stores_done() {
 }
 __device__ __forceinline__ void xwg_pause() {
 #ifdef ISAR_EMU
+    ++isar_emu::pauses;
     std::this_thread::yield();
 #else
     __builtin_amdgcn_s_sleep(2);

@@ -1,7 +1,10 @@
 // emu_driver.cpp — runs the kernel sources on the CPU (hip_emu.hpp) through the same C ABI as
 // the device library. Test infrastructure: built with AddressSanitizer by the CPU test suite.
 //
-// usage: isar_emu_driver <input.bin> <output.bin> [autofocus_mode [ra_split [static [czt_length [czt_threads]]]]]
+// usage: isar_emu_driver <input.bin> <output.bin> [autofocus_mode [ra_split [static [czt_length [czt_threads
+//                        [af_wait_polls late_block]]]]]]
+// late_block: a workgroup of the resident autofocus's grid that is run after the others have ended; the
+// pauses of its waits are printed.
 // static = 1: also images the batch, then its first frame alone, through isar_run_device_static
 // and requires both to equal the context's images bit for bit (exit 10-12 otherwise).
 // input : int32 M, N, W, K; int64 band_width, fc; double Tp; int64 Fs; isar_options;
@@ -13,12 +16,13 @@
 #include <cstdlib>
 #include <vector>
 
+#include "emu/hip_emu.hpp"
 #include "isar_imaging_ext.h"
 
 int main(int argc, char** argv) {
-    if (argc < 3 || argc > 8) {
-        std::fprintf(stderr, "usage: %s input.bin output.bin [autofocus_mode [ra_split [static [czt_length [czt_threads]]]]]\n",
-                     argv[0]);
+    if (argc < 3 || argc > 10) {
+        std::fprintf(stderr, "usage: %s input.bin output.bin [autofocus_mode [ra_split [static [czt_length [czt_threads "
+                     "[af_wait_polls late_block]]]]]]\n", argv[0]);
         return 2;
     }
     FILE* in = std::fopen(argv[1], "rb");
@@ -60,11 +64,16 @@ int main(int argc, char** argv) {
         std::fprintf(stderr, "chirp-z threads: %s\n", isar_last_error());
         return 6;
     }
+    if (argc == 10) {
+        (void)isar_set_af_wait_polls(ctx, std::atoi(argv[8]));
+        isar_emu::late_block = std::atoi(argv[9]);
+    }
     std::vector<float> img(static_cast<size_t>(K) * M * W);
     if (isar_run_host(ctx, K, echo.data(), vel.data(), opt.warm_start ? phi0.data() : nullptr, img.data(), &opt) != 0) {
         std::fprintf(stderr, "run: %s\n", isar_last_error());
         return 7;
     }
+    if (argc == 10) std::printf("late pauses %ld\n", isar_emu::late_pauses);
     if (argc >= 6 && std::atoi(argv[5]) == 1) {
         // the emulated device memory is host memory: the host arrays serve as device buffers
         std::vector<float> img_s(img.size());

@@ -198,7 +198,12 @@ inline void launch(K kernel, dim3 grid, dim3 block, size_t smem, A... args) {
                 for (auto& x : th) x.join();
             }
 }
-// Runs all blocks of the grid concurrently, each with its own LDS and barrier.
+// Runs all blocks of the grid concurrently, each with its own LDS and barrier; block `late_block` (none if
+// negative) only after the others have ended, as a GPU that has no room for it would. The waits' pauses
+// of that block are counted.
+inline int late_block = -1;
+inline std::atomic<long> pauses{0};
+inline long late_pauses = 0;
 template <typename K, typename... A>
 inline void launch_all(K kernel, dim3 grid, dim3 block, size_t smem, A... args) {
     const unsigned nt = block.x * block.y * block.z;
@@ -208,8 +213,7 @@ inline void launch_all(K kernel, dim3 grid, dim3 block, size_t smem, A... args) 
     std::vector<std::unique_ptr<std::barrier<>>> bars;
     for (unsigned b = 0; b < nb; ++b) bars.emplace_back(std::make_unique<std::barrier<>>(static_cast<std::ptrdiff_t>(nt)));
     std::vector<std::thread> th;
-    th.reserve(static_cast<size_t>(nb) * nt);
-    for (unsigned b = 0; b < nb; ++b) {
+    auto start = [&](unsigned b) {
         const unsigned bx = b % grid.x, by = (b / grid.x) % grid.y, bz = b / (grid.x * grid.y);
         for (unsigned t = 0; t < nt; ++t) {
             th.emplace_back([&, b, bx, by, bz, t]() {
@@ -221,8 +225,22 @@ inline void launch_all(K kernel, dim3 grid, dim3 block, size_t smem, A... args) 
                 kernel(args...);
             });
         }
+    };
+    auto join = [&] {
+        for (auto& x : th) x.join();
+        th.clear();
+    };
+    th.reserve(static_cast<size_t>(nb) * nt);
+    const unsigned late = late_block >= 0 ? static_cast<unsigned>(late_block) : nb;
+    for (unsigned b = 0; b < nb; ++b)
+        if (b != late) start(b);
+    join();
+    if (late < nb) {
+        const long before = pauses;
+        start(late);
+        join();
+        late_pauses += pauses - before;
     }
-    for (auto& x : th) x.join();
 }
 }  // namespace isar_emu
 

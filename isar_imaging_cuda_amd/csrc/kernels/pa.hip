@@ -451,6 +451,7 @@ __global__ __launch_bounds__(256) void k_af_start(Job J) {
     HIP_DYNAMIC_SHARED(double, scr);   // M (scan) + 32 (its partial sums), the phase (M float2)
     const int f = blockIdx.x, tid = threadIdx.x;
     float2* phi = reinterpret_cast<float2*>(scr + M + 32);
+    if (tid == 0) J.dec[f].status &= ~2;   // of an earlier run's autofocus
     if (J.phi0_given) {
         for (int m = tid; m < M; m += 256) phi[m] = J.phi0_in[static_cast<size_t>(f) * M + m];
         __syncthreads();
@@ -583,7 +584,9 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_cols(Job J
 
 // Adds n sub-chunk sums of pulse m to acc in order, from exchange words M apart. They are loaded
 // together, and all again until none is empty. A thread that has polled more than `limit` times in a
-// row gives up for the rest of the launch (waiting = false) and sets status bit 2.
+// row gives up (waiting = false) and sets status bit 2; one that waits looks for that bit every
+// kAfStatusPolls polls and gives up as well.
+constexpr int kAfStatusPolls = 64;
 template <int M, int n>
 __device__ __forceinline__ void af_add_words(float2& acc, const uint64_t* w, int limit, bool& waiting, int32_t& status) {
     uint64_t v[n];
@@ -597,6 +600,10 @@ __device__ __forceinline__ void af_add_words(float2& acc, const uint64_t* w, int
         if (polls >= limit) {
             waiting = false;
             atomicOr(&status, 2);
+            break;
+        }
+        if (polls % kAfStatusPolls == kAfStatusPolls - 1 && (xwg_load(&status) & 2)) {
+            waiting = false;
             break;
         }
         xwg_pause();
@@ -641,10 +648,14 @@ __device__ __forceinline__ float2 af_phase_from_words(const uint64_t* words, int
 //   later, so that wait costs nothing).
 // All of a frame's workgroups must be resident together; every XCD takes its share of a grid's
 // workgroups in order, so where the first incomplete frame lacks one, only complete frames are
-// ahead of it, and it completes as those finish. A wait that exceeds J.af_wait_polls polls (about a
-// second by default; a negative bound gives up at once) sets status bit 2 of the frame and stops
-// that thread waiting; the frame's phase is then not valid, and the default form does the frame
-// over with k_autofocus. Workgroup 0 of each frame writes the final phase to J.phi.
+// ahead of it, and it completes as those finish. That holds for one such grid on the GPU; two at once can
+// each hold what the other's frames lack. So a wait that exceeds J.af_wait_polls polls (about a
+// second by default; a negative bound gives up at once) sets status bit 2 of the frame, which
+// k_af_start cleared, and ends its workgroup. Once the bit is set the frame's other workgroups leave too:
+// those that wait within kAfStatusPolls polls, those placed later before their first transform. (The words
+// they would read are those of an iteration that the leavers never finished: each would wait its own
+// bound.) The frame's phase stays the starting phase, and the default form does the frame over with
+// k_autofocus. Otherwise workgroup 0 of each frame writes the final phase to J.phi.
 // Bound by the latency of an iteration (two transforms by one wave per SIMD, the sums, the
 // exchange): 3.6 us at 256 pulses, 6.1 at 512, whether the frames are 1 or 40, as long as every
 // workgroup has a CU for itself and the XCDs share the work (af_subchunk_of). At 256 pulses the
@@ -655,8 +666,9 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(J
     using A = AfCfg<M>;
     using C = ColCfg<M>;
     constexpr int E = A::E, TPF = A::TPF, SUB = A::SUB, NTS = SUB * TPF;
-    HIP_DYNAMIC_SHARED(float2, bufs);   // SUB * lds_padded_size(M), then the phase (M)
+    HIP_DYNAMIC_SHARED(float2, bufs);   // SUB * lds_padded_size(M), then the phase (M) and a flag
     float2* phi = bufs + SUB * lds_padded_size(M);
+    int* const gone = reinterpret_cast<int*>(phi + M);   // the workgroup leaves
     const int f = blockIdx.y, tid = threadIdx.x;
     const int U = J.dec[f].unit2_num;
     const int nsub = (U + SUB - 1) / SUB;
@@ -667,14 +679,19 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(J
     const int u = c0 + tid / TPF, lane = tid % TPF;
     const bool valid = u < U;
     const float2* col = J.su + static_cast<size_t>(f) * W * M + static_cast<size_t>(valid ? u : 0) * M;
+    int32_t& status = J.dec[f].status;
+    if (tid == 0) {
+        if (J.af_wait_polls < 0) atomicOr(&status, 2);   // a negative bound: every wait gives up
+        *gone = (xwg_load(&status) & 2) != 0;
+    }
     const AfTwiddles<M> tw(lane);
     float2 s[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) s[e] = valid ? col[C::in(lane, e)] : make_float2(0.0f, 0.0f);
     for (int m = tid; m < M; m += NTS) phi[m] = J.phi[static_cast<size_t>(f) * M + m];
     __syncthreads();
-    bool waiting = J.af_wait_polls >= 0;   // false once this thread's polls have hit their bound
-    if (!waiting && tid == 0) atomicOr(&J.dec[f].status, 2);   // a negative bound: every wait gives up
+    if (*gone) return;       // the whole workgroup
+    bool waiting = true;     // false once this thread has given up
     for (int it = 0; it < J.iterations; ++it) {
         uint64_t* const words = af_words_of<M>(J, f, it);
         uint64_t* const old = af_words_of<M>(J, f, it + 2) + static_cast<size_t>(j) * M;   // iteration it - 1
@@ -683,10 +700,12 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(J
             xwg_store(words + static_cast<size_t>(j) * M + m, xwg_word(t));
         });
         for (int m = tid; m < M; m += NTS) {
-            phi[m] = af_phase_from_words<M>(words, nsub, m, J.af_wait_polls, waiting, J.dec[f].status);
+            phi[m] = af_phase_from_words<M>(words, nsub, m, J.af_wait_polls, waiting, status);
             xwg_store(old + m, kXwgEmpty);
         }
+        if (!waiting) *gone = 1;
         __syncthreads();
+        if (*gone) return;   // the next write is behind af_subchunk's barrier
     }
     if (j == 0)
         for (int m = tid; m < M; m += NTS) J.phi[static_cast<size_t>(f) * M + m] = phi[m];
@@ -717,7 +736,7 @@ template <int M>
 size_t af_resident_lds(int frames) {
     const int groups = frames * (64 / AfCfg<M>::SUB);
     const size_t per_cu = (4 * groups + 3 * kComputeUnits - 1) / (3 * kComputeUnits);
-    return std::max(af_cols_lds<M>(true), kLdsBytes / (per_cu + 1) + 1024);
+    return std::max(af_cols_lds<M>(true) + sizeof(int), kLdsBytes / (per_cu + 1) + 1024);
 }
 template <int M>
 size_t colfft_lds() {

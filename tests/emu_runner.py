@@ -53,13 +53,15 @@ class EmuFrame:
 
 def run(echo: np.ndarray, velocity: np.ndarray, radar: dict, opts: dict | None = None, phi0=None,
         timeout: float = 900.0, autofocus_mode: int | None = None, ra_split: int | None = None,
-        static_check: bool = False, czt_length: int | None = None, czt_threads: int | None = None) -> list[EmuFrame]:
+        static_check: bool = False, czt_length: int | None = None, czt_threads: int | None = None,
+        late: tuple[int, int] | None = None, log: list | None = None) -> list[EmuFrame]:
     """echo: complex64 (K, M, N); velocity: (K, M). radar: band_width, fc, Tp, Fs.
     autofocus_mode: isar_autofocus_mode (0 auto, 1 one workgroup per frame, 2 split, 4 resident); ra_split:
     isar_set_ra_split (0 by batch size, 1 one grid, 2 two grids). static_check: the driver also
     images the batch and then its first frame through isar_run_device_static and fails unless both
     equal the context's images bit for bit. czt_length, czt_threads: isar_set_czt_length and
-    isar_set_czt_threads."""
+    isar_set_czt_threads. late: the resident autofocus's wait bound in polls and the workgroup of its grid
+    that runs after the others have ended; log then gets what the driver prints."""
     if not DRIVER.exists():
         raise RuntimeError(f"{DRIVER} missing: build with isar_imaging_cuda_amd/build.py --emu")
     opts = opts or default_options()
@@ -82,14 +84,16 @@ def run(echo: np.ndarray, velocity: np.ndarray, radar: dict, opts: dict | None =
             if opts.get("warm_start"):
                 f.write(np.ascontiguousarray(phi0, dtype=np.complex64).tobytes())
         # positional driver arguments; every one before the last given takes its default
-        args = [autofocus_mode, ra_split, 1 if static_check else None, czt_length, czt_threads]
-        defaults = [0, 0, 0, 0, 256]
+        args = [autofocus_mode, ra_split, 1 if static_check else None, czt_length, czt_threads, *(late or (None, None))]
+        defaults = [0, 0, 0, 0, 256, 0, -1]
         last = max((i for i, a in enumerate(args) if a is not None), default=-1)
         extra = [str(defaults[i] if args[i] is None else args[i]) for i in range(last + 1)]
         cmd = [str(DRIVER), str(fin), str(fout)] + extra
         r = subprocess.run(cmd, capture_output=True, text=True, timeout=timeout)
         if r.returncode != 0:
             raise RuntimeError(f"emu driver failed rc={r.returncode}\n{r.stdout}\n{r.stderr[-4000:]}")
+        if log is not None:
+            log.append(r.stdout)
         raw = fout.read_bytes()
     off = 0
 

@@ -83,3 +83,21 @@ def test_emulated_kernels_match_oracle(emu_driver):
     assert np.array_equal(one.img, two.img) and np.array_equal(one.ra_lag, two.ra_lag)
     resident = res["c1, two grids, resident autofocus"][0]
     assert resident.status & 2 == 0 and np.array_equal(resident.img, two.img)
+
+
+def test_resident_workgroup_placed_after_the_others_gave_up(emu_driver):
+    """A frame of the default autofocus one of whose workgroups finds no place until the others have
+    reached their bound (as where two such grids hold each other's places): the frame is marked, the
+    late workgroup leaves without waiting for sums that nobody will write, one workgroup does the frame
+    over, and phase and image are the one-workgroup form's."""
+    cfg = synth.preset(1, echo_num=64, range_num=1024)
+    echo, vel = synth.frame(cfg)
+    radar = synth.radar_header(cfg)
+    opts = emu_runner.default_options(iterations=ITERATIONS)
+    (ref,) = emu_runner.run(echo, vel, radar, opts, autofocus_mode=1, timeout=600)
+    assert ref.unit2_num >= 32   # two or more workgroups of 16 bins
+    log = []
+    (fr,) = emu_runner.run(echo, vel, radar, opts, autofocus_mode=0, late=(2000, 1), log=log, timeout=600)
+    assert "late pauses 0" in log[0].split("\n"), log
+    assert fr.status & 2 == 0
+    assert np.array_equal(fr.phi, ref.phi) and np.array_equal(fr.img, ref.img)
