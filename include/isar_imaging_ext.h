@@ -203,8 +203,8 @@ enum isar_autofocus_mode {
 };
 ISAR_API int isar_set_autofocus_mode(isar_context* ctx, int mode);
 ISAR_API int isar_get_autofocus_mode(isar_context* ctx);
-/* Bound of each wait of the resident autofocus, in polls of about a microsecond (default 2^20; in
- * AUTO at most 2^16);
+/* Bound of each wait of the resident autofocus, in polls of about a quarter of a microsecond
+ * (default 2^20; in AUTO at most 256 for each iteration and 16384 more, 12 ms at 120 iterations);
  * a negative bound makes every wait give up at once, which forces status bit 2 (for tests of the
  * fallback). */
 ISAR_API int isar_set_af_wait_polls(isar_context* ctx, int polls);

@@ -1,6 +1,8 @@
 // pipeline.cpp — imaging context and the batch launch sequence (isar_main.cu:3-227).
 #include "pipeline.hpp"
 
+#include "../autofocus_rules.hpp"
+
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -392,7 +394,7 @@ int Context::enqueue(int frames, const void* echo, const double* velocity, const
     const bool af_auto = af_mode == ISAR_AF_AUTO;
     const bool af_guarded = af_auto && af_auto_resident && frames <= kAfResidentFrames;
     const bool af_split = af_mode == ISAR_AF_SPLIT || af_mode == ISAR_AF_SPLIT_PHASE || (af_auto && frames <= kAfSplitFrames);
-    if (af_guarded) J.af_wait_polls = std::min(J.af_wait_polls, kAfGuardedPolls);
+    if (af_guarded) J.af_wait_polls = std::min(J.af_wait_polls, af_guarded_polls(J.iterations));
     probed(ISAR_STAGE_AUTOFOCUS, s, [&] {
         if (af_guarded || af_mode == ISAR_AF_RESIDENT) launch_autofocus_resident(J, af_guarded, s);
         else if (af_split) launch_autofocus_split(J, af_mode != ISAR_AF_SPLIT_PHASE, s);

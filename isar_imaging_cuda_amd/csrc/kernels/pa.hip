@@ -649,8 +649,8 @@ __device__ __forceinline__ float2 af_phase_from_words(const uint64_t* words, int
 // All of a frame's workgroups must be resident together; every XCD takes its share of a grid's
 // workgroups in order, so where the first incomplete frame lacks one, only complete frames are
 // ahead of it, and it completes as those finish. That holds for one such grid on the GPU; two at once can
-// each hold what the other's frames lack. So a wait that exceeds J.af_wait_polls polls (about a
-// second by default; a negative bound gives up at once) sets status bit 2 of the frame, which
+// each hold what the other's frames lack. So a wait that exceeds J.af_wait_polls polls (a quarter
+// of a second by default; a negative bound gives up at once) sets status bit 2 of the frame, which
 // k_af_start cleared, and ends its workgroup. Once the bit is set the frame's other workgroups leave too:
 // those that wait within kAfStatusPolls polls, those placed later before their first transform. (The words
 // they would read are those of an iteration that the leavers never finished: each would wait its own

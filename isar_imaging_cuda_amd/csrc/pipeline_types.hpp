@@ -28,10 +28,6 @@ constexpr int kCutBandRows = 16;      // rows per workgroup when cutting the ran
 // and 6.0 at 1024; 40 frames of 512 pulses 0.74 and 2.98. A batch that fills the CUs is the other
 // way round: 256 frames of 256 pulses 1.0 ms with one workgroup each, and more than that resident.
 constexpr int kAfResidentFrames = 128;
-// Bound of a resident wait in the default form, in polls of about a microsecond; a frame that
-// reaches it is done over by one workgroup. Frames of a full launch wait for earlier ones, at most a
-// few milliseconds.
-constexpr int kAfGuardedPolls = 1 << 16;
 // Sub-aperture plans run several groups at once; their default is the split form up to this many
 // windows, one workgroup per window above.
 constexpr int kAfSplitFrames = 32;
