@@ -1,8 +1,6 @@
 // pipeline.cpp — imaging context and the batch launch sequence (isar_main.cu:3-227).
 #include "pipeline.hpp"
 
-#include "../autofocus_rules.hpp"
-
 #include <algorithm>
 #include <cmath>
 #include <cstring>

@@ -662,7 +662,7 @@ __device__ __forceinline__ float2 af_phase_from_words(const uint64_t* words, int
 // transforms and products take 5500 cycles, the sums 700 and the exchange, which the number of load
 // instructions decides, 1700; with a tag in every word, so twice as many loads, 2500.
 template <int M>
-__global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(Job J) {
+__global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(Job J, int least, int most) {
     using A = AfCfg<M>;
     using C = ColCfg<M>;
     constexpr int E = A::E, TPF = A::TPF, SUB = A::SUB, NTS = SUB * TPF;
@@ -672,6 +672,7 @@ __global__ __launch_bounds__(AfCfg<M>::SUB * AfCfg<M>::TPF) void k_af_resident(J
     const int f = blockIdx.y, tid = threadIdx.x;
     const int U = J.dec[f].unit2_num;
     const int nsub = (U + SUB - 1) / SUB;
+    if (nsub < least || nsub > most) return;   // another launch's frame
     const int j = af_subchunk_of(f, nsub);
     if (j >= nsub) return;   // the whole workgroup leaves before any barrier
     const int c0 = j * SUB;
@@ -726,18 +727,13 @@ template <int M>
 size_t af_cols_lds(bool fold) {
     return (static_cast<size_t>(AfCfg<M>::SUB) * lds_padded_size(M) + (fold ? M : 0)) * sizeof(float2);
 }
-// LDS of a resident workgroup. The dispatcher fills a CU that has the LDS for another workgroup while
-// other CUs are idle, and the fullest CU sets the pace of every iteration. So a workgroup asks for
-// so much LDS that a CU takes only its share of them, with a quarter of the places to spare; a
-// frame commonly selects up to 64 bins, more only run in more rounds. Of 256 pulses 40 frames take 0.51 ms
-// with the share, 0.78 with the LDS needed, 64 frames 0.57 and 0.81, 128 frames 0.76 and 0.86; of
-// 512 pulses 40 frames 0.74 and 1.10.
 template <int M>
-size_t af_resident_lds(int frames) {
-    const int groups = frames * (64 / AfCfg<M>::SUB);
-    const size_t per_cu = (4 * groups + 3 * kComputeUnits - 1) / (3 * kComputeUnits);
-    return std::max(af_cols_lds<M>(true) + sizeof(int), kLdsBytes / (per_cu + 1) + 1024);
-}
+constexpr size_t kAfResidentNeed = (static_cast<size_t>(AfCfg<M>::SUB) * lds_padded_size(M) + M) * sizeof(float2) + sizeof(int);
+// Resident workgroups that a CU can hold: 16 waves of at most 128 vector registers (384 pulses take 134: 12
+// waves), and their LDS.
+template <int M>
+constexpr int kAfResidentFit = std::min((M == 384 ? 12 : 16) / ((AfCfg<M>::SUB * AfCfg<M>::TPF + 63) / 64),
+                                        static_cast<int>(kLdsBytes / kAfResidentNeed<M>));
 template <int M>
 size_t colfft_lds() {
     using C = ColCfg<M>;
@@ -783,7 +779,7 @@ hipError_t configure_pa_kernels() {
     set(reinterpret_cast<const void*>(&k_autofocus<MM>), autofocus_lds<MM>());   \
     set(reinterpret_cast<const void*>(&k_af_cols<MM, true>), af_cols_lds<MM>(true));   \
     set(reinterpret_cast<const void*>(&k_af_cols<MM, false>), af_cols_lds<MM>(false));   \
-    set(reinterpret_cast<const void*>(&k_af_resident<MM>), af_resident_lds<MM>(1));
+    set(reinterpret_cast<const void*>(&k_af_resident<MM>), std::max(kAfResidentNeed<MM>, kLdsBytes / 2 + 1024));
     ISAR_SET_PA(64) ISAR_SET_PA(128) ISAR_SET_PA(192) ISAR_SET_PA(256) ISAR_SET_PA(384) ISAR_SET_PA(512)
     ISAR_SET_PA(1024)
 #undef ISAR_SET_PA
@@ -842,8 +838,10 @@ void autofocus_resident(const Job& J, bool guarded, hipStream_t s) {
     autofocus_start_spread<MM>(J, true, s);
     if (J.iterations > 0) {
         constexpr int SUB = AfCfg<MM>::SUB;
-        ISAR_LAUNCH_RESIDENT(k_af_resident<MM>, dim3(J.W / SUB, J.K), dim3(SUB * AfCfg<MM>::TPF), af_resident_lds<MM>(J.K),
-                             s, J);
+        const AfResidentShapes shapes = af_resident_shapes(J.K, SUB, kAfResidentNeed<MM>, kAfResidentFit<MM>);
+        for (int i = 0; i < shapes.n; ++i)
+            ISAR_LAUNCH_RESIDENT(k_af_resident<MM>, dim3(J.W / SUB, J.K), dim3(SUB * AfCfg<MM>::TPF), shapes.shape[i].lds, s,
+                                 J, i ? shapes.shape[0].sub_chunks + 1 : 1, shapes.shape[i].sub_chunks);
         if (guarded) {
             Job redo = J;
             redo.af_redo = 1;

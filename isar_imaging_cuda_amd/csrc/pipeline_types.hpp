@@ -14,10 +14,10 @@
 
 #include <stdint.h>
 
+#include "autofocus_rules.hpp"
+
 namespace isar {
 
-constexpr int kComputeUnits = 256;    // of the GPU, in 8 XCDs
-constexpr size_t kLdsBytes = 160 * 1024;   // of a compute unit
 constexpr int kRangeCut = 512;        // RANGE_NUM_CUT (common.cuh:71)
 constexpr int kRangeNumIfdsPc = 4096; // RANGE_NUM_IFDS_PC (common.cuh:72)
 constexpr int kRaChunkRowsDefault = 8;   // rows per workgroup in the alignment update kernel

@@ -263,6 +263,35 @@ def test_default_autofocus_form_equals_the_explicit_forms(M, N, frames, polls):
     assert np.array_equal(out[isar.AF_AUTO][0], out[isar.AF_FUSED][0])
 
 
+@pytest.mark.parametrize("M,frames", [(64, 40), (256, 40), (512, 24), (1024, 9)])
+def test_default_autofocus_form_with_many_selected_bins(M, frames):
+    """Frames so weak that every column maximum truncates to 0 select all 512 bins; their workgroups are
+    placed by a launch of their own, here with more of them than the GPU holds at once (256 pulses and up),
+    beside frames of few bins in the same batch. Phases and images equal those of one workgroup per frame bit
+    for bit and no frame reports status bit 2."""
+    N = 1024
+    cfgs = [synth.preset(1, echo_num=M, range_num=N, seed=380 + k) for k in range(3)]
+    data = [synth.frame(c) for c in cfgs]
+    radar = synth.radar_header(cfgs[0])
+    weak = np.arange(frames) % 8 != 3
+    echo = np.stack([data[k % 3][0] * np.float32(2.0 ** -24 if weak[k] else 1.0) for k in range(frames)])
+    vel = np.stack([data[k % 3][1] for k in range(frames)])
+    print(f"[case] default autofocus form, 512 bins, M={M} frames={frames}", flush=True)
+    params = isar.RadarParams(M, N, radar["band_width"], radar["fc"], radar["Tp"], radar["Fs"])
+    out = {}
+    for mode in (isar.AF_AUTO, isar.AF_FUSED):
+        with isar.Imager(params, max_frames=frames) as im:
+            im.set_autofocus_mode(mode)
+            img = im.run_host(echo, vel, isar.Options(iterations=20))
+            out[mode] = (img, [im.trace(k) for k in range(frames)])
+    for k in range(frames):
+        a, b = out[isar.AF_AUTO][1][k], out[isar.AF_FUSED][1][k]
+        assert (a.unit2_num == 512) == bool(weak[k]) and a.unit2_num == b.unit2_num
+        assert a.status & 2 == 0, f"frame {k}"
+        assert np.array_equal(a.phi, b.phi), f"frame {k}: phases differ"
+    assert np.array_equal(out[isar.AF_AUTO][0], out[isar.AF_FUSED][0])
+
+
 def test_batch_matches_single_frames():
     cfgs = [synth.preset(1, seed=100 + k) for k in range(3)]
     frames = [synth.frame(c) for c in cfgs]
