@@ -273,7 +273,8 @@ ISAR_API int isar_fft_host(int n, int dir, const float* h_in, float* h_out, int 
 ISAR_API int isar_fft_host_grouped(int n, int dir, const float* h_in, float* h_out, int batch);
 
 /* Kernel families that can be probed with HIP events (isar_probe_enable). The IFDS pre-stage and the
- * IFDS profiles come from the first alignment launch (RA_PAIR0): IFDS_PRE counts no launches. */
+ * IFDS profiles come from the first alignment launch: of an IFDS run, IFDS_PRE and RA_PAIR0 both
+ * count that launch. */
 enum isar_stage {
     ISAR_STAGE_IFDS_PRE = 0, ISAR_STAGE_RA_PAIR0 = 1, ISAR_STAGE_RA_CORR = 2, ISAR_STAGE_RA_UPD = 3,
     ISAR_STAGE_CENTER = 4, ISAR_STAGE_CUT = 5, ISAR_STAGE_PA_COLFFT = 6, ISAR_STAGE_PA_SELECT = 7,

@@ -375,7 +375,9 @@ int Context::enqueue(int frames, const void* echo, const double* velocity, const
     if (probe_stage >= 0 && probe_used + 16 > static_cast<int>(probe_events.size()) / 2) probe_collect();
     if (mode != ISAR_RUN_BACK) {
         if (J.hrrp && J.data_type == 2) probed(ISAR_STAGE_HRRP, s, [&] { launch_hrrp(J, s); });
-        probed(ISAR_STAGE_RA_PAIR0, s, [&] { launch_ra_pair0(J, s); });
+        // the first alignment launch holds the IFDS pre-stage: a probe of either counts it
+        const bool ifds_probe = J.data_type == 1 && probe_stage == ISAR_STAGE_IFDS_PRE;
+        probed(ifds_probe ? ISAR_STAGE_IFDS_PRE : ISAR_STAGE_RA_PAIR0, s, [&] { launch_ra_pair0(J, s); });
         int pair_base = M / 2;
         for (int st = 2; st < M; st *= 2) {
             const int ngroups = (M + st - 1) / st, npairs = ngroups / 2, unpaired = ngroups & 1;

@@ -176,6 +176,21 @@ def test_ifds_prestage_at_every_row_length(N):
         assert rep.ok(), f"frame {k}: {rep}"
 
 
+def test_probe_of_the_ifds_prestage_counts_its_launch():
+    """Every run of IFDS frames launches the pre-stage once and a run of STRETCH frames does not, and the
+    probe of that family says so, with the launch's time."""
+    _, echo, vel, radar = _frame(1, echo_num=64, range_num=1024, seed=370)
+    params = isar.RadarParams(64, 1024, radar["band_width"], radar["fc"], radar["Tp"], radar["Fs"])
+    print("[case] probe of the ifds pre-stage", flush=True)
+    with isar.Imager(params, max_frames=1) as im:
+        im.probe_enable(isar.STAGES["ifds_pre"])
+        for data_type, launches in ((1, 3), (2, 0)):
+            for _ in range(3):
+                im.run_host(echo, vel, isar.Options(data_type=data_type, iterations=1))
+            ms, n = im.probe_read()
+            assert n == launches and (ms > 0.0) == (n > 0)
+
+
 @pytest.mark.parametrize("M,N", [(64, 1024), (128, 1024), (192, 1024), (256, 2048), (384, 1024), (512, 1024),
                                  (1024, 2048)])
 def test_autofocus_forms_agree(M, N):
