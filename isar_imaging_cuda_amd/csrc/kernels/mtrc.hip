@@ -109,38 +109,39 @@ __global__ __launch_bounds__(kRowsPerBlock * W / kRowE) void k_mtrc_rows(Job J) 
 // Chirp-z transform along slow time for a tile of range bins (mtrc.cu:42-52, 125-192):
 // X[k] = exp(-j pi a k^2/M) / F * IFFT_F( FFT_F(y) * table_n )[k],
 // y[m] = x[m] exp(j pi a m (M - m) / M) for m < M. Also writes sum_k X[k] per bin.
-// HALF: F = 2 M (a power of two), so slots 8 ... 15 of every thread lie past M: they are zero going in and
-// not formed coming out, with their table entries and transposes. That leaves it the registers to read
-// the table row before the first transform and the output chirps before the second.
+// A thread's slots lie before M or past it for all threads alike (in_offset and M are multiples of the
+// transform's threads): those past M are zero going in and not formed coming out, with their table
+// entries and transposes. HALF: F = 2 M, a power of two, so they are slots 8 ... 15 (fft_zero_half). That leaves it the
+// registers to read the table row before the first transform and the output chirps before the second.
 // Bound by latency between the tile's read and write (2.9 TB/s, vector issue 0.6 of its limit): 1024
 // frames of 256 pulses take 0.73 ms; 0.77 with those reads at their use, 1.19 before the zero half was skipped.
-template <int F, int NTW, bool HALF>
+// With M known only at run time the other lengths tested every slot and spilled 14 to 27 registers: 150 frames of 192
+// pulses at F = 384 205 us instead of 112, of 384 pulses at F = 768 and 1024 429 and 352 instead of 258 and 211.
+template <int F, int M, int NTW>
 __global__ __launch_bounds__(NTW, 4) void k_mtrc_czt(Job J) {
     using C = CztCfg<F, NTW>;
     constexpr int CT = C::CT, TPF = C::TPF, E = C::E, NT = C::NT;
-    constexpr int EM = HALF ? E / 2 : E;   // slots that can lie before M
+    constexpr bool HALF = 2 * M == F && F % 3 != 0;
+    static_assert(M % TPF == 0, "a slot lies before M in every thread or in none");
     HIP_DYNAMIC_SHARED(float2, sm);
     const int tile = xcd_tile(blockIdx.x, gridDim.x), f = blockIdx.y, tid = threadIdx.x;
-    const int M = HALF ? F / 2 : J.M, W = J.W;
+    const int W = J.W;
     const int g = tid / TPF, lane = tid % TPF;
     const int n0 = tile * CT, n = n0 + g;
     const float2* pre = J.czt_pre + static_cast<size_t>(n) * M;
     const float2* post = J.czt_post + static_cast<size_t>(n) * M;
-    auto pos = [&](int e) { return HALF ? C::in(lane, e) : min(C::in(lane, e), M - 1); };
-    auto before_m = [&](int e) { return HALF || C::in(lane, e) < M; };
-    // the table rows are read ahead of their use, in full (past M the last entry, which is not used):
-    // one at a time under a test of the position they cost more than the transforms
-    float2 pre_v[EM];
+    auto before_m = [](int e) { return fft_in_offset<F, E>(e) < M; };
+    // the table rows are read ahead of their use: one at a time they cost more than the transforms
+    float2 pre_v[E];
 #pragma unroll
-    for (int e = 0; e < EM; ++e) pre_v[e] = pre[pos(e)];
+    for (int e = 0; e < E; ++e)
+        if (before_m(e)) pre_v[e] = pre[C::in(lane, e)];
     load_column_tile<NT, CT>(J.stm + static_cast<size_t>(f) * M * W, W, n0, M, sm, tid);
     __syncthreads();
     float2 x[E];
 #pragma unroll
-    for (int e = 0; e < EM; ++e) {
-        const float2 y = cmul(sm[pos(e) * (CT + 1) + g], pre_v[e]);
-        x[e] = before_m(e) ? y : make_float2(0.0f, 0.0f);
-    }
+    for (int e = 0; e < E; ++e)
+        x[e] = before_m(e) ? cmul(sm[C::in(lane, e) * (CT + 1) + g], pre_v[e]) : make_float2(0.0f, 0.0f);
     __syncthreads();
     // a transform within one wave orders its passes by the wave alone (the transpose back below
     // waits for every wave with a barrier of its own)
@@ -155,34 +156,32 @@ __global__ __launch_bounds__(NTW, 4) void k_mtrc_czt(Job J) {
     }
     if constexpr (HALF && FftPlan<F, E>::R[0] == 16) fft_zero_half<F, -1, kWave>(x, buf, lane);
     else fft<F, E, -1, kWave>(x, buf, lane);
-    float2 p[EM];
-    {
-        if constexpr (HALF) {
+    auto read_post = [&](float2 (&p)[E]) {
 #pragma unroll
-            for (int e = 0; e < EM; ++e) p[e] = post[pos(e)];
-        } else {
+        for (int e = 0; e < E; ++e)
+            if (before_m(e)) p[e] = post[C::in(lane, e)];
+    };
+    float2 p[E];
+    if constexpr (HALF) {
+        read_post(p);
+    } else {
 #pragma unroll
-            for (int e = 0; e < E; ++e) t[e] = tab[C::out(lane, e)];
-        }
-        issue_point();
-#pragma unroll
-        for (int e = 0; e < E; ++e) x[e] = cmul(x[e], t[e]);
+        for (int e = 0; e < E; ++e) t[e] = tab[C::out(lane, e)];
     }
+    issue_point();
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = cmul(x[e], t[e]);
     fft<F, E, +1, kWave, true>(x, buf, lane);   // back to the layout of the input
+    if constexpr (!HALF) {
+        read_post(p);
+        issue_point();
+    }
     float2 csum = make_float2(0.0f, 0.0f);
-    float2 y[EM];
-    {
-        if constexpr (!HALF) {
 #pragma unroll
-            for (int e = 0; e < EM; ++e) p[e] = post[pos(e)];
-            issue_point();
-        }
-#pragma unroll
-        for (int e = 0; e < EM; ++e) {
-            const float2 v = cmul(x[e], p[e]);
-            y[e] = before_m(e) ? v : make_float2(0.0f, 0.0f);
-            csum = cadd(csum, y[e]);
-        }
+    for (int e = 0; e < E; ++e) {
+        if (!before_m(e)) continue;
+        x[e] = cmul(x[e], p[e]);
+        csum = cadd(csum, x[e]);
     }
     if constexpr (TPF <= 64) {
         csum = group_sum2<TPF>(csum);
@@ -203,8 +202,8 @@ __global__ __launch_bounds__(NTW, 4) void k_mtrc_czt(Job J) {
     }
     // transpose back through LDS for row-contiguous stores
 #pragma unroll
-    for (int e = 0; e < EM; ++e)
-        if (before_m(e)) sm[C::in(lane, e) * (CT + 1) + g] = y[e];
+    for (int e = 0; e < E; ++e)
+        if (before_m(e)) sm[C::in(lane, e) * (CT + 1) + g] = x[e];
     __syncthreads();
     float2* D = J.czt + static_cast<size_t>(f) * M * W;
     for (int idx = tid; idx < M * CT; idx += NT) {
@@ -397,16 +396,15 @@ hipError_t configure_mtrc_kernels() {
             report_config_error(__FILE__, bytes);
         }
     };
-#define ISAR_SET_F(FF)                                                                          \
-    set(reinterpret_cast<const void*>(&k_czt_table<FF>), lds_padded_size(FF) * sizeof(float2)); \
-    set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, 256, false>), czt_lds<FF, 256>(FF / 2));  \
-    set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, 512, false>), czt_lds<FF, 512>(FF / 2));  \
-    if constexpr (FF % 3 != 0) {                                                                 \
-        set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, 256, true>), czt_lds<FF, 256>(FF / 2)); \
-        set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, 512, true>), czt_lds<FF, 512>(FF / 2)); \
-    }
+#define ISAR_SET_F(FF) set(reinterpret_cast<const void*>(&k_czt_table<FF>), lds_padded_size(FF) * sizeof(float2));
     ISAR_SET_F(128) ISAR_SET_F(256) ISAR_SET_F(384) ISAR_SET_F(512) ISAR_SET_F(768) ISAR_SET_F(1024) ISAR_SET_F(2048)
 #undef ISAR_SET_F
+#define ISAR_SET_CZT(FF, MM)                                                                    \
+    set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, MM, 256>), czt_lds<FF, 256>(MM));         \
+    set(reinterpret_cast<const void*>(&k_mtrc_czt<FF, MM, 512>), czt_lds<FF, 512>(MM));
+    ISAR_SET_CZT(128, 64) ISAR_SET_CZT(256, 128) ISAR_SET_CZT(384, 192) ISAR_SET_CZT(512, 192) ISAR_SET_CZT(512, 256)
+    ISAR_SET_CZT(768, 384) ISAR_SET_CZT(1024, 384) ISAR_SET_CZT(1024, 512) ISAR_SET_CZT(2048, 1024)
+#undef ISAR_SET_CZT
 #define ISAR_SET_M(MM)                                                         \
     set(reinterpret_cast<const void*>(&k_col_window<MM>), col_lds<MM>());     \
     set(reinterpret_cast<const void*>(&k_post_nomtrc<MM>), col_lds<MM>());
@@ -434,17 +432,20 @@ void launch_mtrc_rows(const Job& J, hipStream_t s) {
                 dim3(kRowsPerBlock * kRangeCut / kRowE), rows_lds(), s, J);
 }
 namespace {
+template <int F, int M, int NTW>
+void mtrc_czt(const Job& J, hipStream_t s) {
+    ISAR_LAUNCH((k_mtrc_czt<F, M, NTW>), dim3(J.W / CztCfg<F, NTW>::CT, J.K), dim3(NTW), (czt_lds<F, NTW>(M)), s, J);
+}
+// F = 2 M, or the power of two above 2 M of 192 and 384 pulses (czt_length_candidates)
 template <int F, int NTW>
 void mtrc_czt(const Job& J, hipStream_t s) {
-    const dim3 grid(J.W / CztCfg<F, NTW>::CT, J.K);
-    const size_t lds = czt_lds<F, NTW>(J.M);
-    if constexpr (F % 3 != 0) {
-        if (2 * J.M == F) {
-            ISAR_LAUNCH((k_mtrc_czt<F, NTW, true>), grid, dim3(NTW), lds, s, J);
+    if constexpr (F == 512 || F == 1024) {
+        if (J.M == F * 3 / 8) {
+            mtrc_czt<F, F * 3 / 8, NTW>(J, s);
             return;
         }
     }
-    ISAR_LAUNCH((k_mtrc_czt<F, NTW, false>), grid, dim3(NTW), lds, s, J);
+    mtrc_czt<F, F / 2, NTW>(J, s);
 }
 }  // namespace
 void launch_mtrc_czt(const Job& J, hipStream_t s) {
