@@ -1,5 +1,6 @@
 // learned.cpp — the warm-start network object behind isar_learned.h: FP32 master parameters,
 // BF16 weight copies, Adam moments and per-layer activations, all allocated at creation.
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <string>
@@ -22,7 +23,7 @@ struct Mlp {
     float* m2 = nullptr;
     uint16_t* wbf = nullptr;
     int* bf_index = nullptr;           // parameter -> BF16 slot (-1 for biases)
-    std::vector<float*> act;           // act[l], l = 1..n: batch x widths[l]
+    std::vector<float*> act;           // act[l], 1 <= l < n: batch x widths[l]; act[n] for n = 1 only
     float* dz[2] = {nullptr, nullptr};
     const float* input = nullptr;      // input of the last forward
     int last_batch = 0;
@@ -87,7 +88,8 @@ ISAR_API int isar_mlp_create(int n_layers, const int* widths, int max_batch, isa
     net->wbf = static_cast<uint16_t*>(alloc(nw * sizeof(uint16_t)));
     net->bf_index = static_cast<int*>(alloc(np * sizeof(int)));
     net->act.assign(n_layers + 1, nullptr);
-    for (int l = 1; l <= n_layers; ++l)
+    // the last layer of two or more writes the caller's buffer
+    for (int l = 1; l < std::max(n_layers, 2); ++l)
         net->act[l] = static_cast<float*>(alloc(static_cast<size_t>(max_batch) * widths[l] * sizeof(float)));
     net->dz[0] = static_cast<float*>(alloc(static_cast<size_t>(max_batch) * maxw * sizeof(float)));
     net->dz[1] = static_cast<float*>(alloc(static_cast<size_t>(max_batch) * maxw * sizeof(float)));

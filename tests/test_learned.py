@@ -164,6 +164,23 @@ def test_one_layer_products_at_tile_edges_match_oracle(widths, batch):
 
 
 @pytest.mark.gpu
+def test_network_holds_no_output_buffer():
+    """A network of two layers writes its output into the caller's buffer: of the last layer's width it keeps
+    the two gradient buffers and no third one of max_batch rows."""
+    torch = _torch()
+    from isar_imaging_cuda_amd import learned as L
+    batch, width = 1 << 15, 4096
+    torch.cuda.init()
+    print("[case] buffers of a two-layer network", flush=True)
+    before = torch.cuda.mem_get_info()[0]
+    net = L.Mlp([8, 8, width], batch)
+    held = before - torch.cuda.mem_get_info()[0]
+    buffer = batch * width * 4
+    assert 2 * buffer <= held < 2.5 * buffer, held / buffer
+    del net
+
+
+@pytest.mark.gpu
 def test_adam_step_matches_oracle():
     torch = _torch()
     widths = [32, 16, 8]
