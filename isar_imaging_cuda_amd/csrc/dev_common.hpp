@@ -146,9 +146,6 @@ __device__ __forceinline__ T group_combine(T v, F step) {
 // ------------------------------------------------------------------------------------------
 // reductions
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ float wave_sum(float v) {
-    return group_combine<64>(v, [](float a, float b) { return a + b; });
-}
 __device__ __forceinline__ double wave_sum_d(double v) {
     return group_combine<64>(v, [](double a, double b) { return a + b; });
 }
