@@ -60,6 +60,15 @@ inline thread_local BlockCtx t_ctx;
 #define HIP_DYNAMIC_SHARED(type, var) type* var = reinterpret_cast<type*>(isar_emu::t_ctx.smem)
 
 inline void __syncthreads() { isar_emu::t_ctx.bar->arrive_and_wait(); }
+inline int __syncthreads_or(int v) {
+    auto& xb = *isar_emu::t_ctx.xbuf;
+    xb[threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z)] = v != 0;
+    __syncthreads();
+    int any = 0;
+    for (const uint64_t x : xb) any |= x != 0;
+    __syncthreads();
+    return any;
+}
 inline void __threadfence() { std::atomic_thread_fence(std::memory_order_seq_cst); }
 inline int atomicAdd(int* p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST); }
 inline int atomicOr(int* p, int v) { return __atomic_fetch_or(p, v, __ATOMIC_SEQ_CST); }

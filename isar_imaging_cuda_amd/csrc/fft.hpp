@@ -23,7 +23,7 @@
 // and two sums take eight, and no separate twiddle products (radix 16: 192 instructions instead of
 // 168 for the butterfly, 60 for the twiddles and up to 52 to form their powers). c and t are each
 // rounded once from FP64 (fft_table); the rounding of (1 + j t) b is relative to that sum,
-// which c brings back to the size of b, so a large t costs no accuracy: 512, 4096 and 16384 points
+// which c brings back to the size of b, so a large t costs no accuracy, only range (fft_overflowed). 512, 4096 and 16384 points
 // are 0.95, 1.15 and 1.26e-7 off the FP64 transform (relative, random data; 4096 points with products
 // of rounded twiddles 1.97e-7). A 512-point transform with its 2-point pass takes 388 vector
 // instructions instead of 700, and what is bound by their issue is that much faster: the autofocus
@@ -577,6 +577,18 @@ struct FftPasses {
 template <int N, int E, int DIR, bool WAVE = false, bool REV = false, typename TW>
 __device__ __forceinline__ void fft(float2 (&x)[E], float2* lds, int tid, const TW& tw) {
     FftPasses<N, E, DIR, 0, WAVE, REV, TW>::run(x, lds, tid, tw);
+}
+// The factor t of a butterfly is up to 2^30, so that values whose transform FP32 holds can overflow on the
+// way, from about 2^83 on at 16384 points. A kernel that takes any input does a transform over on
+// kFftLarge times its values where the workgroup's results are not all finite (which an overflow
+// always leaves so), and divides the results by it. Every thread of the workgroup calls it.
+constexpr float kFftLarge = 0x1p-60f;
+template <int E>
+__device__ __forceinline__ bool fft_overflowed(const float2 (&x)[E]) {
+    float m = 0.0f;   // not finite if any value is not
+#pragma unroll
+    for (int e = 0; e < E; ++e) m = fmaf(x[e].x, 0.0f, fmaf(x[e].y, 0.0f, m));
+    return __syncthreads_or(!(m == 0.0f));
 }
 // A kernel's only transform: the constants are loaded ahead of its first pass.
 template <int N, int E, int DIR, bool WAVE = false, bool REV = false>

@@ -11,11 +11,14 @@ __global__ __launch_bounds__(N / E) void k_debug_fft(const float2* in, float2* o
     const size_t base = static_cast<size_t>(blockIdx.x) * N;
     const int tid = threadIdx.x;
     float2 x[E];
+    for (float scale = 1.0f;; scale = kFftLarge) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) x[e] = in[base + fft_in_pos<N, E, REV>(tid, e)];
-    fft<N, E, DIR, false, REV>(x, lds, tid);
+        for (int e = 0; e < E; ++e) x[e] = cscale(in[base + fft_in_pos<N, E, REV>(tid, e)], scale);
+        fft<N, E, DIR, false, REV>(x, lds, tid);
 #pragma unroll
-    for (int e = 0; e < E; ++e) out[base + fft_out_pos<N, E, REV>(tid, e)] = x[e];
+        for (int e = 0; e < E; ++e) out[base + fft_out_pos<N, E, REV>(tid, e)] = cscale(x[e], 1.0f / scale);
+        if (scale != 1.0f || !fft_overflowed(x)) break;
+    }
 }
 
 // 256 / (N / E) transforms per workgroup, each on N / E threads of one wave with its own LDS
@@ -32,12 +35,16 @@ __global__ __launch_bounds__(256) void k_debug_fft_grouped(const float2* in, flo
     const bool valid = t < batch;
     const size_t base = static_cast<size_t>(valid ? t : 0) * N;
     float2 x[E];
+    for (float scale = 1.0f;; scale = kFftLarge) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) x[e] = valid ? in[base + fft_in_pos<N, E, REV>(lane, e)] : make_float2(0.0f, 0.0f);
-    fft<N, E, DIR, true, REV>(x, lds + g * lds_padded_size(N), lane);
-    if (valid) {
+        for (int e = 0; e < E; ++e)
+            x[e] = valid ? cscale(in[base + fft_in_pos<N, E, REV>(lane, e)], scale) : make_float2(0.0f, 0.0f);
+        fft<N, E, DIR, true, REV>(x, lds + g * lds_padded_size(N), lane);
+        if (valid) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) out[base + fft_out_pos<N, E, REV>(lane, e)] = x[e];
+            for (int e = 0; e < E; ++e) out[base + fft_out_pos<N, E, REV>(lane, e)] = cscale(x[e], 1.0f / scale);
+        }
+        if (scale != 1.0f || !fft_overflowed(x)) break;
     }
 }
 

@@ -361,12 +361,17 @@ __global__ __launch_bounds__(N / kE) void k_hrrp(Job J) {
     const int m = blockIdx.x, f = blockIdx.y, tid = threadIdx.x;
     float2 x[kE];
     RowSamples<N, true> row;
-    row.load(J, f, m, tid);
-    row.spectrum(x, J, tid, 1.0f);
-    fft<N, kE, -1>(x, lds, tid);
     float2* dst = J.hrrp + (static_cast<size_t>(f) * J.M + m) * N;
+#pragma unroll 1
+    for (float scale = 1.0f;; scale = kFftLarge) {
+        const int t = opaque(tid);   // nothing is kept in registers for the second time
+        row.load(J, f, m, t);
+        row.spectrum(x, J, t, scale);
+        fft<N, kE, -1>(x, lds, t);
 #pragma unroll
-    for (int e = 0; e < kE; ++e) dst[row_pos<N>(tid, e)] = x[e];
+        for (int e = 0; e < kE; ++e) dst[row_pos<N>(t, e)] = cscale(x[e], 1.0f / scale);
+        if (scale != 1.0f || !fft_overflowed(x)) break;
+    }
 }
 
 // Merge level 0 fused with the spectrum preparation (range_alignment.cu:13-18 and :34-73 at

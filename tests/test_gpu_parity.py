@@ -37,6 +37,26 @@ def test_wave_ordered_fft_equals_workgroup_ordered(n, inverse):
         assert np.array_equal(isar.fft(x, inverse=inverse, grouped=True), isar.fft(x, inverse=inverse))
 
 
+@pytest.mark.parametrize("n", [64, 128, 192, 256, 384, 512, 1024, 2048, 4096, 8192, 16384])
+def test_fft_of_large_values(n):
+    """Multiplied by 2^100, a row of unit size has a transform that FP32 holds, and every operation on it
+    scales exactly, in a batch beside rows of ordinary size too."""
+    rng = np.random.default_rng(n)
+    x = (rng.standard_normal((5, n)) + 1j * rng.standard_normal((5, n))).astype(np.complex64)
+    big = x.copy()
+    big[1::2] *= np.float32(2.0 ** 100)
+    for inverse in (False, True):
+        for grouped in ((False, True) if n <= 1024 else (False,)):
+            print(f"[case] large values n={n} inverse={inverse} grouped={grouped}", flush=True)
+            y = isar.fft(x, inverse=inverse, grouped=grouped)
+            z = isar.fft(big, inverse=inverse, grouped=grouped)
+            assert np.array_equal(z[1::2], y[1::2] * np.float32(2.0 ** 100))
+            if grouped:   # transforms of one workgroup share the factor: 2^-60 of a small one may be subnormal
+                assert np.abs(z[::2] - y[::2]).max() <= 1e-6 * np.abs(y[::2]).max()
+            else:
+                assert np.array_equal(z[::2], y[::2])
+
+
 def _frame(config_id, **over):
     cfg = synth.preset(config_id, **over)
     echo, vel = synth.frame(cfg)
@@ -174,6 +194,24 @@ def test_ifds_prestage_at_every_row_length(N):
         img_o, tro = oracle_run(data[k][1], data[k][2], radar, 64, N, data_type=1)
         rep = compare(img[k], tr[k], img_o, tro, 64)
         assert rep.ok(), f"frame {k}: {rep}"
+
+
+@pytest.mark.parametrize("N", [1024, 4096, 16384])
+def test_range_profiles_of_large_values(N):
+    """Echoes multiplied by 2^85 (whose energies leave FP32, so nothing after the profiles is of use) have
+    the profiles of the echoes multiplied by 2^85."""
+    import torch
+    _, echo, vel, radar = _frame(1, echo_num=64, range_num=N, seed=390)
+    params = isar.RadarParams(64, N, radar["band_width"], radar["fc"], radar["Tp"], radar["Fs"])
+    print(f"[case] range profiles of large values N={N}", flush=True)
+    out = []
+    with isar.Imager(params, max_frames=1) as im:
+        for scale in (1.0, 2.0 ** 85):
+            hrrp = torch.zeros((64, N, 2), dtype=torch.float32, device="cuda:0")
+            im.set_hrrp_output(hrrp.data_ptr())
+            im.run_host(echo * np.float32(scale), vel, isar.Options(if_hrrp=True, iterations=1))
+            out.append(hrrp.cpu().numpy())
+    assert np.array_equal(out[1], out[0] * np.float32(2.0 ** 85))
 
 
 def test_probe_of_the_ifds_prestage_counts_its_launch():
