@@ -309,7 +309,7 @@ def large_batch(frames: int = 8, steps: int = 3, learned_frames: int = 16, two_s
     dev = torch.device("cuda:0")
     img = torch.empty((frames, M5, W), dtype=torch.float32, device=dev)
     im = isar.Imager(isar.RadarParams(M5, N5, h["band_width"], h["fc"], h["Tp"], h["Fs"]), max_frames=frames)
-    im.set_autofocus_mode(isar.AF_RESIDENT)   # all iterations in one launch (a launch per iteration at AUTO)
+    im.set_autofocus_mode(isar.AF_RESIDENT)   # all iterations in one launch (as at AUTO, which does over a frame that gives up)
     s = torch.cuda.current_stream(dev)
     run = lambda: im.run_device(echo.data_ptr(), vel.data_ptr(), img.data_ptr(), frames, isar.Options(),
                                 stream=s.cuda_stream)

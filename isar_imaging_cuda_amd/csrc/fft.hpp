@@ -21,7 +21,8 @@
 // Every step is a +- z b for one of a few z, kept as z = c (1 + j t), t = tan: two fused
 // multiply-adds form (1 + j t) b and four add c times it to +-a, six instructions where a rotation
 // and two sums take eight, and no separate twiddle products (radix 16: 192 instructions instead of
-// 168 for the butterfly, 60 for the twiddles and up to 52 to form their powers). c and t are each
+// 168 for the butterfly, 60 for the twiddles and up to 52 to form their powers; E. N. Linzer and E. Feig,
+// "Implementation of efficient FFT algorithms on fused multiply-add architectures", 1993). c and t are each
 // rounded once from FP64 (fft_table); the rounding of (1 + j t) b is relative to that sum,
 // which c brings back to the size of b, so a large t costs no accuracy, only range (fft_overflowed). 512, 4096 and 16384 points
 // are 0.95, 1.15 and 1.26e-7 off the FP64 transform (relative, random data; 4096 points with products

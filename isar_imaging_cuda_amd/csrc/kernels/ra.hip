@@ -380,10 +380,10 @@ __global__ __launch_bounds__(N / kE) void k_hrrp(Job J) {
 // merged level-1 energy. Rows 0 and 1 never move again: their aligned profiles and column sums
 // are written here. The spectra carry the inverse transforms' 1 / N (a power of two), so no
 // profile or energy is scaled later.
-// Bound by memory and by vector issue alike: 1024 frames of 256 x 4096 take 5.4 ms, in which it moves
-// 23.2 MB a frame at 4.4 TB/s (a plain copy reaches 4.7) and issues 2.66 M vector instructions a
-// frame, 1.1 of the rate of one in 4 cycles. (S0 of row 2p+1 kept in registers instead of read again
-// saves 4.2 MB, but then the fourth wave of a SIMD does not fit: 5.7 ms.)
+// Bound by memory and by vector issue alike: 256 frames of 256 x 4096 take 1.21 ms, in which it moves
+// 23.2 MB a frame at 4.9 TB/s (a plain copy reaches 4.7) and issues 2.66 M vector instructions a
+// frame, 1.11 of the rate of one in 4 cycles; 1024 frames take 5.5 ms. (S0 of row 2p+1 kept in registers
+// instead of read again saves 4.2 MB a frame, but then the fourth wave of a SIMD does not fit: 5.7 ms.)
 template <int N, bool IFDS>
 __global__ __launch_bounds__(N / kE, 4) void k_ra_pair0(Job J) {
     HIP_DYNAMIC_SHARED(float2, lds);
