@@ -94,10 +94,12 @@ def test_resident_workgroup_placed_after_the_others_gave_up(emu_driver):
     echo, vel = synth.frame(cfg)
     radar = synth.radar_header(cfg)
     opts = emu_runner.default_options(iterations=ITERATIONS)
-    (ref,) = emu_runner.run(echo, vel, radar, opts, autofocus_mode=1, timeout=600)
-    assert ref.unit2_num >= 32   # two or more workgroups of 16 bins
     log = []
-    (fr,) = emu_runner.run(echo, vel, radar, opts, autofocus_mode=0, late=(2000, 1), log=log, timeout=600)
+    with cf.ThreadPoolExecutor(max_workers=2) as ex:
+        fref = ex.submit(emu_runner.run, echo, vel, radar, opts, autofocus_mode=1, timeout=600)
+        flate = ex.submit(emu_runner.run, echo, vel, radar, opts, autofocus_mode=0, late=(500, 1), log=log, timeout=600)
+        (ref,), (fr,) = fref.result(), flate.result()
+    assert ref.unit2_num >= 32   # two or more workgroups of 16 bins
     assert "late pauses 0" in log[0].split("\n"), log
     assert fr.status & 2 == 0
     assert np.array_equal(fr.phi, ref.phi) and np.array_equal(fr.img, ref.img)
