@@ -196,9 +196,9 @@ ISAR_API int isar_session_dump(unsigned mask, const char* dir);
  * to 32 windows and FUSED above. So up to 128 frames AUTO's workgroups wait for each other, and
  * those of a single run always find room. Runs of several contexts in flight at once take CUs
  * from each other, and in rare orders of placing could block each other until a wait gives up (12 ms
- * at 120 iterations); results stay the same. Two such contexts are faster on two streams than on
- * one, but with 96 or 128 frames of 256 pulses, or 128 of 64, FUSED is 4 to 13 percent faster
- * still; FUSED and SPLIT never wait. All forms give the same phases bit for bit. */
+ * at 120 iterations); results stay the same. Two such contexts gain by two streams, but with 96 or
+ * 128 frames of 256 pulses, or 128 of 64, FUSED is 4 to 13 percent faster there, and weak frames
+ * that select all bins fill the GPU by themselves; FUSED and SPLIT never wait. All forms give the same phases bit for bit. */
 enum isar_autofocus_mode {
     ISAR_AF_AUTO = 0,
     ISAR_AF_FUSED = 1,

@@ -42,7 +42,7 @@ constexpr AfResidentShape af_shape(int share, size_t need, int fit) {
 // own with shape[1], the share of a batch whose frames all have 512 bins; n = 1 where no frame
 // can need it. At 512
 // bins, in ms with one shape for all and with two: 32 frames of 256 pulses 3.31 and 1.33 (split 1.98), 16 of 64 1.55 and
-// 0.83, 128 of 64 4.77 and 1.41 (one workgroup a frame 2.94), 40 of 512 5.6 and 3.9, 8 of 1024 4.9 and 2.9.
+// 0.83, 128 of 64 4.77 and 1.41 (one workgroup a frame 2.84), 40 of 512 5.6 and 3.9, 8 of 1024 4.9 and 2.9.
 // With the LDS needed for all, 40 frames of 256 pulses with 64 bins take 0.78 instead of 0.51, 128 of
 // them 0.86 instead of 0.75, 40 of 512 1.10 instead of 0.72. The launch that has no frames takes 3 us.
 struct AfResidentShapes {

@@ -24,15 +24,15 @@ constexpr int kRaChunkRowsDefault = 8;   // rows per workgroup in the alignment 
 constexpr int kCutBandRows = 16;      // rows per workgroup when cutting the range window
 // Default autofocus form by batch size: several resident workgroups per frame up to this many frames,
 // one workgroup per frame above. The latter takes a CU per frame and leaves the others idle: at 64
-// selected bins 128 frames take 0.76 (resident) and 0.94 ms at 256 pulses, 2.0 and 3.0 at 512, 4.0
-// and 6.0 at 1024; 40 frames of 512 pulses 0.74 and 2.98. A batch that fills the CUs is the other
+// selected bins 128 frames take 0.75 (resident) and 0.84 ms at 256 pulses, 2.0 and 2.8 at 512, 3.9
+// and 5.4 at 1024; 40 frames of 512 pulses 0.73 and 2.62. A batch that fills the CUs is the other
 // way round: 256 frames of 256 pulses 1.0 ms with one workgroup each, and more than that resident.
 constexpr int kAfResidentFrames = 128;
 // Sub-aperture plans run several groups at once; their default is the split form up to this many
-// windows, one workgroup per window above. 64 windows of 128 to 512 pulses (9 to 17 a group) take 4.13 ms with
-// it, 4.28 with one workgroup a window in every group. By itself a group of 256 pulses takes 0.77 (split)
-// and 0.79 ms at 8 windows, 0.95 and 0.79 at 16, 1.30 and 0.80 at 32, one of 512 pulses 1.13 and 2.64, 1.54 and
-// 2.64, 1.57 and 2.67, at 64 selected bins; at 512 bins the split form is 4 to 12 times as fast.
+// windows, one workgroup per window above. 64 windows of 128 to 512 pulses (9 to 17 a group) take 4.08 ms with
+// it, 4.16 with one workgroup a window in every group. By itself a group of 256 pulses takes 0.77 (split)
+// and 0.79 ms at 8 windows, 0.95 and 0.79 at 16, 1.30 and 0.79 at 32, one of 512 pulses 1.13 and 2.58, 1.54 and
+// 2.60, 1.58 and 2.60, at 64 selected bins; at 512 bins the split form is 3 to 12 times as fast.
 constexpr int kAfSplitFrames = 32;
 // Batches of at least this many frames update the final rows of range alignment in a launch of their
 // own, since then it fills the GPU by itself: all levels of 1024 frames of 256 x 4096 take 8.3 instead
