@@ -365,7 +365,9 @@ __global__ __launch_bounds__(AfCfg<M>::NT) void k_autofocus(Job J) {
             __syncthreads();
         }
     };
-    if (U <= CF) {
+    if (J.iterations == 0) {
+        // the starting phase as it is
+    } else if (U <= CF) {
         const float2* col = su + static_cast<size_t>(g < U ? g : 0) * M;
 #pragma unroll
         for (int e = 0; e < E; ++e) s[e] = g < U ? col[C::in(lane, e)] : make_float2(0.0f, 0.0f);
