@@ -345,8 +345,7 @@ __device__ __forceinline__ double log_by_table(double q, int k, const LogRow* ro
     const uint64_t mb = (static_cast<uint64_t>((hi & 0x000fffffu) | 0x3ff00000u) << 32) | (bits & 0xffffffffu);
     const double r = fma(__builtin_bit_cast(double, mb), t.c, -1.0);
     const double e = static_cast<double>(static_cast<int>(hi >> 20) - k);
-    double y = fma(r, 1.0 / 7.0, -1.0 / 6.0);
-    y = fma(y, r, 1.0 / 5.0);
+    double y = fma(r, -1.0 / 6.0, 1.0 / 5.0);   // the next term is below 2e-18
     y = fma(y, r, -1.0 / 4.0);
     y = fma(y, r, 1.0 / 3.0);
     y = fma(y, r, -0.5);
@@ -361,8 +360,8 @@ __device__ __forceinline__ double log_by_table(double q, int k, const LogRow* ro
 // second sum, and the terms that count have q near r. Off by as much as -sum p ln p or less
 // (131072 cells, amplitudes 1e-15 to 1e15), and the same bits for an image scaled by a power of two.
 // A single bright cell gives 0 exactly, as both terms are then the same product. Bound by the loads'
-// latency and FP64 issue: 256 images of 256 x 512 take 34 us (3.9 TB/s), 1024 of them 121; 32 and 112
-// with r = 1; 34 and 132 with the registers left free, as a CU then holds one workgroup; 390 the 256 in
+// latency and FP64 issue: 256 images of 256 x 512 take 33 us (4.1 TB/s), 1024 of them 116; 32 and 113
+// with r = 1; the 1024 132 with the registers left free, as a CU then holds one workgroup; 390 the 256 in
 // two passes with the library's logarithm.
 struct EntropySums {
     double total, s;
@@ -530,7 +529,7 @@ void launch_accept_image(int frames, int n, const float* img_a, const double* en
                 ent_a, img_b, ent_b, rel_tol, out, accepted);
 }
 // 1024 threads an image from 8192 cells on, where every thread has a whole group of loads, 256 below:
-// 2000 images of 100 cells take 4.5 us (10.4 with 1024 threads), 1024 of 1000 cells 4.3 (6.1), of 8192
+// 2000 images of 100 cells take 4.5 us (10.4 with 1024 threads), 1024 of 1000 cells 4.4 (6.1), of 8192
 // cells 10.1 (11.3); but one image of 16384 cells 7.0 (5.5), 256 of 32768 14 (10).
 constexpr int kEntropyWideCells = 8192;
 void launch_image_entropy(int frames, int n, const float* img, double* out, hipStream_t s) {
